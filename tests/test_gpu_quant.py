@@ -241,3 +241,26 @@ def test_prune_sparse24_kat_and_matmul(ctx):
     torch.cuda.synchronize()
     ref = oracle.sparse24_gpu_matmul(meta, scale, xf, M, K, N)
     assert_close_f32(host(y), np.asarray(ref).reshape(M, N))
+
+
+@pytest.mark.parametrize("N,K", [(1023, 528), (1024, 2064), (2049, 1040), (4097, 528), (8200, 528), (3, 8224)])
+@pytest.mark.parametrize("wt", ["f32", "bf16"])
+def test_quantize_vector_path_equals_general(ctx, N, K, wt):
+    """The 16-byte-load kernels (each count of rows per wave, rows that end
+    inside a chunk) against the oracle on some rows and, bit for bit, against
+    the value-by-value kernels that an unaligned w takes."""
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    w = 0.02 * torch.randn((N, K), generator=g, device=DEV)
+    w[1, :5] = torch.tensor([float("nan"), float("inf"), -0.0, 0.5, -0.5], device=DEV)
+    w[2] = 0.0
+    w[2, ::4] = 1.0  # alpha 1 / 4 under the STE rule, 0.5 alpha a value of w
+    w[2, 1::4] = -0.125
+    w = w.to(torch.float32 if wt == "f32" else torch.bfloat16)
+    shifted = torch.empty(N * K + 1, dtype=w.dtype, device=DEV)[1:].view(N, K).copy_(w)
+    for rule in RULES:
+        packed, scale = _quantize(ctx, w, rule)
+        packed2, scale2 = _quantize(ctx, shifted, rule)
+        np.testing.assert_array_equal(scale.view(np.uint32), scale2.view(np.uint32))
+        np.testing.assert_array_equal(packed, packed2)
+        rows = sorted({0, 1, 2, N // 2, N - 1})
+        _check_rows(host(w.float())[rows], packed[rows], scale[rows], rule)

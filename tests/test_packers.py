@@ -102,3 +102,22 @@ def test_sparse_indices_host_equals_oracle():
     b = oracle.ternary_sparse_indices(t, 57, 130)
     for x, y in zip(a, b):
         np.testing.assert_array_equal(x[:len(y)], y)
+
+
+def test_ste_rule_without_a_division():
+    """fl(w / alpha) > 0.5 is w > alpha / 2 for every alpha from 1e-10 up (the
+    device codes compare instead of dividing): the floats around alpha / 2,
+    any mantissa and exponent, infinities and NaN."""
+    rng = np.random.default_rng(5)
+    alpha = np.concatenate([rng.uniform(1, 2, 20000).astype(np.float32) * np.float32(2.0) ** rng.integers(-33, 127, 20000),
+                            np.nextafter(np.float32(2.0) ** np.arange(-30, 120), np.float32(0)),
+                            np.float32(2.0) ** np.arange(-33, 128), [np.inf, np.nan, 1e-10]]).astype(np.float32)
+    alpha = alpha[~(alpha < np.float32(1e-10))]
+    half = np.float32(0.5) * alpha
+    up = np.nextafter(half, np.float32(np.inf))
+    down = np.nextafter(half, np.float32(0))
+    with np.errstate(all="ignore"):
+        for w in (half, up, down, np.nextafter(up, np.float32(np.inf)), alpha, np.full_like(alpha, np.inf),
+                  np.full_like(alpha, np.nan), np.zeros_like(alpha)):
+            np.testing.assert_array_equal(w / alpha > np.float32(0.5), w > half)
+            np.testing.assert_array_equal(-w / alpha < np.float32(-0.5), -w < -half)
