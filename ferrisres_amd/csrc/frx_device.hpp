@@ -125,6 +125,25 @@ __device__ __forceinline__ void unpack32_kil(uint32_t w0, uint32_t w1, u32x4 &lo
   hi1 = (u32x4){d1[4], d1[5], d1[6], d1[7]};
 }
 
+// K-interleaved staging of x for the decode of unpack32_kil: the 16-column
+// block b is pieces 2b (columns 0..7) and 2b+1 (8..15) of 8 bf16, held by
+// neighbouring lanes (piece index parity = lane parity). After swapping
+// pieces with its neighbour, the even lane returns block dwords 0..3 and the
+// odd lane dwords 4..7, dword i = x[16b + i] | x[16b + i + 8] << 16, to be
+// stored where its own piece would go. Every lane of the wave must call it
+// (DPP); pieces past the data are zeros.
+__device__ __forceinline__ u32x4 stage_kil(const u32x4 &mine, int tid) {
+  u32x4 other;
+#pragma unroll
+  for (int d = 0; d < 4; d++)
+    other[d] = (uint32_t)__builtin_amdgcn_mov_dpp((int)mine[d], 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
+  const bool odd = tid & 1;
+  const u32x4 A = odd ? other : mine, B = odd ? mine : other;
+  const uint32_t a0 = odd ? A.z : A.x, a1 = odd ? A.w : A.y, c0 = odd ? B.z : B.x, c1 = odd ? B.w : B.y;
+  return (u32x4){__builtin_amdgcn_perm(c0, a0, 0x05040100u), __builtin_amdgcn_perm(c0, a0, 0x07060302u),
+                 __builtin_amdgcn_perm(c1, a1, 0x05040100u), __builtin_amdgcn_perm(c1, a1, 0x07060302u)};
+}
+
 // Natural bf16 dwords n[0..7] of a 16-column block (x0..x15) -> interleaved
 // dwords d[i] = x[i] | x[i+8] << 16.
 // One byte permute per output dword.

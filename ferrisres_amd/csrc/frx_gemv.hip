@@ -719,25 +719,6 @@ __device__ __forceinline__ float dpp_f32(float v) {
 // XPL = 2: the activations arrive as two bf16 planes (X hi, X2 lo) whose sum
 // is an fp32 vector to 2^-17; both are staged and each word runs four MFMAs
 // into the same accumulator.
-// K-interleaved staging of x for the decode of unpack32_kil: the 16-column
-// block b is pieces 2b (columns 0..7) and 2b+1 (8..15) of 8 bf16, held by
-// neighbouring lanes (piece index parity = lane parity). After swapping
-// pieces with its neighbour, the even lane returns block dwords 0..3 and the
-// odd lane dwords 4..7, dword i = x[16b + i] | x[16b + i + 8] << 16, to be
-// stored where its own piece would go. Every lane of the wave must call it
-// (DPP); pieces past the data are zeros.
-__device__ __forceinline__ u32x4 stage_kil(const u32x4 &mine, int tid) {
-  u32x4 other;
-#pragma unroll
-  for (int d = 0; d < 4; d++)
-    other[d] = (uint32_t)__builtin_amdgcn_mov_dpp((int)mine[d], 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
-  const bool odd = tid & 1;
-  const u32x4 A = odd ? other : mine, B = odd ? mine : other;
-  const uint32_t a0 = odd ? A.z : A.x, a1 = odd ? A.w : A.y, c0 = odd ? B.z : B.x, c1 = odd ? B.w : B.y;
-  return (u32x4){__builtin_amdgcn_perm(c0, a0, 0x05040100u), __builtin_amdgcn_perm(c0, a0, 0x07060302u),
-                 __builtin_amdgcn_perm(c1, a1, 0x05040100u), __builtin_amdgcn_perm(c1, a1, 0x07060302u)};
-}
-
 template <typename YT, int WAVES, int RW, int NI, int NW = 1, int XPL = 1, int EPI = GEMV_LINEAR>
 __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(
     const uint32_t *__restrict__ W, const float *__restrict__ scale, const uint32_t *__restrict__ W2,

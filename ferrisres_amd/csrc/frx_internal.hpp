@@ -247,6 +247,16 @@ hipError_t launch_router_transpose(const void *src, int rt_bf16, void *dst, int 
 // MoE pipeline (frx_moe.hip).
 // Most routed rows (tokens x top_k) of the MoE decode path.
 constexpr int MOE_DEC_MAXA = 4;
+// Most routed rows of the decode-batch path (per-expert row tiles, frx_moe.hip),
+// and whether a batch takes it: up to 16 routes per expert. Above, an expert
+// has more tokens than the 16 columns of its row tiles and its weights are
+// decoded more than once, as the grouped GEMMs' 64-row tiles fill up (2048 /
+// 5632, 16 experts, top 2, bf16: 8 / 32 / 128 tokens 115.6 / 133.0 / 141.6 ->
+// 55.5 / 73.9 / 116.1 us; f32 157.6 / 186.1 / 196.3 -> 68.5 / 85.5 / 158.6).
+constexpr int MOE_ROWS_MAXA = 512;
+inline bool moe_rows_fits(int A, int T, int H, int E) {
+  return A <= MOE_ROWS_MAXA && (size_t)(H + 127) / 128 * T <= (size_t)GEMV_SK_MAX_TILES && A <= 16 * E;
+}
 
 struct MoeWorkspace {
   uint32_t *idx;       // [T*k] selected experts (sorted order per token)
@@ -269,6 +279,8 @@ struct MoeWorkspace {
   float *dout_lo;      // [T*k][H] second partial (engine-2 path: the second
                        // K part)
   uint16_t *x2;        // [T][2H] f32 x as bf16 hi | lo rows (engine-2 path)
+  float *dpart;        // [S][T*k][H] K parts of the down projection (decode
+                       // batch; null above MOE_ROWS_MAXA routed rows)
   unsigned *cnt = nullptr;  // decode path: (column block, token) arrival
                             // counters, zero between launches; null: the
                             // combine runs as a launch of its own

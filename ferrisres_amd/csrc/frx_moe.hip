@@ -26,6 +26,8 @@
 //                    exactly the reference's accumulation (deterministic).
 #include "frx_gemm2.hpp"
 #include "frx_gemm_core.hpp"
+#include <algorithm>
+
 #include "frx_internal.hpp"
 
 namespace frx {
@@ -35,6 +37,8 @@ constexpr int MOE_BM = 64;   // tokens per grouped-GEMM tile
 constexpr int MOE_BN = 128;  // weight rows per tile
 
 static inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+static size_t mr_dpart_bytes(int A, int H, int I);
 
 size_t moe_workspace_bytes(int T, int H, int I, int E, int top_k) {
   const size_t A = (size_t)T * top_k;
@@ -50,6 +54,7 @@ size_t moe_workspace_bytes(int T, int H, int I, int E, int top_k) {
   b += align256(A * I * 2) * 2;         // h planes
   b += align256(A * H * 4) * 2;         // dout, dout_lo
   b += align256((size_t)T * H * 4);     // f32 x as bf16 hi | lo rows
+  b += align256(mr_dpart_bytes((int)A, H, I));  // decode batch: the down projection's K parts
   return b;
 }
 
@@ -75,6 +80,8 @@ void moe_workspace_carve(void *base, int T, int H, int I, int E, int top_k,
   ws->dout = reinterpret_cast<float *>(take(A * H * 4));
   ws->dout_lo = reinterpret_cast<float *>(take(A * H * 4));
   ws->x2 = reinterpret_cast<uint16_t *>(take((size_t)T * H * 4));
+  const size_t db = mr_dpart_bytes((int)A, H, I);
+  ws->dpart = db ? reinterpret_cast<float *>(take(db)) : nullptr;
 }
 
 template <typename T>
@@ -1462,6 +1469,396 @@ __global__ __launch_bounds__(512) void moe_dec_down_kernel(const DownArgs args, 
   else reinterpret_cast<float *>(y)[(size_t)t * H + n] = accy;
 }
 
+// ---- a decode batch: per-expert row tiles over the tokens routed to it ---------
+// From a few routed rows to a few per expert, the grouped GEMMs multiply
+// tiles of 64 token rows for experts that have one or two, in a K loop three
+// steps deep: 16 rows over 16 experts (8 tokens, top 2, 2048 / 5632) took 57
+// us for gate/up and 52 us for down, against 18 us to read the reached
+// experts' weights. Here the tokens of an expert are the 16 columns of the
+// MFMA (fp32 activations as 8 tokens' hi planes and the same 8 tokens' lo
+// planes, added across lanes at the end), a wave owns whole 16-row tiles and
+// has its weights in flight before the activations are staged, and no wave
+// adds to another's sums. More tokens than columns: further passes.
+// A workgroup finds its expert's routes by a ballot over the selected
+// experts, so nothing has to group them first.
+constexpr int MR_COLS = 16;
+constexpr int MR_GU_CH = 2;          // 256-column blocks per weight batch (two batches in flight)
+constexpr int MR_DN_CH = 6;          // 256-column blocks of a down K part, all in flight
+constexpr int MR_DN_W = 4;           // waves of a down workgroup, 32 rows each
+constexpr int MR_DN_MAXS = 8;        // K parts of the down projection
+constexpr uint32_t MR_OOB = 0x80000000u;
+
+// LDS row of `n` staged columns: whole 256-column blocks (zeros past n) and
+// 16 bytes that put the 16 rows of an operand read on different banks.
+__host__ __device__ constexpr int mr_stride(int n) { return (n + 255) / 256 * 256 + 8; }
+
+// Routes of expert e, in order, into list (by wave 0); every wave returns their
+// number.
+__device__ __forceinline__ int mr_routes(const uint32_t *idx, int A, int e, int *list) {
+  const int lane = threadIdx.x & 63;
+  int n = 0;
+  for (int a0 = 0; a0 < A; a0 += 64) {
+    const bool in = a0 + lane < A && (int)idx[min(a0 + lane, A - 1)] == e;
+    const unsigned long long m = __ballot(in);
+    if (in && threadIdx.x < 64) list[n + __popcll(m & ((1ull << lane) - 1ull))] = a0 + lane;
+    n += __popcll(m);
+  }
+  return n;
+}
+
+// Rows src(r), r < rows, of n columns (n % 8 == 0, 16-byte aligned) into LDS
+// rows r, zeros up to the next 256 columns; f32 rows split into row r and row
+// r + lo_row. A thread moves 8 columns of MR_U rows at a time with
+// unconditional loads and writes: rows and columns past the end are clamped to
+// the last ones, which are then written more than once with the same values (a
+// write under a branch takes its load with it, behind the weights). The
+// first batch is loaded by mr_load and written by mr_write
+// so that the weight loads can go in between: vector loads complete in issue
+// order, so the activations do not wait for the weights.
+constexpr int MR_U = 4;
+template <typename XT>
+struct MrBatch {
+  u32x4 v[MR_U][sizeof(XT) == 2 ? 1 : 2];
+};
+// The words decode in K-interleaved pairs (unpack32_kil: 11.5 VALU ops a word,
+// 15 in natural order), so the rows are staged to match (stage_kil, once per
+// workgroup); clamped columns stay on their own half of the 16-column block.
+__device__ __forceinline__ int mr_col(int c, int n) {
+  return min(c & ~15, (n + 255) / 256 * 256 - 16) + (c & 8);
+}
+template <typename XT, typename Src>
+__device__ __forceinline__ void mr_load(MrBatch<XT> &b, Src src, int r0, int rows, int c, int n) {
+#pragma unroll
+  for (int u = 0; u < MR_U; u++) {
+    const XT *p = src(min(r0 + u, rows - 1)) + min(c, n - 8);
+#pragma unroll
+    for (int k = 0; k < (sizeof(XT) == 2 ? 1 : 2); k++) b.v[u][k] = *reinterpret_cast<const u32x4 *>(p + 4 * k);
+  }
+}
+template <typename XT>
+__device__ __forceinline__ void mr_write(const MrBatch<XT> &b, int r0, int rows, int c, int n, int stride,
+                                         uint16_t *dst, int lo_row) {
+  const uint32_t keep = c < n ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+  for (int u = 0; u < MR_U; u++) {
+    const int r = min(r0 + u, rows - 1);
+    u32x4 h = b.v[u][0], l;
+    if constexpr (sizeof(XT) == 4) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        uint32_t hq, lq;
+        split2_bf16(__uint_as_float(b.v[u][q >> 1][2 * (q & 1)]), __uint_as_float(b.v[u][q >> 1][2 * (q & 1) + 1]), hq,
+                    lq);
+        h[q] = hq;
+        l[q] = lq & keep;
+      }
+      *reinterpret_cast<u32x4 *>(dst + (r + lo_row) * stride + c) = stage_kil(l, threadIdx.x);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) h[q] &= keep;
+    *reinterpret_cast<u32x4 *>(dst + r * stride + c) = stage_kil(h, threadIdx.x);
+  }
+}
+// The rest of the batches after the first.
+template <typename XT, typename Src>
+__device__ __forceinline__ void mr_rest(Src src, int rows, int n, int stride, uint16_t *dst, int lo_row) {
+  const int step = (int)blockDim.x * 8;
+  for (int c0 = 0; c0 < n; c0 += step)
+    for (int r0 = c0 ? 0 : MR_U; r0 < rows; r0 += MR_U) {
+      MrBatch<XT> b;
+      const int c = mr_col(c0 + (int)threadIdx.x * 8, n);
+      mr_load<XT>(b, src, r0, rows, c, n);
+      mr_write<XT>(b, r0, rows, c, n, stride, dst, lo_row);
+    }
+}
+
+// part[f][.] += W fragment f . staged activations over the 256-column blocks
+// [k0, k0 + CH) below nb; xc: the lane's staged row at column 64 g.
+template <int NF, int CH>
+__device__ __forceinline__ void mr_mul(const u32x4 (&wq)[NF][CH], int k0, int nb, const uint16_t *xc,
+                                       f32x4 (&part)[NF][2]) {
+#pragma unroll
+  for (int c = 0; c < CH; c++) {
+    if (k0 + c < nb) {  // workgroup-uniform
+      u32x4 x[8];
+#pragma unroll
+      for (int w = 0; w < 8; w++) x[w] = *reinterpret_cast<const u32x4 *>(xc + (k0 + c) * 256 + 8 * w);
+      __builtin_amdgcn_sched_barrier(0);  // all eight reads before their MFMAs
+#pragma unroll
+      for (int w = 0; w < 4; w += 2)
+#pragma unroll
+        for (int f = 0; f < NF; f++) {
+          u32x4 a0, a1, b0, b1;
+          unpack32_kil(wq[f][c][w], wq[f][c][w + 1], a0, a1, b0, b1);
+          part[f][0] = mfma16(a0, x[2 * w], part[f][0]);
+          part[f][1] = mfma16(a1, x[2 * w + 1], part[f][1]);
+          part[f][0] = mfma16(b0, x[2 * w + 2], part[f][0]);
+          part[f][1] = mfma16(b1, x[2 * w + 3], part[f][1]);
+        }
+    }
+  }
+}
+
+// v + the value of the lane 8 columns away (the other plane of the token).
+__device__ __forceinline__ f32x4 mr_add_planes(f32x4 v) {
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    v[q] += __uint_as_float(
+        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v[q]), 0x128, 0xF, 0xF, true));  // row_ror:8
+  return v;
+}
+
+// grid (ceil(I / (16 WAVES)), E): a wave's 16 gate and 16 up rows of expert
+// blockIdx.y against its tokens; h = act(g, u) as bf16 hi and lo planes of
+// the routes' rows [A][I].
+template <typename XT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void moe_rows_gateup_kernel(const GateUpArgs args, const XT *__restrict__ x,
+                                                                     int H, int I, int A, int top_k,
+                                                                     const uint32_t *__restrict__ idx,
+                                                                     uint16_t *__restrict__ h_hi,
+                                                                     uint16_t *__restrict__ h_lo, int act) {
+  constexpr int NP = sizeof(XT) == 2 ? 1 : 2, TP = MR_COLS / NP;  // planes, tokens per pass
+  extern __shared__ __align__(16) uint16_t dsm[];
+  __shared__ int list[MOE_ROWS_MAXA];
+  const int e = blockIdx.y;
+  const int n = mr_routes(idx, A, e, list);
+  if (n == 0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  const int n0 = (blockIdx.x * WAVES + wave) * 16, kw = H >> 4, nb = (H + 255) >> 8;
+  const int stride = mr_stride(H);
+  const uint32_t wbytes = (uint32_t)I * (uint32_t)kw * 4u;
+  const __amdgpu_buffer_rsrc_t wr[2] = {buffer_rsrc(args.wg[e], wbytes), buffer_rsrc(args.wu[e], wbytes)};
+  const uint32_t wo = ((uint32_t)(n0 + i) * (uint32_t)kw + 4u * g) * 4u;
+  const bool rok = n0 + i < I;
+  auto fetch = [&](u32x4(&d)[2][MR_GU_CH], int b0) {
+#pragma unroll
+    for (int c = 0; c < MR_GU_CH; c++)
+#pragma unroll
+      for (int f = 0; f < 2; f++)
+        d[f][c] = __builtin_amdgcn_raw_buffer_load_b128(
+            wr[f], rok && (b0 + c) * 256 + 64 * g < H ? wo + (uint32_t)(b0 + c) * 64u : MR_OOB, 0, 0);
+  };
+  // the lane's output rows and their scales (read early: the epilogue is short)
+  const int r = n0 + 4 * g;
+  float sg[4], su[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    sg[q] = args.sg[e][min(r + q, I - 1)];
+    su[q] = args.su[e][min(r + q, I - 1)];
+  }
+  for (int p0 = 0; p0 < n; p0 += TP) {
+    const int np = min(TP, n - p0);
+    u32x4 wa[2][MR_GU_CH], wb[2][MR_GU_CH];
+    __syncthreads();  // the list, or the previous pass's reads
+    const int lv = list[p0 + min(i, np - 1)] / top_k;  // lane r: the token of row r
+    auto src = [&](int r) { return x + (size_t)__builtin_amdgcn_readlane(lv, r) * H; };
+    const int c = mr_col((int)threadIdx.x * 8, H);
+    MrBatch<XT> xb;
+    mr_load<XT>(xb, src, 0, np, c, H);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(wa, 0);
+    fetch(wb, MR_GU_CH);
+    __builtin_amdgcn_sched_barrier(0);
+    mr_write<XT>(xb, 0, np, c, H, stride, dsm, TP);
+    mr_rest<XT>(src, np, H, stride, dsm, TP);
+    __syncthreads();
+    f32x4 part[2][2];
+#pragma unroll
+    for (int f = 0; f < 2; f++) part[f][0] = part[f][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    // columns without a token repeat the last one; their sums are not stored
+    const uint16_t *xc = dsm + (min(i % TP, np - 1) + i / TP * TP) * stride + 64 * g;
+    for (int b = 0; b < nb; b += 2 * MR_GU_CH) {
+      mr_mul(wa, b, nb, xc, part);
+      if (b + 2 * MR_GU_CH < nb) fetch(wa, b + 2 * MR_GU_CH);
+      mr_mul(wb, b + MR_GU_CH, nb, xc, part);
+      if (b + 3 * MR_GU_CH < nb) fetch(wb, b + 3 * MR_GU_CH);
+    }
+    f32x4 gv = part[0][0] + part[0][1], uv = part[1][0] + part[1][1];
+    if constexpr (NP == 2) {
+      gv = mr_add_planes(gv);
+      uv = mr_add_planes(uv);
+    }
+    if (i < np && r < I) {  // I % 64 == 0: all four rows
+      const size_t o = (size_t)list[p0 + i] * I + r;
+      float h[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++)  // 0.5 undoes the 2*dec(c) encoding
+        h[q] = moe_act(act, gv[q] * (0.5f * sg[q]), uv[q] * (0.5f * su[q]));
+      u32x2 hi, lo;
+      uint32_t a, b;
+      split2_bf16(h[0], h[1], a, b);
+      hi.x = a;
+      lo.x = b;
+      split2_bf16(h[2], h[3], a, b);
+      hi.y = a;
+      lo.y = b;
+      *reinterpret_cast<u32x2 *>(h_hi + o) = hi;
+      *reinterpret_cast<u32x2 *>(h_lo + o) = lo;
+    }
+  }
+}
+
+// grid (ceil(H / 128), S, E): a wave's 32 rows of W_down[e] over K part
+// blockIdx.y (ks columns) against h's planes of the expert's routes; the
+// part's rows go to dpart[s][route][H] (device-coherent), and the last of a
+// token's S top_k workgroups of a row block adds them in order (d = part 0 +
+// part 1 + ..., acc from 0, k = 0, 1, ..., d * w rounded before the add,
+// CpuMoELayer's skip of |w| < 1e-8) and writes y.
+__global__ __launch_bounds__(MR_DN_W * 64, 3) void moe_rows_down_kernel(
+    const DownArgs args, const uint16_t *__restrict__ h_hi, const uint16_t *__restrict__ h_lo, int H, int I, int ks,
+    int A, int top_k, const uint32_t *__restrict__ idx, float *__restrict__ dpart, unsigned *__restrict__ cnt,
+    const float *__restrict__ wts, int skip_small, void *__restrict__ y, int y_bf16) {
+  constexpr int TP = MR_COLS / 2;
+  constexpr int SC1 = 16;  // cache policy: performed at the point of coherence of all XCDs
+  extern __shared__ __align__(16) uint16_t dsm[];
+  __shared__ int list[MOE_ROWS_MAXA];
+  __shared__ int last[MOE_ROWS_MAXA];
+  const int e = blockIdx.z, s = blockIdx.y, S = gridDim.y;
+  const int n = mr_routes(idx, A, e, list);
+  if (n == 0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  const int n0 = (blockIdx.x * MR_DN_W + wave) * 32, kw = I >> 4;
+  const int k0 = s * ks, kl = min(ks, I - k0), nb = (kl + 255) >> 8, stride = mr_stride(ks);
+  const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(args.wd[e], (uint32_t)H * (uint32_t)kw * 4u);
+  float sd[2][4];  // read early: the epilogue is short
+#pragma unroll
+  for (int f = 0; f < 2; f++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) sd[f][q] = args.sd[e][min(n0 + 16 * f + 4 * g + q, H - 1)];
+  u32x4 wq[2][MR_DN_CH];
+  const __amdgpu_buffer_rsrc_t pr = buffer_rsrc(dpart, (uint32_t)S * (uint32_t)A * (uint32_t)H * 4u);
+  // one pass: up to TP routes, staged (the first batch of rows is in hb)
+  auto row_of = [&](int lv, int np) {
+    return [=](int r) {
+      return (r < np ? h_hi : h_lo) + (size_t)__builtin_amdgcn_readlane(lv, r < np ? r : r - np) * I + k0;
+    };
+  };
+  const int c = mr_col((int)threadIdx.x * 8, kl);
+  auto pass = [&](int np, int lv, const MrBatch<uint16_t> &hb) __attribute__((always_inline)) {
+    mr_write<uint16_t>(hb, 0, 2 * np, c, kl, stride, dsm, 0);
+    mr_rest<uint16_t>(row_of(lv, np), 2 * np, kl, stride, dsm, 0);
+    __syncthreads();
+    f32x4 part[2][2];
+#pragma unroll
+    for (int f = 0; f < 2; f++) part[f][0] = part[f][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    // columns without a route repeat the last one; their sums are not stored
+    mr_mul(wq, 0, nb, dsm + (min(i % TP, np - 1) + i / TP * np) * stride + 64 * g, part);
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+      const f32x4 v = mr_add_planes(part[f][0] + part[f][1]);
+      const int r = n0 + 16 * f + 4 * g;
+      f32x4 o;
+#pragma unroll
+      for (int q = 0; q < 4; q++) o[q] = v[q] * (0.5f * sd[f][q]);
+      const bool ok = i < np && r < H;  // H % 64 == 0: all four rows; lv: the route of column i
+      const uint32_t off =
+          ok ? (((uint32_t)s * (uint32_t)A + (uint32_t)lv) * (uint32_t)H + (uint32_t)r) * 4u : MR_OOB;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), pr, off, 0, SC1);
+    }
+  };
+  __syncthreads();  // the list
+  {
+    const int np = min(TP, n), lv = list[min(i, np - 1)];  // lane r: the route of rows r and np + r
+    MrBatch<uint16_t> hb;
+    mr_load<uint16_t>(hb, row_of(lv, np), 0, 2 * np, c, kl);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < MR_DN_CH; q++)
+#pragma unroll
+      for (int f = 0; f < 2; f++) {
+        const int row = n0 + 16 * f + i;
+        wq[f][q] = __builtin_amdgcn_raw_buffer_load_b128(
+            wr,
+            row < H && q * 256 + 64 * g < kl
+                ? ((uint32_t)row * (uint32_t)kw + (uint32_t)(k0 >> 4) + 16u * q + 4u * g) * 4u
+                : MR_OOB,
+            0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    pass(np, lv, hb);
+  }
+  for (int p0 = TP; p0 < n; p0 += TP) {
+    const int np = min(TP, n - p0), lv = list[p0 + min(i, np - 1)];
+    __syncthreads();  // the previous pass's reads
+    // decode the words again: unpacked once for all passes they would fill
+    // (and spill) every register
+#pragma unroll
+    for (int q = 0; q < MR_DN_CH; q++)
+#pragma unroll
+      for (int f = 0; f < 2; f++) asm volatile("" : "+v"(wq[f][q]));
+    MrBatch<uint16_t> hb;
+    mr_load<uint16_t>(hb, row_of(lv, np), 0, 2 * np, c, kl);
+    pass(np, lv, hb);
+  }
+  wait_vmcnt<0>();  // this wave's partial rows are stored
+  __syncthreads();
+  const int T = A / top_k;
+  for (int r = threadIdx.x; r < n; r += MR_DN_W * 64) {
+    unsigned *c = cnt + (size_t)blockIdx.x * T + list[r] / top_k;
+    const unsigned old = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last[r] = old == (unsigned)(S * top_k) - 1u;
+    if (last[r]) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  // 32 column quads per token, MR_DN_W * 2 tokens at a time
+  for (int r = threadIdx.x >> 5; r < n; r += MR_DN_W * 2) {
+    const int t = list[r] / top_k, c = blockIdx.x * (MR_DN_W * 32) + (threadIdx.x & 31) * 4;
+    if (!last[r] || c >= H) continue;
+    constexpr int Q = 8;  // loads in flight
+    const int terms = S * top_k;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, d = acc;
+    int k = 0, sp = 0;
+    for (int q0 = 0; q0 < terms; q0 += Q) {
+      f32x4 v[Q];
+      int kk = k, ss = sp;
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+        const uint32_t off =
+            q0 + q < terms ? (((uint32_t)ss * (uint32_t)A + (uint32_t)(t * top_k + kk)) * (uint32_t)H + (uint32_t)c) * 4u
+                           : MR_OOB;
+        v[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, off, 0, SC1));
+        if (++ss == S) {
+          ss = 0;
+          kk++;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+#pragma clang fp contract(off)
+        if (q0 + q < terms) {
+          d = sp == 0 ? v[q] : d + v[q];
+          if (++sp == S) {
+            sp = 0;
+            const float w = wts[t * top_k + k];
+            k++;
+            if (!(skip_small && fabsf(w) < 1e-8f)) {  // src/model/cpu_moe.rs:172
+              const f32x4 prod = d * w;
+              acc = acc + prod;
+            }
+          }
+        }
+      }
+    }
+    if (y_bf16) YStore<uint16_t>::store4(reinterpret_cast<uint16_t *>(y) + (size_t)t * H + c, acc, 4);
+    else YStore<float>::store4(reinterpret_cast<float *>(y) + (size_t)t * H + c, acc, 4);
+  }
+}
+
+// K parts of the down projection: whole 64-column steps, at most what a wave
+// holds in registers.
+static int mr_down_parts(int I, int *ks) {
+  const int S = (I + MR_DN_CH * 256 - 1) / (MR_DN_CH * 256);
+  *ks = ((I + S - 1) / S + 63) / 64 * 64;
+  return (I + *ks - 1) / *ks;
+}
+
+static size_t mr_dpart_bytes(int A, int H, int I) {
+  int ks;
+  return A <= MOE_ROWS_MAXA ? (size_t)mr_down_parts(I, &ks) * A * H * 4 : 0;
+}
+
 // ---- 5. combine ---------------------------------------------------------------
 // cpu_block_attn_res.rs:1179 `expert_outputs[t*hd+d] += w * down[d]`, k order.
 // dout_lo != nullptr: the down rows arrive as two partials (the engine-2 K
@@ -1641,6 +2038,38 @@ hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
     else
       hipLaunchKernelGGL((moe_combine_kernel<float>), dim3(T), dim3(256), 0, stream, ws.dout, ws.dout_lo, ws.wts,
                          ws.inv, H, top_k, (float *)y, routing);
+    return hipGetLastError();
+  }
+  int mks = 0;
+  const int mS = mr_down_parts(I, &mks);
+  const int cols = xt_bf16 ? std::min(T, MR_COLS) : MR_COLS / 2 + std::min(T, MR_COLS / 2);
+  const size_t gu_lds_rows = (size_t)cols * mr_stride(H) * 2;
+  if (engine2 && ws.dpart && !lora.tbl && moe_rows_fits(A, T, H, E) && mS <= MR_DN_MAXS &&
+      gu_lds_rows <= 144 * 1024 && (size_t)mS * A * H * 4 < ((size_t)1 << 31) &&
+      (size_t)H * I / 4 < ((size_t)1 << 31) && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+    // four-wave workgroups while four of them fit a compute unit's LDS, else
+    // eight waves to a staged copy
+    const int wv = gu_lds_rows <= 38 * 1024 ? 4 : 8;
+    const dim3 gg((I + 16 * wv - 1) / (16 * wv), E);
+#define FRX_MR_GU(XT, WV)                                                                                            \
+  {                                                                                                                  \
+    static std::atomic<uint64_t> done;                                                                               \
+    if ((err = opt_in_lds(reinterpret_cast<const void *>(&moe_rows_gateup_kernel<XT, WV>), 144 * 1024, done)) !=     \
+        hipSuccess)                                                                                                  \
+      return err;                                                                                                    \
+    hipLaunchKernelGGL((moe_rows_gateup_kernel<XT, WV>), gg, dim3(WV * 64), gu_lds_rows, stream, ga, (const XT *)x, H, \
+                       I, A, top_k, ws.idx, ws.h_hi, ws.h_lo, act);                                                  \
+  }
+    if (xt_bf16 && wv == 4) FRX_MR_GU(uint16_t, 4)
+    else if (xt_bf16) FRX_MR_GU(uint16_t, 8)
+    else if (wv == 4) FRX_MR_GU(float, 4)
+    else FRX_MR_GU(float, 8)
+#undef FRX_MR_GU
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+    const size_t dl = (size_t)2 * std::min(T, MR_COLS / 2) * mr_stride(mks) * 2;
+    hipLaunchKernelGGL(moe_rows_down_kernel, dim3((H + 32 * MR_DN_W - 1) / (32 * MR_DN_W), mS, E), dim3(MR_DN_W * 64),
+                       dl, stream, da, ws.h_hi, ws.h_lo, H, I, mks, A, top_k, ws.idx, ws.dpart, ws.cnt, ws.wts,
+                       routing, y, yt_bf16);
     return hipGetLastError();
   }
   // 2. group

@@ -93,6 +93,32 @@ def test_moe_decode_rows_parity(ctx, T, H, I, E, k, act, xt):
     assert_bf16_within_1ulp(yb.view(torch.int16).cpu().numpy().view(np.uint16), ref)
 
 
+@pytest.mark.parametrize("T,H,I,E,k,act,xt", [
+    (5, 64, 64, 5, 1, frx.ACT_SILU, "bf16"), (8, 2048, 5632, 16, 2, frx.ACT_SILU, "f32"),
+    (16, 320, 1600, 8, 2, frx.ACT_GELU_TANH, "bf16"), (17, 4096, 192, 3, 2, frx.ACT_SILU, "bf16"),
+    (40, 128, 3136, 6, 2, frx.ACT_SILU, "f32"), (64, 1088, 256, 32, 4, frx.ACT_GELU_TANH_GATE, "bf16"),
+    (16, 2304, 8192, 2, 2, frx.ACT_SILU, "f32"), (9, 192, 128, 64, 3, frx.ACT_GELU_TANH, "f32")])
+def test_moe_row_tiles_parity(ctx, T, H, I, E, k, act, xt):
+    """A decode batch (up to 16 routes per expert): the experts' tokens as the
+    columns of their row tiles. Row tiles and K parts that end inside a wave
+    or a 256-column block, experts without a token, more tokens than columns
+    (further passes), one to six K parts of the down projection; twice, so
+    that the arrival counters were left at zero."""
+    name = f"moe/rows/{T}x{H}x{I}x{E}x{k}"
+    xf, xb, rf, rb, ex = make_moe(name, T, H, I, E)
+    if xt == "f32":
+        xf = synth.normal(synth.seed_of(name, "xf32"), T * H).reshape(T, H)
+    ref, ridx, rw = run_oracle(xf, rf, ex, E, k, act)
+    for yt in ("f32", "bf16"):
+        y, idx, w = run_gpu(ctx, xf, xb, rf, rb, ex, E, k, act, xt=xt, yt=yt, no_up=act == frx.ACT_GELU_TANH_GATE)
+        np.testing.assert_array_equal(idx, ridx)
+        np.testing.assert_allclose(w, rw, rtol=0, atol=1e-6)
+        if yt == "f32":
+            assert_close_f32(host(y), ref)
+        else:
+            assert_bf16_within_1ulp(y.view(torch.int16).cpu().numpy().view(np.uint16), ref)
+
+
 @pytest.mark.parametrize("T", [1, 40])
 def test_moe_unaligned_tokens_and_router(ctx, T):
     """x and the router one bf16 element into larger buffers (element-aligned,
