@@ -585,6 +585,27 @@ frx_status frx_ternary_linear_group(frx_ctx *ctx, const void *x, frx_dtype xt, u
   return FRX_OK;
 }
 
+// A 2:4 decode batch on aligned operands through the row-tile GEMV; *done says
+// whether the call took it.
+static frx_status sp24_rows_auto(frx_ctx *ctx, const uint32_t *w, int prepared, const Staged &sg, frx_dtype xt,
+                                 frx_dtype yt, uint32_t M, uint32_t K, uint32_t N, bool *done) {
+  int ncs = 0, S = 0;
+  // NEVER keeps the unsplit engine from 5 tokens, where it has one worth keeping
+  *done = (ctx->gemv_split != FRX_GEMV_SPLIT_NEVER || M <= 4) &&
+          frx::sp24_rows_plan((int)M, (int)K, (int)N, xt == FRX_BF16, prepared, ctx->cus, &ncs, &S);
+  if (!*done) return FRX_OK;
+  frx_status st = ensure_buffer(ctx, &ctx->gk_ws, &ctx->gk_ws_bytes, frx::sp24_rows_workspace_bytes((int)M, (int)N, S),
+                                "split-K GEMM workspace allocation");
+  if (st != FRX_OK) return st;
+  if ((st = ensure_sk_counters(ctx)) != FRX_OK) return st;
+  hipError_t e = frx::launch_sp24_rows(w, prepared, sg.scale, sg.x, xt == FRX_BF16, sg.y, yt == FRX_BF16, (int)M,
+                                       (int)K, (int)N, ncs, S, reinterpret_cast<float *>(ctx->gk_ws), ctx->sk_cnt,
+                                       ctx->stream);
+  if (e == hipSuccess) e = unstage_linear(ctx, sg);
+  if (e != hipSuccess) return hip_fail(ctx, e, "sparse24_ternary_linear launch");
+  return FRX_OK;
+}
+
 // Token count from which a 2:4 linear decodes its metadata once into the
 // prepared form (one pass over the matrix, 10.6 us at 11008 x 4096) before
 // the GEMM: at 512 tokens and more the cheaper operand decode repays it
@@ -602,18 +623,20 @@ frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
   if ((st = stage_linear(ctx, x, xt, scale, y, yt, M, K, N, &sg)) != FRX_OK) return st;
   hipError_t e = hipSuccess;
   int S = 0, sp = 0;
-  if (frx::sp24_gemv_plan((int)M, (int)K, (int)N, xt == FRX_BF16, &S)) {
+  if (frx::sp24_gemv_plan((int)M, (int)K, (int)N, &S)) {
     // decode: the metadata read once by a table-driven GEMV
     if ((st = ensure_buffer(ctx, &ctx->gk_ws, &ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S),
                             "split-K GEMM workspace allocation")) != FRX_OK)
       return st;
     if ((st = ensure_sk_counters(ctx)) != FRX_OK) return st;
-    e = frx::launch_sp24_gemv(meta, sg.scale, sg.x, xt == FRX_BF16, sg.y, yt == FRX_BF16, (int)M, (int)K, (int)N, S,
+    e = frx::launch_sp24_gemv(meta, sg.scale, sg.x, xt == FRX_BF16, sg.y, yt == FRX_BF16, (int)K, (int)N, S,
                               reinterpret_cast<float *>(ctx->gk_ws), ctx->sk_cnt, ctx->stream);
     if (e == hipSuccess) e = unstage_linear(ctx, sg);
     if (e != hipSuccess) return hip_fail(ctx, e, "sparse24_ternary_linear launch");
     return FRX_OK;
   }
+  bool done = false;
+  if ((st = sp24_rows_auto(ctx, meta, 0, sg, xt, yt, M, K, N, &done)) != FRX_OK || done) return st;
   // f32 x runs as bf16 hi | lo rows ([M][2K], |x - hi - lo| <= 2^-17 |x|)
   // through the same sparse engine, both halves against the same weights
   const bool planes = xt == FRX_F32 && aligned16(sg.x) && K % 64 == 0 && (size_t)M * K * 4 < ((size_t)1 << 31);
@@ -693,6 +716,8 @@ frx_status frx_sparse24_prepared_linear(frx_ctx *ctx, const uint32_t *prepared, 
     return fail(ctx, FRX_ERR_UNSUPPORTED, "x of %zu bytes exceeds 2 GiB", (size_t)M * K * 2);
   Staged sg;
   if ((st = stage_linear(ctx, x, xt, scale, y, yt, M, K, N, &sg)) != FRX_OK) return st;
+  bool done = false;
+  if ((st = sp24_rows_auto(ctx, prepared, 1, sg, xt, yt, M, K, N, &done)) != FRX_OK || done) return st;
   hipError_t e;
   int S = 0, sp = 0;
   if (ctx->gemv_split != FRX_GEMV_SPLIT_NEVER && frx::gemm_sp_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &sp)) {

@@ -319,35 +319,33 @@ static hipError_t launch_gemm2sp_parts(const uint32_t *meta, const void *x, int 
   return hipGetLastError();
 }
 
-// ---- 2:4 decode GEMV over the 5-bit layout (1-4 tokens, VALU) ----------------
+// ---- 2:4 decode GEMV over the 5-bit layout (one token, VALU) -----------------
 // The metadata is read once at 1.25 bits per weight. A workgroup owns 256
 // rows (one per lane) and a chunk of W metadata words of each row (6 groups
 // of 4 columns per word). It first tabulates, for each group of the chunk
 // and each of the 32 five-bit codes, the value the group adds:
 // 2 (s0 x[4g + p0] + s1 x[4g + p1]) (pattern > 5 read as 5, sign bits 3 and
 // 4; twice the sum, the 2 dec(c) scale of the other kernels). A code then
-// costs one LDS read and one add per token; the lanes of a wave read the same
+// costs one LDS read and one add; the lanes of a wave read the same
 // group's 32 entries at a time, one bank each. The chunks' sums go to
-// part[chunk][M][N] and are added in chunk order: by the last chunk of each
+// part[chunk][N] and are added in chunk order: by the last chunk of each
 // row block to arrive (up to SPV_FUSED_MAX chunks), else by
 // gemm_splitk_reduce in a second launch.
-template <int MT>
-__host__ __device__ constexpr int spv_words() { return 16; }  // LDS <= 54 KB at 4 tokens
+constexpr int SPV_WORDS = 16;  // one metadata load per 4 lanes and row
 // Most chunks that the last-arriving workgroup adds itself, all loads in
 // flight at once; above, a second launch does (4096 x 11008, 29 chunks:
 // 12.9 against 10.8 us with 8 loads in flight, 11.5 against 10.4 with all
 // 29; a limit of 32 also slowed the shapes of 11 chunks, 9.3 -> 9.5 us).
 constexpr int SPV_FUSED_MAX = 12;
 
-template <typename XT, int MT, typename YT, bool XMAP>
+template <typename XT, typename YT, bool XMAP>
 __global__ __launch_bounds__(256) void sp24_gemv_kernel(const uint32_t *__restrict__ meta, const XT *__restrict__ x,
                                                         float *__restrict__ part, unsigned *__restrict__ counters,
-                                                        const float *__restrict__ scale, YT *__restrict__ Y, int M,
-                                                        int N, int K, int S) {
-  constexpr int W = spv_words<MT>(), G = 6 * W;
-  static_assert(W == 16, "one metadata load per 16 lanes and row");
-  __shared__ float xs[MT][4 * G];
-  __shared__ float tab[MT][G * 32];
+                                                        const float *__restrict__ scale, YT *__restrict__ Y, int N,
+                                                        int K, int S) {
+  constexpr int W = SPV_WORDS, G = 6 * W;
+  __shared__ float xs[4 * G];
+  __shared__ float tab[G * 32];
   __shared__ uint32_t mw[256][W + 1];  // the block's rows' words (padded: conflict-free row reads)
   // XMAP: a one-dimensional grid, workgroup i dispatched to XCD i % 8, and
   // every chunk of a row block on the XCD of that block (rb % 8), so the
@@ -366,15 +364,15 @@ __global__ __launch_bounds__(256) void sp24_gemv_kernel(const uint32_t *__restri
   // in issue order, so the tabulation waits only for the activations and
   // runs while the metadata streams in (11008 x 4096, one token: the table
   // was ready only after all 16 KB of a workgroup's metadata had landed)
-  constexpr int XPT = (MT * 4 * G + 255) / 256;  // activations per thread
+  constexpr int XPT = (4 * G + 255) / 256;  // activations per thread
   float xv[XPT];
 #pragma unroll
   for (int q = 0; q < XPT; q++) {
-    const int i = (int)threadIdx.x + 256 * q, m = i / (4 * G), c = i - m * 4 * G;
+    const int i = (int)threadIdx.x + 256 * q;
     xv[q] = 0.f;
-    if (i < MT * 4 * G && m < M && c0 + c < K) {
-      if constexpr (sizeof(XT) == 2) xv[q] = __uint_as_float((uint32_t)x[(size_t)m * K + c0 + c] << 16);
-      else xv[q] = x[(size_t)m * K + c0 + c];
+    if (i < 4 * G && c0 + i < K) {
+      if constexpr (sizeof(XT) == 2) xv[q] = __uint_as_float((uint32_t)x[c0 + i] << 16);
+      else xv[q] = x[c0 + i];
     }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -393,15 +391,15 @@ __global__ __launch_bounds__(256) void sp24_gemv_kernel(const uint32_t *__restri
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int q = 0; q < XPT; q++) {
-    const int i = (int)threadIdx.x + 256 * q, m = i / (4 * G), c = i - m * 4 * G;
-    if (i < MT * 4 * G) xs[m][c] = xv[q];
+    const int i = (int)threadIdx.x + 256 * q;
+    if (i < 4 * G) xs[i] = xv[q];
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < MT * G * 32; i += 256) {
-    const int m = i / (G * 32), r = i - m * G * 32, gl = r >> 5, code = r & 31;
+  for (int i = threadIdx.x; i < G * 32; i += 256) {
+    const int gl = i >> 5, code = i & 31;
     const uint32_t nib = __builtin_amdgcn_ubfe(0xEEED9C84u, (uint32_t)(code & 7) << 2, 4);
-    const float a = xs[m][4 * gl + (nib & 3)], b = xs[m][4 * gl + (nib >> 2)];
-    tab[m][r] = 2.0f * ((code & 8 ? -a : a) + (code & 16 ? -b : b));
+    const float a = xs[4 * gl + (nib & 3)], b = xs[4 * gl + (nib >> 2)];
+    tab[i] = 2.0f * ((code & 8 ? -a : a) + (code & 16 ? -b : b));
   }
 #pragma unroll
   for (int i = 0; i < 4; i++)
@@ -412,18 +410,15 @@ __global__ __launch_bounds__(256) void sp24_gemv_kernel(const uint32_t *__restri
   uint32_t wq[W];
 #pragma unroll
   for (int w = 0; w < W; w++) wq[w] = mw[threadIdx.x][w];
-  // two chains per token (even and odd words), added at the end
-  float acc[MT][2];
-#pragma unroll
-  for (int m = 0; m < MT; m++) acc[m][0] = acc[m][1] = 0.f;
+  // two chains (even and odd words), added at the end
+  float acc[2] = {0.f, 0.f};
 #pragma unroll
   for (int w = 0; w < W; w++) {
     if (w >= nw) break;
 #pragma unroll
     for (int q = 0; q < 6; q++) {
       const uint32_t code = (wq[w] >> (5 * q)) & 31u;
-#pragma unroll
-      for (int m = 0; m < MT; m++) acc[m][w & 1] += tab[m][(w * 6 + q) * 32 + code];
+      acc[w & 1] += tab[(w * 6 + q) * 32 + code];
     }
   }
   // the chunk's sums, stored device-coherent (the workgroup that adds the
@@ -432,13 +427,9 @@ __global__ __launch_bounds__(256) void sp24_gemv_kernel(const uint32_t *__restri
   // workgroup for the next launch)
   constexpr int SC1 = 16;  // cache policy: performed at the point of coherence of all XCDs
   constexpr uint32_t OOB = 0x80000000u;
-  const __amdgpu_buffer_rsrc_t pr = buffer_rsrc(part, (uint32_t)S * (uint32_t)M * (uint32_t)N * 4u);
-#pragma unroll
-  for (int m = 0; m < MT; m++) {
-    const uint32_t off =
-        (m < M && row < N) ? (((uint32_t)chunk * (uint32_t)M + (uint32_t)m) * (uint32_t)N + (uint32_t)row) * 4u : OOB;
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[m][0] + acc[m][1]), pr, off, 0, SC1);
-  }
+  const __amdgpu_buffer_rsrc_t pr = buffer_rsrc(part, (uint32_t)S * (uint32_t)N * 4u);
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[0] + acc[1]), pr,
+                                        row < N ? ((uint32_t)chunk * (uint32_t)N + (uint32_t)row) * 4u : OOB, 0, SC1);
   if (!counters) return;  // a separate launch adds the chunks
   __shared__ int last;
   wait_vmcnt<0>();
@@ -451,92 +442,67 @@ __global__ __launch_bounds__(256) void sp24_gemv_kernel(const uint32_t *__restri
   __syncthreads();
   if (!last || row >= N) return;
   const float sc = 0.5f * scale[row];  // 0.5 undoes the 2 dec(c) scale of the table
+  // every chunk's partial in flight at once (the fused path takes up to
+  // SPV_FUSED_MAX chunks): one round trip to the point of coherence
+  float v[SPV_FUSED_MAX], sum = 0.f;
 #pragma unroll
-  for (int m = 0; m < MT; m++) {
-    if (m >= M) break;
-    // every chunk's partial in flight at once (the fused path takes up to
-    // SPV_FUSED_MAX chunks): one round trip to the point of coherence
-    float sum = 0.f;
-    for (int c0 = 0; c0 < S; c0 += SPV_FUSED_MAX) {
-      float v[SPV_FUSED_MAX];
+  for (int k = 0; k < SPV_FUSED_MAX; k++)
+    v[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+        pr, k < S ? ((uint32_t)k * (uint32_t)N + (uint32_t)row) * 4u : OOB, 0, SC1));
 #pragma unroll
-      for (int k = 0; k < SPV_FUSED_MAX; k++) {
-        const uint32_t off = c0 + k < S ? (((uint32_t)(c0 + k) * (uint32_t)M + (uint32_t)m) * (uint32_t)N +
-                                           (uint32_t)row) * 4u
-                                        : OOB;
-        v[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(pr, off, 0, SC1));
-      }
-#pragma unroll
-      for (int k = 0; k < SPV_FUSED_MAX; k++)
-        if (c0 + k < S) sum = (c0 + k == 0) ? v[k] : sum + v[k];
-    }
-    const float o = sum * sc;
-    if constexpr (sizeof(YT) == 4) Y[(size_t)m * N + row] = o;
-    else Y[(size_t)m * N + row] = (uint16_t)bf16_rne(o);
-  }
+  for (int k = 0; k < SPV_FUSED_MAX; k++)
+    if (k < S) sum = k == 0 ? v[k] : sum + v[k];
+  const float o = sum * sc;
+  if constexpr (sizeof(YT) == 4) Y[row] = o;
+  else Y[row] = (uint16_t)bf16_rne(o);
 }
 
-// 1-2 tokens, or 3-4 fp32 tokens over matrices of 32 M codes and more with
-// rows up to 16384 (bf16 ones are faster on the sparse pipe, split over K:
-// 16.8 against about 21 us at 11008 x 4096; fp32 ones there run twice, as hi
-// and lo: 28 against 21.5 us; at 4096 x 4096 and 8192 x 28672 the split
-// stays ahead: 16.3 / 68 against 17.3 / 84 us)
-bool sp24_gemv_plan(int M, int K, int N, int xt_bf16, int *S) {
-  if (M < 1 || K % 4 != 0 || N % 4 != 0 || (N + 255) / 256 > GEMV_SK_MAX_TILES) return false;
-  if (M > 2 && (xt_bf16 || M > 4 || K > 16384 || (long)N * K < (1L << 25))) return false;
-  const int wpr = ((K >> 2) + 5) / 6, w = M <= 2 ? spv_words<2>() : spv_words<4>();
+// One token over tall matrices: its grid of 256-row blocks then covers the
+// compute units and a code costs one LDS read and one add. Below 8192 rows,
+// and from two tokens, the sparse pipe is ahead (frx_sp24.hip): 4096 x 4096
+// f32 / bf16 7.6 / 7.8 here against 7.1 / 6.9 us, 4096 x 11008 9.7 / 9.7
+// against 9.4 / 8.9, 11008 x 4096 8.8 / 8.9 against 10.5 / 9.9.
+bool sp24_gemv_plan(int M, int K, int N, int *S) {
+  if (M != 1 || N < 8192 || K % 4 != 0 || N % 4 != 0 || (N + 255) / 256 > GEMV_SK_MAX_TILES) return false;
+  const int wpr = ((K >> 2) + 5) / 6;
   if ((long)N * wpr * 4 >= (1L << 32)) return false;  // the metadata's buffer range
-  *S = (wpr + w - 1) / w;
+  *S = (wpr + SPV_WORDS - 1) / SPV_WORDS;
   return true;
 }
 
 hipError_t launch_sp24_gemv(const uint32_t *meta, const float *scale, const void *x, int xt_bf16, void *y,
-                            int yt_bf16, int M, int K, int N, int S, float *part, unsigned *counters,
-                            hipStream_t stream) {
-  // the XCD-grouped order for 1-2 tokens where the plain order spreads a row
-  // block's chunks (with nrb % 8 == 0 it already keeps them on one XCD); at
-  // 3-4 tokens (about 66 KB of LDS, two workgroups per CU) grouping 43 row
-  // blocks put 66 workgroups on the 64 slots of some XCDs (11008 x 4096, 4
-  // f32 tokens: 20.5 -> 28.2 us)
+                            int yt_bf16, int K, int N, int S, float *part, unsigned *counters, hipStream_t stream) {
+  // the XCD-grouped order where the plain order spreads a row block's chunks
+  // (with nrb % 8 == 0 it already keeps them on one XCD)
   const int nrb = (N + 255) / 256;
-  const bool xmap = M <= 2 && nrb % 8 != 0;
+  const bool xmap = nrb % 8 != 0;
   const dim3 g = xmap ? dim3(8 * S * ((nrb + 7) / 8)) : dim3(nrb, S);
+  const bool fused = S <= SPV_FUSED_MAX;
+  if (!fused) counters = nullptr;
   auto run = [&](auto xp, auto yp) {
     using XT = std::remove_const_t<std::remove_pointer_t<decltype(xp)>>;
     using YT = std::remove_pointer_t<decltype(yp)>;
-    if (M == 1 && xmap)
-      hipLaunchKernelGGL((sp24_gemv_kernel<XT, 1, YT, true>), g, dim3(256), 0, stream, meta, xp, part, counters, scale,
-                         yp, M, N, K, S);
-    else if (M == 1)
-      hipLaunchKernelGGL((sp24_gemv_kernel<XT, 1, YT, false>), g, dim3(256), 0, stream, meta, xp, part, counters,
-                         scale, yp, M, N, K, S);
-    else if (M == 2 && xmap)
-      hipLaunchKernelGGL((sp24_gemv_kernel<XT, 2, YT, true>), g, dim3(256), 0, stream, meta, xp, part, counters, scale,
-                         yp, M, N, K, S);
-    else if (M == 2)
-      hipLaunchKernelGGL((sp24_gemv_kernel<XT, 2, YT, false>), g, dim3(256), 0, stream, meta, xp, part, counters,
-                         scale, yp, M, N, K, S);
+    if (xmap)
+      hipLaunchKernelGGL((sp24_gemv_kernel<XT, YT, true>), g, dim3(256), 0, stream, meta, xp, part, counters, scale, yp,
+                         N, K, S);
     else
-      hipLaunchKernelGGL((sp24_gemv_kernel<XT, 4, YT, false>), g, dim3(256), 0, stream, meta, xp, part, counters,
-                         scale, yp, M, N, K, S);
+      hipLaunchKernelGGL((sp24_gemv_kernel<XT, YT, false>), g, dim3(256), 0, stream, meta, xp, part, counters, scale,
+                         yp, N, K, S);
   };
   auto runx = [&](auto yp) {
     if (xt_bf16) run(reinterpret_cast<const uint16_t *>(x), yp);
     else run(reinterpret_cast<const float *>(x), yp);
   };
-  const bool fused = S <= SPV_FUSED_MAX;
-  if (!fused) counters = nullptr;
   if (yt_bf16) runx(reinterpret_cast<uint16_t *>(y));
   else runx(reinterpret_cast<float *>(y));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || fused) return e;
-  const size_t quads = (size_t)M * N / 4;
-  const dim3 gr((unsigned)((quads + 255) / 256));
+  const dim3 gr((unsigned)(((size_t)N / 4 + 255) / 256));
   if (yt_bf16)
-    hipLaunchKernelGGL(gemm_splitk_reduce<uint16_t>, gr, dim3(256), 0, stream, part, S, M, N, scale, nullptr,
+    hipLaunchKernelGGL(gemm_splitk_reduce<uint16_t>, gr, dim3(256), 0, stream, part, S, 1, N, scale, nullptr,
                        reinterpret_cast<uint16_t *>(y));
   else
-    hipLaunchKernelGGL(gemm_splitk_reduce<float>, gr, dim3(256), 0, stream, part, S, M, N, scale, nullptr,
+    hipLaunchKernelGGL(gemm_splitk_reduce<float>, gr, dim3(256), 0, stream, part, S, 1, N, scale, nullptr,
                        reinterpret_cast<float *>(y));
   return hipGetLastError();
 }

@@ -124,13 +124,21 @@ hipError_t launch_gemm_sp_splitk(const uint32_t *meta, const float *scale, const
 // metadata), one K loop of 2K columns.
 hipError_t launch_gemm_sp_planes(const uint32_t *meta, int prepared, const float *scale, const uint16_t *x2, void *y,
                                  int yt_bf16, int M, int K, int N, hipStream_t stream);
-// 1-2 tokens (3-4 fp32 tokens) over 2:4 metadata (GPU 5-bit layout, K % 4
-// == 0, N % 4 == 0): S chunk partials of M * N fp32 in part, added in order
-// into y by the last chunk of each 256-row block (counters: the split-K
-// GEMV's, zero between launches).
-bool sp24_gemv_plan(int M, int K, int N, int xt_bf16, int *S);
+// One token over tall 2:4 matrices (GPU 5-bit layout, K % 4 == 0, N % 4 ==
+// 0): S chunk partials of N fp32 in part, added in order into y by the last
+// chunk of each 256-row block (counters: the split-K GEMV's, zero between
+// launches).
+bool sp24_gemv_plan(int M, int K, int N, int *S);
 hipError_t launch_sp24_gemv(const uint32_t *meta, const float *scale, const void *x, int xt_bf16, void *y,
-                            int yt_bf16, int M, int K, int N, int S, float *part, unsigned *counters,
+                            int yt_bf16, int K, int N, int S, float *part, unsigned *counters, hipStream_t stream);
+// A decode batch over 2:4 metadata (GPU 5-bit layout, or prepared with bf16 x)
+// on the sparse pipe (frx_sp24.hip): slices of ncs 16-byte loads per lane, S
+// of them; part: sp24_rows_workspace_bytes; counters: the split-K GEMV's.
+constexpr int SP24_ROWS_MAX_BF16 = 32, SP24_ROWS_MAX_F32 = 24;  // most tokens
+bool sp24_rows_plan(int M, int K, int N, int xt_bf16, int prepared, int cus, int *ncs, int *S);
+size_t sp24_rows_workspace_bytes(int M, int N, int S);
+hipError_t launch_sp24_rows(const uint32_t *w, int prepared, const float *scale, const void *x, int xt_bf16, void *y,
+                            int yt_bf16, int M, int K, int N, int ncs, int S, float *part, unsigned *counters,
                             hipStream_t stream);
 // 2:4 metadata (GPU 5-bit layout) -> its prepared form, [N][K/16] words
 // (K % 64 == 0), and the whole-K GEMM over it (bf16 x, aligned).

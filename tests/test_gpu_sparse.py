@@ -89,6 +89,31 @@ def test_sparse_decode_gemv_ragged(ctx, M, K, N, xt, yt):
         assert_bf16_within_1ulp(y.view(torch.int16).cpu().numpy().view(np.uint16), ref)
 
 
+@pytest.mark.parametrize("M,K,N,xt", [(1, 100, 12, "bf16"), (2, 4, 1, "f32"), (8, 4100, 129, "f32"), (9, 396, 131, "f32"),
+                                      (16, 388, 260, "bf16"), (17, 1540, 514, "bf16"), (24, 6004, 255, "f32"),
+                                      (32, 772, 8196, "bf16"), (3, 14340, 127, "bf16"), (1, 5000, 8196, "f32")])
+@pytest.mark.parametrize("yt", ["f32", "bf16"])
+def test_sparse_row_tiles_ragged(ctx, M, K, N, xt, yt):
+    """The decode-batch row tiles at their edges: rows that end inside a
+    16-byte metadata load or a chunk, K % 8 == 4 (half an activation load past
+    the row), N not a multiple of 4, partly filled column sets, every chunk
+    count of a slice; twice (the arrival counters are left at zero)."""
+    name = f"sp24/rows/{M}x{K}x{N}"
+    t = synth.sparse24_uniform(name, "w", N, K)
+    meta = frx.pack_sparse24_gpu(t)
+    s = synth.row_scales(name, "s", N, samples=min(K, 256))
+    xf, xb = synth.activations(name, "x", M, K)
+    if xt == "f32":
+        xf = synth.normal(13, M * K).reshape(M, K)
+    ref = oracle.sparse24_gpu_matmul(meta, s, xf, M, K, N)
+    for _ in range(2):
+        y = _run(ctx, meta, s, xf, xb, xt, yt)
+        if yt == "f32":
+            assert_close_f32(host(y), ref)
+        else:
+            assert_bf16_within_1ulp(y.view(torch.int16).cpu().numpy().view(np.uint16), ref)
+
+
 @pytest.mark.parametrize("M,K,N", [(2048, 4096, 4096), (2048, 4096, 11008), (16, 4096, 11008), (64, 11008, 512)])
 def test_sparse_bit_exact_on_dyadic(ctx, M, K, N):
     """Whole output, bit for bit (dyadic x, power-of-two scales: every
