@@ -336,7 +336,8 @@ class Context:
 
     def ternary_linear_group(self, x, ws, scales, ys):
         """frx_ternary_linear_group: y_i = x W_i^T * s_i for up to four
-        matrices with the same K against one x (one launch at one token)."""
+        matrices with the same K against one x (one launch at one token and
+        for decode batches)."""
         M, K = _shape2(x, "x")
         count = len(ws)
         if not (len(scales) == len(ys) == count):

@@ -553,6 +553,24 @@ frx_status frx_ternary_linear_bias(frx_ctx *ctx, const uint32_t *w, const float 
   return ternary_linear_run(ctx, w, scale, bias, x, xt, y, yt, M, K, N);
 }
 
+// 2-16 tokens: the matrices of a group run as one launch of the staged kernel
+// (x staged once for all their rows, one start-up) where each of them alone
+// would run that kernel, whose order of additions depends on K only, so the
+// outputs are the separate calls' bit for bit; and while a workgroup per compute
+// unit holds all the 16-row tiles, four each. 3 x 4096 x 4096, 5 / 16 bf16
+// tokens 13.6 / 14.2 -> 7.6 / 8.0 us, 2 / 5 / 16 f32 tokens 16.9 / 17.3 / 23.3 ->
+// 9.3 / 9.5 / 11.2; 2 x 11008 x 4096 (1376 tiles) would go from 14.0 / 15.0 to
+// 14.4 / 15.6 (bf16) and from 17.7 / 22.0 to 19.6 / 23.0 (f32).
+static bool group_one_launch(const frx_ctx *ctx, const void *x, frx_dtype xt, uint32_t M, uint32_t K, uint32_t count,
+                             const uint32_t *const *w, const int *n) {
+  size_t rows = 0;
+  for (uint32_t i = 0; i < count; i++) {
+    rows += (size_t)n[i];
+    if (use_split(ctx, w[i], x, M, K, (uint32_t)n[i], xt)) return false;
+  }
+  return rows <= (size_t)64 * ctx->cus && frx::gemv_group_xs_fits(x, xt == FRX_BF16, (int)M, (int)K, (int)count, w, n);
+}
+
 frx_status frx_ternary_linear_group(frx_ctx *ctx, const void *x, frx_dtype xt, uint32_t M, uint32_t K,
                                     uint32_t count, const uint32_t *const *w, const float *const *scale,
                                     const uint32_t *N, void *const *y, frx_dtype yt) {
@@ -572,12 +590,13 @@ frx_status frx_ternary_linear_group(frx_ctx *ctx, const void *x, frx_dtype xt, u
   hipError_t e = hipSuccess;
   int n[frx::GEMV_GROUP_MAX];
   for (uint32_t i = 0; i < count; i++) n[i] = (int)N[i];
-  if (M == 1 && aligned && frx::gemv_group_fits(x, 1, (int)K, (int)count, w, n)) {
+  if (aligned && (M == 1 ? frx::gemv_group_fits(x, 1, (int)K, (int)count, w, n)
+                         : group_one_launch(ctx, x, xt, M, K, count, w, n))) {
     e = frx::launch_gemv_group(x, xt == FRX_BF16, yt == FRX_BF16, (int)M, (int)K, (int)count, w, scale, y, n,
                                ctx->stream);
   } else {
-    // several tokens, prefill, shapes past the one-launch group, or
-    // sub-slices that need staging: one linear per matrix
+    // prefill, shapes past the one-launch groups, or sub-slices that need
+    // staging: one linear per matrix
     for (uint32_t i = 0; i < count; i++)
       if ((st = ternary_linear_run(ctx, w[i], scale[i], nullptr, x, xt, y[i], yt, M, K, N[i])) != FRX_OK) return st;
   }

@@ -1562,12 +1562,13 @@ static hipError_t launch_gemv_rows_pass(const uint32_t *w, const float *scale, c
 constexpr int XS_QUAD_BYTES = 8192;  // one plane of a quad: 16 tokens x 256 bf16
 enum { XS_BF16 = 0, XS_PLANES = 1, XS_F32 = 2 };
 
-template <typename YT, int WAVES, int T, int UMAX, int NW, int EPI, int XS, bool YSPLIT>
+template <typename YT, int WAVES, int T, int UMAX, int NW, int EPI, int XS, bool YSPLIT, bool GRP>
 __global__ __launch_bounds__(WAVES * 64) void gemv_xs_kernel(
     const uint32_t *__restrict__ W, const float *__restrict__ scale, const uint32_t *__restrict__ W2,
     const float *__restrict__ scale2, const void *__restrict__ Xv, const uint16_t *__restrict__ X2,
-    YT *__restrict__ Y, int B, int K, int N, const float *__restrict__ bias) {
+    YT *__restrict__ Y, int B, int K, int N, const float *__restrict__ bias, const GemvGroup grp) {
   static_assert((NW == 2) == (EPI != GEMV_LINEAR), "two matrices exactly for the GLU epilogues");
+  static_assert(!GRP || NW == 1, "a group is several linears");
   static_assert(!YSPLIT || (NW == 2 && sizeof(YT) == 2), "split output is the GLU's bf16 planes");
   constexpr int XP = XS == XS_BF16 ? 1 : 2;  // planes staged per quad
   constexpr int NL = 8 * XP;  // 16-byte loads per lane and quad (fp32: two per piece)
@@ -1575,6 +1576,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_xs_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
+  // the workgroup's rows (GRP: its 16-row tiles; every matrix of the group has
+  // whole tiles of its own, grp.start in tiles, N = their total)
   const int b0 = (int)((long long)blockIdx.x * N / gridDim.x);
   const int b1 = (int)((long long)(blockIdx.x + 1) * N / gridDim.x);
   const int wpr = K >> 4;
@@ -1635,10 +1638,20 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_xs_kernel(
     for (int tt = 0; tt < T; tt++)
 #pragma unroll
       for (int u = 0; u < UMAX; u++) {
-        const int row = b0 + 16 * tt + r, q = qa + u, wi = 16 * q + 4 * g;
-        const uint32_t off =
-            (row < b1 && q < qb && wi < wpr) ? ((uint32_t)row * (uint32_t)wpr + (uint32_t)wi) * 4u : OOB;
-        wv[mw][tt][u] = __builtin_amdgcn_raw_buffer_load_b128(mw ? wr2 : wr, off, 0, 0);
+        const int q = qa + u, wi = 16 * q + 4 * g;
+        if constexpr (GRP) {
+          const int tile = b0 + tt, m = grp.matrix_of(tile), row = (tile - grp.start_of(m)) * 16 + r, n = grp.rows_of(m);
+          const uint32_t off = (tile < b1 && row < n && q < qb && wi < wpr)
+                                   ? ((uint32_t)row * (uint32_t)wpr + (uint32_t)wi) * 4u
+                                   : OOB;
+          wv[mw][tt][u] = __builtin_amdgcn_raw_buffer_load_b128(
+              buffer_rsrc(grp.w_of(m), (uint32_t)n * (uint32_t)wpr * 4u), off, 0, 0);
+        } else {
+          const int row = b0 + 16 * tt + r;
+          const uint32_t off =
+              (row < b1 && q < qb && wi < wpr) ? ((uint32_t)row * (uint32_t)wpr + (uint32_t)wi) * 4u : OOB;
+          wv[mw][tt][u] = __builtin_amdgcn_raw_buffer_load_b128(mw ? wr2 : wr, off, 0, 0);
+        }
       }
   f32x4 acc[NW][T];
 #pragma unroll
@@ -1699,16 +1712,27 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_xs_kernel(
   __syncthreads();
   if (wave < T) {
     const int tt = wave;
-    const int n_out = b0 + 16 * tt + 4 * g;  // rows 4g..4g+3 of token t
-    if (t < B && n_out < b1) {
-      const int nok = min(4, b1 - n_out);
+    int n_out = b0 + 16 * tt + 4 * g, n_end = b1;  // rows 4g..4g+3 of token t
+    int ldy = N;
+    const float *gs = scale;
+    YT *gy = Y;
+    if constexpr (GRP) {
+      const int tile = b0 + tt, m = grp.matrix_of(tile);
+      ldy = grp.rows_of(m);
+      n_out = (tile - grp.start_of(m)) * 16 + 4 * g;
+      n_end = tile < b1 ? ldy : 0;
+      gs = grp.s_of(m);
+      gy = reinterpret_cast<YT *>(grp.y_of(m));
+    }
+    if (t < B && n_out < n_end) {
+      const int nok = min(4, n_end - n_out);
       f32x4 v[NW];
 #pragma unroll
       for (int mw = 0; mw < NW; mw++) {
         const f32x4 *rp = red + (mw * T + tt) * WAVES * 64 + lane;
         f32x4 s = rp[0];
         for (int w = 1; w < WAVES; w++) s += rp[w * 64];
-        const float *sp2 = mw ? scale2 : scale;
+        const float *sp2 = mw ? scale2 : gs;
         const f32x4 sc = {sp2[n_out], nok > 1 ? sp2[n_out + 1] : 0.f, nok > 2 ? sp2[n_out + 2] : 0.f,
                           nok > 3 ? sp2[n_out + 3] : 0.f};
         v[mw] = s * sc * 0.5f;  // 0.5: the 2*dec(c) operand encoding
@@ -1728,30 +1752,30 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_xs_kernel(
         YStore<uint16_t>::store4(reinterpret_cast<uint16_t *>(Y) + (size_t)t * N + n_out, hi, nok);
         YStore<uint16_t>::store4(reinterpret_cast<uint16_t *>(Y) + (size_t)B * N + (size_t)t * N + n_out, lo, nok);
       } else {
-        if constexpr (NW == 1)
+        if constexpr (NW == 1 && !GRP)
           if (bias) o = add_bias4(o, bias, n_out, N);
-        YStore<YT>::store4(Y + (size_t)t * N + n_out, o, nok);
+        YStore<YT>::store4(gy + (size_t)t * ldy + n_out, o, nok);
       }
     }
   }
 }
 
-template <typename YT, int WAVES, int T, int UMAX, int NW, int EPI, int XS, bool YSPLIT>
+template <typename YT, int WAVES, int T, int UMAX, int NW, int EPI, int XS, bool YSPLIT, bool GRP>
 static hipError_t launch_gemv_xs_w(const uint32_t *w, const float *scale, const uint32_t *w2, const float *scale2,
                                    const void *x, const void *x2, void *y, int B, int K, int N, int G,
-                                   hipStream_t stream, const float *bias) {
+                                   hipStream_t stream, const float *bias, const GemvGroup &grp) {
   constexpr int XP = XS == XS_BF16 ? 1 : 2;
   static_assert(NW * T * 1024 <= XP * XS_QUAD_BYTES, "the partial tiles reuse the staging area");
   const size_t lds = (size_t)WAVES * XP * XS_QUAD_BYTES;
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> done;
     const hipError_t e = opt_in_lds(
-        reinterpret_cast<const void *>(&gemv_xs_kernel<YT, WAVES, T, UMAX, NW, EPI, XS, YSPLIT>), (int)lds, done);
+        reinterpret_cast<const void *>(&gemv_xs_kernel<YT, WAVES, T, UMAX, NW, EPI, XS, YSPLIT, GRP>), (int)lds, done);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((gemv_xs_kernel<YT, WAVES, T, UMAX, NW, EPI, XS, YSPLIT>), dim3(G), dim3(WAVES * 64), lds,
+  hipLaunchKernelGGL((gemv_xs_kernel<YT, WAVES, T, UMAX, NW, EPI, XS, YSPLIT, GRP>), dim3(G), dim3(WAVES * 64), lds,
                      stream, w, scale, w2, scale2, x, reinterpret_cast<const uint16_t *>(x2),
-                     reinterpret_cast<YT *>(y), B, K, N, bias);
+                     reinterpret_cast<YT *>(y), B, K, N, bias, grp);
   return hipGetLastError();
 }
 
@@ -1777,17 +1801,20 @@ static int gemv_xs_grid(int N, int tmax) {
 // 4096x11008, B = 16); 16 waves of four above. Two planes (16 KB per wave)
 // or two matrices (twice the weight registers): 8 waves of up to 2, 4 or 6
 // quads, so that a wave has 256 registers.
-template <typename YT, int NW, int EPI, int XS, bool YSPLIT>
+// grp: the matrices of a same-x group (N = their 16-row tiles), else null.
+template <typename YT, int NW, int EPI, int XS, bool YSPLIT, bool GRP = false>
 static hipError_t launch_gemv_xs(const uint32_t *w, const float *scale, const uint32_t *w2, const float *scale2,
                                  const void *x, const void *x2, void *y, int B, int K, int N, hipStream_t stream,
-                                 const float *bias = nullptr) {
-  const int nq = (K + 255) / 256;
-#define FRX_XS(WV, TT, UM)                                                                                    \
-  return launch_gemv_xs_w<YT, WV, TT, UM, NW, EPI, XS, YSPLIT>(w, scale, w2, scale2, x, x2, y, B, K, N, \
-                                                                gemv_xs_grid(N, TT), stream, bias)
-#define FRX_XS_T(WV, UM, TMAX)                                                               \
-  {                                                                                          \
-    const int tiles = ((N + gemv_xs_grid(N, TMAX) - 1) / gemv_xs_grid(N, TMAX) + 15) / 16; \
+                                 const float *bias = nullptr, const GemvGroup *grp = nullptr) {
+  const int nq = (K + 255) / 256, rows = GRP ? 16 * N : N;
+  const GemvGroup none{};
+#define FRX_XS(WV, TT, UM)                                                                                         \
+  return launch_gemv_xs_w<YT, WV, TT, UM, NW, EPI, XS, YSPLIT, GRP>(w, scale, w2, scale2, x, x2, y, B, K, N,       \
+                                                                    gemv_xs_grid(rows, TT), stream, bias,          \
+                                                                    GRP ? *grp : none)
+#define FRX_XS_T(WV, UM, TMAX)                                                                        \
+  {                                                                                                   \
+    const int tiles = ((rows + gemv_xs_grid(rows, TMAX) - 1) / gemv_xs_grid(rows, TMAX) + 15) / 16; \
     if (tiles <= 1 || TMAX == 1) FRX_XS(WV, 1, UM);                                          \
     if (tiles <= 2 || TMAX == 2) FRX_XS(WV, (TMAX >= 2 ? 2 : 1), UM);                        \
     if (tiles <= 3 || TMAX == 3) FRX_XS(WV, (TMAX >= 3 ? 3 : 1), UM);                        \
@@ -2265,11 +2292,21 @@ bool gemv_group_fits(const void *x, int B, int K, int count, const uint32_t *con
   return gemv_group_grid(x, B, K, count, w, N, &total, &G);
 }
 
+bool gemv_group_xs_fits(const void *x, int xt_bf16, int B, int K, int count, const uint32_t *const *w,
+                        const int *N) {
+  // the token counts and rows that launch_gemv sends to the staged kernel
+  bool ok = count >= 2 && count <= GEMV_GROUP_MAX && B >= (xt_bf16 ? GEMV_XS_MIN_B : 2) && B <= 16 &&
+            gemv_xs_ok(x, B, K, xt_bf16 ? 1 : 2, 1);
+  for (int i = 0; i < count && ok; i++)
+    ok = (reinterpret_cast<uintptr_t>(w[i]) & 3) == 0 && (size_t)N[i] * K / 4 < ((size_t)1 << 31);
+  return ok;
+}
+
 hipError_t launch_gemv_group(const void *x, int xt_bf16, int yt_bf16, int B, int K, int count,
                              const uint32_t *const *w, const float *const *s, void *const *y, const int *N,
                              hipStream_t stream) {
   int total = 0, G = 0;
-  if (gemv_group_grid(x, B, K, count, w, N, &total, &G)) {
+  if (B == 1 && gemv_group_grid(x, B, K, count, w, N, &total, &G)) {
     GemvGroup g{};
     int st = 0;
     for (int i = 0; i < GEMV_GROUP_MAX; i++) {
@@ -2286,11 +2323,31 @@ hipError_t launch_gemv_group(const void *x, int xt_bf16, int yt_bf16, int B, int
     if (yt_bf16) return launch_gemv_bal<uint16_t, true, true>(w[0], s[0], x, y[0], K, total, G, stream, nullptr, &g);
     return launch_gemv_bal<float, true, true>(w[0], s[0], x, y[0], K, total, G, stream, nullptr, &g);
   }
-  for (int i = 0; i < count; i++) {
-    const hipError_t e = launch_gemv(w[i], s[i], x, xt_bf16, y[i], yt_bf16, B, K, N[i], stream, nullptr);
-    if (e != hipSuccess) return e;
+  if (!gemv_group_xs_fits(x, xt_bf16, B, K, count, w, N)) return hipErrorInvalidValue;
+  GemvGroup g{};
+  int tiles = 0;
+  for (int i = 0; i < GEMV_GROUP_MAX; i++) {
+    const int k = i < count ? i : 0;
+    g.w[i] = w[k];
+    g.s[i] = s[k];
+    g.y[i] = y[k];
+    g.rows[i] = N[k];
+    g.start[i] = i < count ? tiles : 0x7fffffff;
+    if (i < count) tiles += (N[i] + 15) / 16;
   }
-  return hipSuccess;
+  constexpr int L = GEMV_LINEAR;
+  if (xt_bf16) {
+    if (yt_bf16)
+      return launch_gemv_xs<uint16_t, 1, L, XS_BF16, false, true>(w[0], s[0], w[0], s[0], x, x, y[0], B, K, tiles, stream,
+                                                                  nullptr, &g);
+    return launch_gemv_xs<float, 1, L, XS_BF16, false, true>(w[0], s[0], w[0], s[0], x, x, y[0], B, K, tiles, stream,
+                                                             nullptr, &g);
+  }
+  if (yt_bf16)
+    return launch_gemv_xs<uint16_t, 1, L, XS_F32, false, true>(w[0], s[0], w[0], s[0], x, x, y[0], B, K, tiles, stream,
+                                                               nullptr, &g);
+  return launch_gemv_xs<float, 1, L, XS_F32, false, true>(w[0], s[0], w[0], s[0], x, x, y[0], B, K, tiles, stream,
+                                                          nullptr, &g);
 }
 
 hipError_t launch_gemv_glu(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up,

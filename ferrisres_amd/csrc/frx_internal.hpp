@@ -49,7 +49,9 @@ struct GemvGroup {
   const uint32_t *w[GEMV_GROUP_MAX];
   const float *s[GEMV_GROUP_MAX];
   void *y[GEMV_GROUP_MAX];
-  int start[GEMV_GROUP_MAX];  // first row of each matrix in the launch; 0x7fffffff past the group
+  int start[GEMV_GROUP_MAX];  // first row of each matrix in the launch (several tokens: first 16-row
+                              // tile); 0x7fffffff past the group
+  int rows[GEMV_GROUP_MAX];   // rows of each matrix (several tokens)
   // matrix holding launch row r (r below the total)
   __host__ __device__ __forceinline__ int matrix_of(int r) const {
     int m = 0;
@@ -68,6 +70,7 @@ struct GemvGroup {
   __host__ __device__ __forceinline__ const float *s_of(int m) const { return pick(s, m); }
   __host__ __device__ __forceinline__ void *y_of(int m) const { return pick(y, m); }
   __host__ __device__ __forceinline__ int start_of(int m) const { return pick(start, m); }
+  __host__ __device__ __forceinline__ int rows_of(int m) const { return pick(rows, m); }
   // weights, scales and first launch row of the matrix holding launch row r,
   // as a chain of selects on r (the starts ascend, so the last start <= r
   // wins): a wave-uniform r gives scalar selects and no branches (a select
@@ -90,6 +93,8 @@ struct GemvGroup {
 // 64 == 0 up to 16384, rows within the slots); else launch_gemv_group runs
 // one launch per matrix.
 bool gemv_group_fits(const void *x, int B, int K, int count, const uint32_t *const *w, const int *N);
+// 2-16 tokens: one launch over the 16-row tiles of all matrices.
+bool gemv_group_xs_fits(const void *x, int xt_bf16, int B, int K, int count, const uint32_t *const *w, const int *N);
 hipError_t launch_gemv_group(const void *x, int xt_bf16, int yt_bf16, int B, int K, int count,
                              const uint32_t *const *w, const float *const *s, void *const *y, const int *N,
                              hipStream_t stream);

@@ -164,7 +164,9 @@ frx_status frx_ternary_linear_bias(frx_ctx *ctx, const uint32_t *w,
  * At one token (bf16 or f32 x, K % 64 == 0 up to 16384, 16-byte aligned
  * weights, x, scales and outputs) the group is one launch over the
  * matrices' concatenated rows, so x is read once and the launch's fixed
- * cost is paid once; otherwise each matrix runs as frx_ternary_linear. */
+ * cost is paid once; so is a group at 5-16 bf16 (2-16 f32) tokens whose
+ * matrices would each run the staged decode GEMV; otherwise each matrix runs
+ * as frx_ternary_linear. The outputs are the separate calls' bit for bit. */
 frx_status frx_ternary_linear_group(frx_ctx *ctx, const void *x, frx_dtype xt, uint32_t M,
                                     uint32_t K, uint32_t count, const uint32_t *const *w,
                                     const float *const *scale, const uint32_t *N, void *const *y,

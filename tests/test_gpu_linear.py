@@ -479,6 +479,31 @@ def test_linear_group_equals_separate_calls(ctx, M, K, Ns, xt, yt):
             assert_close_f32(host(y), ref)
 
 
+@pytest.mark.parametrize("M,K,Ns,xt,yt", [
+    (5, 4096, (4096, 1024, 1000), "bf16", "bf16"), (16, 1040, (33, 16, 7, 520), "bf16", "f32"),
+    (6, 8192, (3000, 5000), "bf16", "f32"), (16, 14336, (1024, 2048), "bf16", "bf16"), (9, 16, (5, 3000), "bf16", "f32"),
+    (2, 2048, (2048, 2048, 2048), "f32", "f32"), (16, 4096, (4096, 4096, 4096), "f32", "f32"),
+    (5, 1104, (17, 1031), "f32", "bf16"), (8, 4096, (11008, 11008), "f32", "f32"), (5, 5120, (512, 300), "f32", "f32")])
+def test_linear_group_of_a_decode_batch(ctx, M, K, Ns, xt, yt):
+    """The one-launch group of 2-16 tokens: ragged rows (every matrix has whole
+    16-row tiles of its own), one to four tiles per workgroup, every wave split
+    of K, and the shapes that stay separate: the separate calls' outputs bit
+    for bit."""
+    g = torch.Generator(device="cuda:0").manual_seed(M * K)
+    x = torch.randn((M, K), generator=g, device="cuda:0").to(torch.bfloat16 if xt == "bf16" else torch.float32)
+    ydt = torch.bfloat16 if yt == "bf16" else torch.float32
+    ws = [torch.randint(-2 ** 31, 2 ** 31 - 1, (n, K // 16), generator=g, device="cuda:0", dtype=torch.int32) for n in Ns]
+    ss = [torch.rand(n, generator=g, device="cuda:0") for n in Ns]
+    ys = [torch.full((M, n), float("nan"), dtype=ydt, device="cuda:0") for n in Ns]
+    sep = [torch.empty((M, n), dtype=ydt, device="cuda:0") for n in Ns]
+    ctx.ternary_linear_group(x, ws, ss, ys)
+    for w, s, y in zip(ws, ss, sep):
+        ctx.ternary_linear(w, s, x, y)
+    torch.cuda.synchronize()
+    for y, y2 in zip(ys, sep):
+        np.testing.assert_array_equal(host(y.float()), host(y2.float()))
+
+
 def test_linear_group_errors(ctx):
     x = torch.zeros((1, 64), dtype=torch.bfloat16, device="cuda:0")
     w = torch.zeros((8, 4), dtype=torch.int32, device="cuda:0")
