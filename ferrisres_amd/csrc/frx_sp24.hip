@@ -94,7 +94,7 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
   const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(W, (uint32_t)N * (uint32_t)wpr * 4u);
   // 8-column pieces of a set's tokens, zeros past M and K and past the slice
   // (pieces past the set repeat the last one)
-  u32x4 xv[XR][XL];
+  u32x4 xv[SETS][XR][XL];
   auto xload = [&](int set) {
 #pragma unroll
     for (int r = 0; r < XR; r++) {
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
       const uint32_t e = ((uint32_t)t * (uint32_t)K + (uint32_t)col) * (uint32_t)sizeof(XT);
 #pragma unroll
       for (int l = 0; l < XL; l++)
-        xv[r][l] = __builtin_amdgcn_raw_buffer_load_b128(xr, ok && (!l || col + 4 < K) ? e + 16u * l : SPR_OOB, 0, 0);
+        xv[set][r][l] = __builtin_amdgcn_raw_buffer_load_b128(xr, ok && (!l || col + 4 < K) ? e + 16u * l : SPR_OOB, 0, 0);
     }
   };
   auto xstore = [&](int set) {
@@ -115,14 +115,14 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           uint32_t h, l;
-          split2_bf16(__uint_as_float(xv[r][q >> 1][2 * (q & 1)]), __uint_as_float(xv[r][q >> 1][2 * (q & 1) + 1]), h,
+          split2_bf16(__uint_as_float(xv[set][r][q >> 1][2 * (q & 1)]), __uint_as_float(xv[set][r][q >> 1][2 * (q & 1) + 1]), h,
                       l);
           hi[q] = h;
           lo[q] = l;
         }
         *reinterpret_cast<u32x4 *>(xs + (row + 8) * STRIDE + o) = lo;
       } else {
-        hi = xv[r][0];
+        hi = xv[set][r][0];
         // K % 8 == 4: the second half of the last piece is the next row's
         const uint32_t keep = k0 + o + 4 < K ? 0xFFFFFFFFu : 0u;
         hi.z &= keep;
@@ -133,7 +133,8 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
   };
   // activations first (vector loads complete in issue order), then the wave's
   // metadata, every chunk of the slice
-  xload(0);
+#pragma unroll
+  for (int set = 0; set < SETS; set++) xload(set);
   __builtin_amdgcn_sched_barrier(0);
   const int i = lane & 15, g = lane >> 4;
   const int row = blockIdx.x * SPR_ROWS + wave * 16 + i;
@@ -144,12 +145,8 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
         wr,
         c < nc && row < N ? ((uint32_t)row * (uint32_t)wpr + (uint32_t)(c0 + c) * 16u + 4u * g) * 4u : SPR_OOB, 0, 0);
   __builtin_amdgcn_sched_barrier(0);
-  xstore(0);
 #pragma unroll
-  for (int set = 1; set < SETS; set++) {
-    xload(set);
-    xstore(set);
-  }
+  for (int set = 0; set < SETS; set++) xstore(set);
   __syncthreads();
   f32x4 acc[SETS][2];
 #pragma unroll
@@ -233,7 +230,8 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
 
 // Chunks per slice: the fewest that keep the grid within three workgroups per
 // compute unit (11008 x 4096, 16 f32 tokens: 16.7 us within two, 14.7 within
-// three) and the slices within one batch of the last workgroup's loads
+// three; the prepared form decodes faster and is ahead within two: 8 / 32
+// tokens 8.5 / 14.5 against 9.4 / 17.0) and the slices within one batch of the last workgroup's loads
 // (prepared 1024 x 14336, 16 tokens: 15.0 us in 56 slices, 8.0 in 14).
 // Measured over the tile engine that served these calls (launches back to
 // back, 4096 x 11008): f32 x, 2 / 8 / 16 / 24 tokens 11.6 / 30.1 / 30.7 / 31.5
@@ -247,7 +245,7 @@ bool sp24_rows_plan(int M, int K, int N, int xt_bf16, int prepared, int cus, int
   if (tiles > GEMV_SK_MAX_TILES || (size_t)N * wpr * 4 >= SPR_OOB || (size_t)M * K * 4 >= SPR_OOB) return false;
   const int ch = spr_chunk(prepared), nch = (K + ch - 1) / ch;
   int n = 1;
-  while (n < SPR_NC && (tiles * ((nch + n - 1) / n) > (size_t)3 * cus || (nch + n - 1) / n > SPR_CG)) n++;
+  while (n < SPR_NC && (tiles * ((nch + n - 1) / n) > (size_t)(prepared ? 2 : 3) * cus || (nch + n - 1) / n > SPR_CG)) n++;
   *ncs = n;
   *S = (nch + n - 1) / n;
   return sp24_rows_workspace_bytes(M, N, *S) < SPR_OOB;
