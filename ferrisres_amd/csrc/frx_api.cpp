@@ -976,12 +976,12 @@ static frx_status check_ffn_down(frx_ctx *ctx, const uint32_t *w_down, const flo
 // the context's barrier words).
 // The down launch over h's bf16 planes [2][M][I] at 3-16 tokens: the split-K
 // GEMV (planes staged once per 128-row tile and column slice) where it
-// measured faster, i.e. I >= 8192, and only where the call may allocate its
+// measured faster, i.e. I > 4096 (FFN_NUMS), and only where the call may allocate its
 // workspace; else the planes kernels of frx_gemv.hip.
 static frx_status ffn_down_planes(frx_ctx *ctx, const uint32_t *w_down, const float *s_down, const uint16_t *hp,
                                   void *y, frx_dtype yt, uint32_t M, uint32_t H, uint32_t I, bool may_alloc) {
   const bool split = may_alloc && ctx->gemv_split != FRX_GEMV_SPLIT_NEVER &&
-                     (ctx->gemv_split == FRX_GEMV_SPLIT_ALWAYS || I >= 8192) &&
+                     (ctx->gemv_split == FRX_GEMV_SPLIT_ALWAYS || I > 4096) &&
                      (H + 127) / 128 <= (uint32_t)frx::GEMV_SK_MAX_TILES && (size_t)M * I * 4 < ((size_t)1 << 32);
   hipError_t e;
   if (split) {
@@ -1003,7 +1003,6 @@ static frx_status ffn_run(frx_ctx *ctx, const void *x, frx_dtype xt, const uint3
                           uint32_t M, uint32_t H, uint32_t I, frx_activation act, void *y, frx_dtype yt, void *ws,
                           float *u_ws, bool allow_one) {
   hipError_t e;
-  const bool two_only = ctx->ffn_mode == FRX_FFN_TWO_LAUNCH || !allow_one;
   // the one-launch kernel's context (allow_one) is the allocating entry point
   const bool may_alloc = allow_one;
   if ((!allow_one || ctx->ffn_mode != FRX_FFN_ONE_LAUNCH) && xt == FRX_BF16 && aligned16(w_gate) &&
@@ -1055,7 +1054,10 @@ static frx_status ffn_run(frx_ctx *ctx, const void *x, frx_dtype xt, const uint3
   }
   int grid = 0;
   size_t lds = 0;
-  const bool one = !two_only && aligned16(w_gate) && aligned16(w_up) && aligned16(w_down) &&
+  // only on request: fp32 x of up to three tokens, which used to take it by
+  // default, is faster in two launches (1024 / 4096 18.4 -> 8.5 us, 2048 / 5632
+  // 19.1 -> 11.3, 4096 / 11008 20.8 -> 18.6)
+  const bool one = allow_one && ctx->ffn_mode == FRX_FFN_ONE_LAUNCH && aligned16(w_gate) && aligned16(w_up) && aligned16(w_down) &&
                    frx::ffn1_supported((int)M, (int)H, (int)I, xt == FRX_BF16, ctx->cus, &grid, &lds);
   if (allow_one && ctx->ffn_mode == FRX_FFN_ONE_LAUNCH && !one)
     return fail(ctx, FRX_ERR_UNSUPPORTED,

@@ -1788,7 +1788,10 @@ static bool gemv_xs_ok(const void *x, int B, int K, int XP, int NW) {
 
 // Grid: one workgroup per CU, fewer where that would leave tiles of fewer
 // than 16 rows, more where a workgroup would hold more tiles than its
-// weight registers allow (tiles x quads per wave x matrices <= 8).
+// weight registers allow (tiles x quads per wave x matrices <= 8, 16 with two
+// matrices: at 11008 rows, 16-row tiles for all of a compute unit's 43 rows, one
+// workgroup each, instead of 344 workgroups on 256 units; the FFN of 16 tokens
+// at 4096 / 11008 25.0 -> 23.4 us bf16, 33.4 -> 27.6 f32).
 static int gemv_xs_grid(int N, int tmax) {
   int G = std::min(device_cu_count(), (N + 15) / 16);
   if ((N + G - 1) / G > 16 * tmax) G = (N + 16 * tmax - 1) / (16 * tmax);
@@ -1830,8 +1833,8 @@ static hipError_t launch_gemv_xs(const uint32_t *w, const float *scale, const ui
     if (nq <= 32) FRX_XS_T(8, 4, 2);
     FRX_XS_T(8, 6, 1);
   } else {
-    if (nq <= 16) FRX_XS_T(8, 2, 2);
-    if (nq <= 32) FRX_XS_T(8, 4, 1);
+    if (nq <= 16) FRX_XS_T(8, 2, 4);
+    if (nq <= 32) FRX_XS_T(8, 4, 2);
     FRX_XS_T(8, 6, 1);
   }
 #undef FRX_XS_T
@@ -2353,14 +2356,16 @@ hipError_t launch_gemv_group(const void *x, int xt_bf16, int yt_bf16, int B, int
 hipError_t launch_gemv_glu(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up,
                            const float *s_up, const void *x, int xt_bf16, float *h, int B, int K,
                            int N, int gelu, hipStream_t stream) {
-  if (xt_bf16 && B >= GEMV_GLU_XS_MIN_B && gemv_xs_ok(x, B, K, 1, 2)) {
+  if (xt_bf16 && B >= gemv_glu_xs_min_b(K) && gemv_xs_ok(x, B, K, 1, 2)) {
     if (gelu)
       return launch_gemv_xs<float, 2, GEMV_GEGLU, XS_BF16, false>(w_gate, s_gate, w_up, s_up, x, x, h, B, K, N,
                                                                    stream);
     return launch_gemv_xs<float, 2, GEMV_SWIGLU, XS_BF16, false>(w_gate, s_gate, w_up, s_up, x, x, h, B, K, N,
                                                                   stream);
   }
-  if (!xt_bf16 && B >= 2 && gemv_xs_ok(x, B, K, 2, 2)) {
+  // fp32 x; one token over more than 4096 columns stays with the 16-row tiles
+  // (5120 / 13824 FFN 31.8 us so, 35.9 staged; 2048 / 5632 11.3 us staged)
+  if (!xt_bf16 && (B >= 2 || K <= 4096) && gemv_xs_ok(x, B, K, 2, 2)) {
     if (gelu)
       return launch_gemv_xs<float, 2, GEMV_GEGLU, XS_F32, false>(w_gate, s_gate, w_up, s_up, x, x, h, B, K, N,
                                                                   stream);
@@ -2403,7 +2408,7 @@ hipError_t launch_glu_combine(const float *g, const float *u, float *h, size_t n
 hipError_t launch_gemv_glu_planes(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up,
                                   const float *s_up, const void *x, uint16_t *h_planes, int B, int K,
                                   int N, int gelu, hipStream_t stream) {
-  if (B >= GEMV_GLU_XS_MIN_B && gemv_xs_ok(x, B, K, 1, 2)) {
+  if (B >= gemv_glu_xs_min_b(K) && gemv_xs_ok(x, B, K, 1, 2)) {
     if (gelu)
       return launch_gemv_xs<uint16_t, 2, GEMV_GEGLU, XS_BF16, true>(w_gate, s_gate, w_up, s_up, x, x, h_planes, B,
                                                                      K, N, stream);

@@ -66,9 +66,8 @@ typedef enum frx_activation {
 } frx_activation;
 /* How frx_ternary_ffn runs at decode sizes (see frx_set_ffn_mode). */
 typedef enum frx_ffn_mode {
-  FRX_FFN_AUTO = 0,        /* M <= 4: two whole-row launches where the
-                              shape allows, else the one-launch kernel at
-                              M <= 3 where it allows; otherwise two */
+  FRX_FFN_AUTO = 0,        /* two launches (M <= 4 bf16: whole-row kernels
+                              where the shape allows) */
   FRX_FFN_ONE_LAUNCH = 1,  /* one launch or FRX_ERR_UNSUPPORTED */
   FRX_FFN_TWO_LAUNCH = 2,  /* gate/up/act launch + down launch */
   FRX_FFN_MODE_RANGE_ = 0x7fffffff
@@ -311,15 +310,14 @@ frx_status frx_ternary_glu(frx_ctx *ctx, const void *x, frx_dtype xt,
  *    14336), 16-byte aligned weights: two launches that read whole weight
  *    rows per wave (4 row segments per MFMA from 2 tokens); h as bf16 hi +
  *    lo planes, |h - hi - lo| <= 2^-17 |h|. At M = 3 and 4 the down launch
- *    is the split-K GEMV over both planes (frx_set_gemv_split) where I >=
- *    8192.
+ *    is the split-K GEMV over both planes (frx_set_gemv_split) where I >
+ *    4096.
  *  - bf16 x, 5 <= M <= 16: gate/up/act launch writing h as bf16 hi + lo
  *    planes (2^-17), then the down GEMV over both planes (split-K where
- *    I >= 8192).
- *  - M = 3 in FRX_FFN_ONE_LAUNCH mode (H <= 4096, I <= 11520, multiples of
+ *    I > 4096).
+ *  - M <= 3 in FRX_FFN_ONE_LAUNCH mode (H <= 4096, I <= 11520, multiples of
  *    64, 16-byte aligned weights): one launch with a grid barrier between
- *    the halves; h as bf16 hi + lo planes (2^-17). Other M <= 3 shapes that
- *    the paths above do not take run it in FRX_FFN_AUTO too.
+ *    the halves; h as bf16 hi + lo planes (2^-17).
  *  - f32 x at M <= 16, and every other shape at M <= 16: h in fp32, then the
  *    down GEMV with fp32 input, as the reference keeps it.
  *  - M > 16: gate and up GEMMs (the up projection in a second context

@@ -340,3 +340,33 @@ def test_ffn_one_launch_unsupported(one_launch):
         ctx.ternary_ffn(dev_bf16(xb), d["gate"][0], d["gate"][1], d["up"][0], d["up"][1], d["down"][0],
                         d["down"][1], y)
     assert ei.value.kind == "Unsupported"
+
+
+@pytest.mark.parametrize("M,H,I,xt", [(1, 1024, 2048, "f32"), (3, 2048, 5632, "f32"), (2, 4096, 16320, "f32"),
+                                      (1, 5120, 1040, "f32"), (5, 2048, 4160, "bf16"), (7, 1024, 8208, "bf16"),
+                                      (16, 4096, 16400, "bf16"), (9, 8192, 8208, "bf16"), (16, 2064, 5632, "f32")])
+def test_ffn_decode_batch_launches(ctx, M, H, I, xt):
+    """The gate/up launch with three and four 16-row tiles per workgroup, its
+    token and width limits, f32 x of up to three tokens in two launches, and the
+    split down launch from 4097 columns, against an fp64 reference of the same
+    codes: relative error of f32 sums over bf16 hi and lo planes (2^-17 an
+    element, so 2^-16 of the result's norm) and, for bf16 outputs, one rounding
+    (2^-9 an element)."""
+    g = torch.Generator(device="cuda:0").manual_seed(M * I)
+    x = torch.randn((M, H), generator=g, device="cuda:0").to(torch.bfloat16 if xt == "bf16" else torch.float32)
+    mat = lambda n, k: (torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 16), generator=g, device="cuda:0",  # noqa: E731
+                                      dtype=torch.int32), 0.01 + 0.01 * torch.rand(n, generator=g, device="cuda:0"))
+    wg, wu, wd = mat(I, H), mat(I, H), mat(H, I)
+
+    def lin(v, w):
+        sh = torch.arange(0, 32, 2, device="cuda:0", dtype=torch.int32)
+        c = ((w[0][:, :, None] >> sh) & 3).view(w[0].shape[0], -1)
+        return (v @ ((c == 2).double() - (c == 0).double()).t()) * w[1].double()
+
+    gv = lin(x.double(), wg)
+    ref = lin(gv / (1 + torch.exp(-gv)) * lin(x.double(), wu), wd)
+    for yt, tol in ((torch.float32, 2.0 ** -16), (torch.bfloat16, 2.0 ** -8)):
+        y = torch.full((M, H), float("nan"), dtype=yt, device="cuda:0")
+        ctx.ternary_ffn(x, *wg, *wu, *wd, y)
+        torch.cuda.synchronize()
+        assert (torch.linalg.norm(y.double() - ref) / torch.linalg.norm(ref)).item() < tol
