@@ -256,25 +256,75 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float *__restric
 
 constexpr int GEMM_SK_BM = 64;
 
-// The split: 64-token tiles; when they leave at least half of the compute
-// units idle, S K parts (whole 64-column steps) bring the grid to about two
-// workgroups per CU. (With more tiles the fp32 parts cost more than the
-// idle units: 11008 x 4096 at 256 tokens, 172 tiles, 40.2 us whole against
-// 46.9 us in three parts; 4096 x 11008 at 512 tokens, 128 tiles, 91.8 us
-// whole against 54.5 us in four.)
+// Time of a launch of `tiles` dense tiles of bm tokens x 256 rows over `steps`
+// 64-column steps, in us, from the number of tiles a compute unit runs: alone,
+// two at a time (at most two fit), and whole rounds of two with a rest that
+// starts as they finish; a tile's fill and epilogue count as steps, fewer where
+// a second tile hides them. Measured over 11008 x 4096 (43 tiles a token
+// block), tokens and us for tiles of 64 / 96 / 128:
+//   256: 40.3 / 50.1 / 61.5    333: 54.4 / 50.3 / 61.9    517: 58.2 / 73.1 / 63.3
+//   680: 65.8 / 75.9 / 92.8    900: 92.2 / 82.0 / 95.3   1300: 123 / 122 / 109
+// and over 5632 x 2048 alone 23.3 / 29.1 / 35.8, 1300 tokens 35.8 / 43.9 / 39.4.
+static float gemm_tile_cost(int bm, long tiles, int steps, int cus) {
+  const float busy = fminf((float)tiles / (float)cus, 1.f);
+  const float one = (bm == 64   ? 36.5f + 3.5f * busy  // a tile alone
+                     : bm == 96 ? 46.f + 5.5f * busy
+                                : 57.f + 7.f * busy) / 74.f * (float)(steps + 10);
+  const float fill2 = (float)steps + 6.5f;
+  const float more = (bm == 64 ? 54.f : bm == 96 ? 73.f : 93.f) / 70.5f * fill2;   // the first units with two
+  const float two = (bm == 64 ? 67.f : bm == 96 ? 86.f : 112.f) / 70.5f * fill2;  // two on every unit
+  const long q = tiles / (2L * cus), r = tiles % (2L * cus);
+  float t = (float)q * two;
+  if (r > cus) t += (q ? 0.93f : 1.f) * (more + (two - more) * (float)(r - cus) / (float)cus);
+  else if (r > 0) t += (q ? 0.7f : 1.f) * one;
+  return t;
+}
+
+// Tokens of a tile with the least time: 64, 96 or 128.
+// halves = 2: the fp32 planes kernel, whose 128-token tiles run 8% longer
+// (5632 x 2048, 1300 tokens 71 us against 66 in tiles of 64).
+static int gemm_tile_tokens(int M, int N, int steps, int cus, int halves) {
+  int best = 64;
+  float t = 0.f;
+  for (int bm = 64; bm <= 128; bm += 32) {
+    const float c = gemm_tile_cost(bm, (long)((M + bm - 1) / bm) * ((N + 255) / 256), steps, cus) *
+                    (halves == 2 && bm == 128 ? 1.08f : 1.f);
+    if (bm == 64 || c < t) {
+      best = bm;
+      t = c;
+    }
+  }
+  return best;
+}
+
+// K in S parts where that is the faster way to fill the compute units: the
+// parts' tiles by gemm_tile_cost and the partial sums' way to memory and back
+// (measured at 4.5 TB/s) and the reduction launch, against the whole-K tiles.
+// 4096 x 11008, 517 tokens: 96 us in 144 whole-K tiles, 70 in parts.
 bool gemm_splitk_plan(int M, int K, int N, int cus, int *S, int *kp, int halves) {
   if (M <= 16 || K % 64 != 0 || N % 4 != 0) return false;
   const long tiles = (long)((M + GEMM_SK_BM - 1) / GEMM_SK_BM) * ((N + 255) / 256);
-  if (2 * tiles > cus) return false;
-  const int nks = K / 64;
+  if (tiles > 2L * cus) return false;
+  const int nks = K / 64, bm = gemm_tile_tokens(M, N, halves * nks, cus, halves);
+  // per 64 steps, so that short and long parts compare by their fill alone
+  float best = gemm_tile_cost(bm, (long)((M + bm - 1) / bm) * ((N + 255) / 256), 64, cus) *
+               (float)(halves * nks + 4) / 64.f;
+  bool split = false;
   // at least 8 steps of 64 columns per part: shorter parts are mostly the
   // pipeline's fill and drain, and their fp32 partials outweigh the weights
-  int s = (int)std::min<long>((2L * cus + tiles * halves - 1) / (tiles * halves), nks / 8);
-  if (s < 1 || halves * s < 2) return false;
-  const int steps = (nks + s - 1) / s;
-  *kp = steps * 64;
-  *S = halves * ((K + *kp - 1) / *kp);
-  return true;
+  for (int s = 1; s <= nks / 8 && tiles * halves * s <= 2L * cus + tiles * halves; s++) {
+    if (halves * s < 2) continue;
+    const int steps = (nks + s - 1) / s, parts = halves * ((nks + steps - 1) / steps);
+    const float t = gemm_tile_cost(GEMM_SK_BM, tiles * parts, 64, cus) * (float)(steps + 4) / 64.f + 3.f +
+                    (float)parts * (float)M * (float)N * 8.f / 4.5e6f;
+    if (t < best) {
+      best = t;
+      split = true;
+      *kp = steps * 64;
+      *S = parts;
+    }
+  }
+  return split;
 }
 
 
@@ -600,8 +650,7 @@ static int device_cus() {
 hipError_t launch_gemm_planes(const uint32_t *w, const float *scale, const uint16_t *x2, void *y, int yt_bf16, int M,
                               int K, int N, hipStream_t stream, const float *bias) {
   constexpr int BN = 256, WM = GEMM2_WM, WN = GEMM2_WN, NS = GEMM2_NS;
-  const long tiles128 = (long)((M + 127) / 128) * ((N + BN - 1) / BN);
-  const bool small = tiles128 <= device_cus();
+  const int bm = gemm_tile_tokens(M, N, K / 32, device_cus(), 2);
 #define FRX_PLANES(BM, YT)                                                                                    \
   {                                                                                                           \
     using Core = Gemm2<BM, BN, WM, WN, NS, false>;                                                            \
@@ -614,9 +663,13 @@ hipError_t launch_gemm_planes(const uint32_t *w, const float *scale, const uint1
                        dim3(WM * WN * 64), lds, stream, w, scale, x2, reinterpret_cast<YT *>(y), M, K, N, bias);   \
     return hipGetLastError();                                                                                 \
   }
-  if (small) {
+  if (bm == 64) {
     if (yt_bf16) FRX_PLANES(64, uint16_t)
     FRX_PLANES(64, float)
+  }
+  if (bm == 96) {
+    if (yt_bf16) FRX_PLANES(96, uint16_t)
+    FRX_PLANES(96, float)
   }
   if (yt_bf16) FRX_PLANES(128, uint16_t)
   FRX_PLANES(128, float)
@@ -639,18 +692,16 @@ static hipError_t launch_gemm2_bm(const uint32_t *w, const float *scale, const v
   return hipGetLastError();
 }
 
-// Dense tiles: 128 tokens x 256 rows, or 64 x 256 when the 128-token grid
-// would give each CU at most one workgroup: the 64-token tile (48 KB of LDS,
-// 64 accumulation registers per lane) runs two workgroups per CU, so each
-// SIMD interleaves two waves (2048 x 4096 x 4096: 64 us against 70 us; at
-// N = 11008 the 128-token tile stays ahead, 175 against 198 us). A 128 x 128
-// tile there (half the decode per MFMA, twice the activation reads from LDS)
-// measured 66.1 against 63.8 us.
+// Dense tiles: 64, 96 or 128 tokens x 256 rows, two workgroups per CU, by how
+// the grid falls on the compute units (gemm_tile_tokens). A 128 x 128 tile at
+// 2048 x 4096 x 4096 (half the decode per MFMA, twice the activation reads from
+// LDS) measured 66.1 against 63.8 us in 64 x 256 tiles.
 template <typename YT>
 static hipError_t launch_gemm2_t(const uint32_t *w, const float *scale, const void *x, void *y,
                                  int M, int K, int N, hipStream_t stream, const float *bias) {
-  const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
-  if (tiles128 <= device_cus()) return launch_gemm2_bm<64, YT>(w, scale, x, y, M, K, N, stream, bias);
+  const int bm = gemm_tile_tokens(M, N, K / 64, device_cus(), 1);
+  if (bm == 64) return launch_gemm2_bm<64, YT>(w, scale, x, y, M, K, N, stream, bias);
+  if (bm == 96) return launch_gemm2_bm<96, YT>(w, scale, x, y, M, K, N, stream, bias);
   return launch_gemm2_bm<128, YT>(w, scale, x, y, M, K, N, stream, bias);
 }
 

@@ -705,3 +705,32 @@ def test_f32_prefill_planes_random_parity(ctx, M, K, N):
     assert_close_f32(host(_run(ctx, w, s, xf, xb, "f32", "f32")), ref)
     yb = _run(ctx, w, s, xf, xb, "f32", "bf16")
     assert_bf16_within_1ulp(yb.view(torch.int16).cpu().numpy().view(np.uint16), ref)
+
+
+@pytest.mark.parametrize("M,K,N,xt", [(333, 1024, 11008, "bf16"), (680, 512, 11008, "bf16"), (900, 576, 11004, "f32"),
+                                      (1300, 1024, 13824, "bf16"), (517, 4096, 4096, "bf16"), (97, 4096, 2052, "f32"),
+                                      (517, 1088, 13824, "f32"), (1201, 4160, 4096, "f32")])
+def test_gemm_tile_heights_and_splits(ctx, M, K, N, xt):
+    """Tiles of 64, 96 and 128 tokens and the K splits that the launch plans
+    choose between (last tiles of a few tokens, N and K past whole tiles),
+    against fp64 of the same codes: f32 sums of bf16 hi and lo planes are within
+    2^-16 of the result's norm, and dyadic activations give the exact product."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + K)
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 16), generator=g, device="cuda:0", dtype=torch.int32)
+    s = 2.0 ** torch.randint(-4, 1, (N,), generator=g, device="cuda:0").float()
+    sh = torch.arange(0, 32, 2, device="cuda:0", dtype=torch.int32)
+    c = ((w[:, :, None] >> sh) & 3).view(N, K)
+    dense = ((c == 2).double() - (c == 0).double()) * s.double()[:, None]
+    dt = torch.bfloat16 if xt == "bf16" else torch.float32
+    for dyadic in (True, False):
+        x = torch.randint(-8, 9, (M, K), generator=g, device="cuda:0").float() / 4 if dyadic else torch.randn(
+            (M, K), generator=g, device="cuda:0")
+        x = x.to(dt)
+        y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda:0")
+        ctx.ternary_linear(w, s, x, y)
+        torch.cuda.synchronize()
+        ref = x.double() @ dense.t()
+        if dyadic:
+            assert torch.equal(y.double(), ref)
+        else:
+            assert (torch.linalg.norm(y.double() - ref) / torch.linalg.norm(ref)).item() < 2.0 ** -16
