@@ -1093,8 +1093,30 @@ static frx_status ffn_run(frx_ctx *ctx, const void *x, frx_dtype xt, const uint3
     if (e != hipSuccess) return hip_fail(ctx, e, "ffn gate/up launch");
     return ffn_down_planes(ctx, w_down, s_down, hp, y, yt, M, H, I, may_alloc);
   }
+  frx_status st;
+  int bm = 0;
+  const int halves = xt == FRX_F32 ? 2 : 1;
+  if (M > 16 && (halves == 1 || may_alloc) && aligned16(w_gate) && aligned16(w_up) && aligned16(w_down) &&
+      (size_t)M * H * 4 < ((size_t)1 << 31) && frx::gemm_glu_plan((int)M, (int)H, (int)I, ctx->cus, halves, &bm)) {
+    // h as bf16 hi | lo rows straight from the gate/up launch
+    const uint16_t *xin = reinterpret_cast<const uint16_t *>(x);
+    if (halves == 2) {
+      if ((st = ensure_buffer(ctx, &ctx->xpl_ws, &ctx->xpl_ws_bytes, a256((size_t)M * H * 4),
+                              "activation planes workspace allocation")) != FRX_OK)
+        return st;
+      uint16_t *x2 = reinterpret_cast<uint16_t *>(ctx->xpl_ws);
+      if ((e = frx::launch_to_planes(reinterpret_cast<const float *>(x), x2, (int)M, (int)H, ctx->stream)) != hipSuccess)
+        return hip_fail(ctx, e, "activation planes launch");
+      xin = x2;
+    }
+    uint16_t *h2 = reinterpret_cast<uint16_t *>(ws);
+    e = frx::launch_gemm_glu(w_gate, s_gate, w_up, s_up, xin, h2, (int)M, (int)H, (int)I, halves,
+                             act == FRX_ACT_GELU_TANH, bm, ctx->stream);
+    if (e != hipSuccess) return hip_fail(ctx, e, "ffn gate/up launch");
+    return gemm_planes_auto(ctx, w_down, s_down, nullptr, h2, y, yt, M, I, H, may_alloc);
+  }
   float *h = reinterpret_cast<float *>(ws);
-  frx_status st = glu_into(ctx, x, xt, w_gate, s_gate, w_up, s_up, M, H, I, act == FRX_ACT_GELU_TANH, h, u_ws);
+  st = glu_into(ctx, x, xt, w_gate, s_gate, w_up, s_up, M, H, I, act == FRX_ACT_GELU_TANH, h, u_ws);
   if (st != FRX_OK) return st;
   if (M > 16 && I % 64 == 0 && aligned16(w_down)) {
     // h as bf16 hi | lo rows in the up projection's buffer (no longer

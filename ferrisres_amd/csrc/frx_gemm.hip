@@ -254,6 +254,15 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float *__restric
   YStore<YT>::store4(Y + i, o, 4);
 }
 
+// Pipeline stages of the K loop.
+constexpr int GEMM2_NS = 4;
+// One wave per SIMD, each over the tile's tokens x 64 rows. Waves split
+// 2 x 2 over tokens and rows instead (half the activation reads from LDS,
+// twice each wave's weight decode) measured slower at 2048 x 4096 x 4096 /
+// 11008: dense 76 / 184 us against 65 / 175 us, 2:4 87 / 195 us against
+// 71 / 157 us.
+constexpr int GEMM2_WM = 1, GEMM2_WN = 4;
+
 constexpr int GEMM_SK_BM = 64;
 
 // Time of a launch of `tiles` dense tiles of bm tokens x 256 rows over `steps`
@@ -301,15 +310,15 @@ static int gemm_tile_tokens(int M, int N, int steps, int cus, int halves) {
 // parts' tiles by gemm_tile_cost and the partial sums' way to memory and back
 // (measured at 4.5 TB/s) and the reduction launch, against the whole-K tiles.
 // 4096 x 11008, 517 tokens: 96 us in 144 whole-K tiles, 70 in parts.
-bool gemm_splitk_plan(int M, int K, int N, int cus, int *S, int *kp, int halves) {
-  if (M <= 16 || K % 64 != 0 || N % 4 != 0) return false;
-  const long tiles = (long)((M + GEMM_SK_BM - 1) / GEMM_SK_BM) * ((N + 255) / 256);
-  if (tiles > 2L * cus) return false;
+// Returns the time of the faster of the two; *S = 0: whole-K tiles.
+static float gemm_plan(int M, int K, int N, int cus, int halves, int *S, int *kp) {
   const int nks = K / 64, bm = gemm_tile_tokens(M, N, halves * nks, cus, halves);
   // per 64 steps, so that short and long parts compare by their fill alone
   float best = gemm_tile_cost(bm, (long)((M + bm - 1) / bm) * ((N + 255) / 256), 64, cus) *
                (float)(halves * nks + 4) / 64.f;
-  bool split = false;
+  *S = 0;
+  const long tiles = (long)((M + GEMM_SK_BM - 1) / GEMM_SK_BM) * ((N + 255) / 256);
+  if (tiles > 2L * cus) return best;
   // at least 8 steps of 64 columns per part: shorter parts are mostly the
   // pipeline's fill and drain, and their fp32 partials outweigh the weights
   for (int s = 1; s <= nks / 8 && tiles * halves * s <= 2L * cus + tiles * halves; s++) {
@@ -319,14 +328,118 @@ bool gemm_splitk_plan(int M, int K, int N, int cus, int *S, int *kp, int halves)
                     (float)parts * (float)M * (float)N * 8.f / 4.5e6f;
     if (t < best) {
       best = t;
-      split = true;
       *kp = steps * 64;
       *S = parts;
     }
   }
-  return split;
+  return best;
 }
 
+bool gemm_splitk_plan(int M, int K, int N, int cus, int *S, int *kp, int halves) {
+  if (M <= 16 || K % 64 != 0 || N % 4 != 0) return false;
+  (void)gemm_plan(M, K, N, cus, halves, S, kp);
+  return *S > 0;
+}
+
+// ---- gate, up and the activation product in one launch (more than 16 tokens) ---
+// Tiles of BM tokens x (128 gate rows and the same 128 up rows): waves 0-1
+// multiply gate, 2-3 up, and the epilogue writes h = act(g) * u as bf16 hi | lo
+// halves of the [M][2I] rows that the down projection reads. Against two GEMMs
+// with fp32 outputs, their product and its split into planes this takes 20
+// bytes per element of h out of memory traffic and three launches, and one grid
+// of twice the tiles fills the chip better (FFN of 333 tokens, 4096 / 11008: 190.3
+// -> 158.2 us; 256 tokens, 2048 / 5632: 82.9 -> 51.7).
+template <int BM>
+__global__ __launch_bounds__(256) void gemm2_glu_kernel(const uint32_t *__restrict__ Wg, const float *__restrict__ sg,
+                                                        const uint32_t *__restrict__ Wu, const float *__restrict__ su,
+                                                        const uint16_t *__restrict__ X, uint16_t *__restrict__ h2,
+                                                        int M, int H, int I, int ldx, int gelu) {
+  constexpr int BN = 256, HN = BN / 2;
+  using Core = Gemm2<BM, BN, GEMM2_WM, GEMM2_WN, GEMM2_NS, false>;
+  extern __shared__ __align__(16) uint32_t lds[];
+  int nt, mt;
+  xcd_tile(nt, mt);
+  const int n0 = nt * HN, m0 = mt * BM;
+  const int m_count = min(BM, M - m0), nc = min(HN, I - n0);
+  f32x4 acc[Core::FN][Core::FM];
+  // ldx = 2 H: x as bf16 hi | lo halves, the weight columns wrap at H
+  Core::run(lds, X + (size_t)m0 * ldx, (uint32_t)m_count * (uint32_t)ldx * 2u, nullptr, m_count,
+            Wg + (size_t)n0 * (H >> 4), nc, ldx, acc, Wu + (size_t)n0 * (H >> 4), H, ldx);
+  // the fragments go to LDS in passes of PB token blocks; a thread then owns 4
+  // gate columns (and the same 4 up columns HN further) of a run of tokens
+  constexpr int PF = BN + 16, PB = BM == 64 ? 2 : 3;
+  static_assert(PB * 16 * PF <= Core::LDS_DWORDS, "epilogue staging");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
+  float *st = reinterpret_cast<float *>(lds);
+  const int c = 4 * (threadIdx.x % (HN / 4)), rr = threadIdx.x / (HN / 4);
+  f32x4 sgv, suv;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int n = n0 + min(c + j, nc - 1);
+    sgv[j] = 0.5f * sg[n];  // 0.5 undoes the 2*dec(c) operand encoding
+    suv[j] = 0.5f * su[n];
+  }
+#pragma unroll
+  for (int f0 = 0; f0 < Core::FM; f0 += PB) {
+#pragma unroll
+    for (int fn = 0; fn < Core::FN; fn++)
+#pragma unroll
+      for (int fi = 0; fi < PB; fi++)
+        if (f0 + fi < Core::FM)
+          *reinterpret_cast<f32x4 *>(st + (fi * 16 + l16) * PF + wave * Core::TN + fn * 16 + 4 * g) = acc[fn][f0 + fi];
+    __syncthreads();
+    const int rows = min(min(PB, Core::FM - f0) * 16, m_count - f0 * 16);
+    if (c < nc)  // I % 16 == 0: all four columns
+      for (int lr = rr; lr < rows; lr += 8) {
+        const f32x4 gv = *reinterpret_cast<const f32x4 *>(st + lr * PF + c) * sgv;
+        const f32x4 uv = *reinterpret_cast<const f32x4 *>(st + lr * PF + HN + c) * suv;
+        u32x2 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          uint32_t a, b;
+          split2_bf16(moe_act(gelu, gv[2 * j], uv[2 * j]), moe_act(gelu, gv[2 * j + 1], uv[2 * j + 1]), a, b);
+          hi[j] = a;
+          lo[j] = b;
+        }
+        uint16_t *d = h2 + (size_t)(m0 + f0 * 16 + lr) * (2 * (size_t)I) + n0 + c;
+        *reinterpret_cast<u32x2 *>(d) = hi;
+        *reinterpret_cast<u32x2 *>(d + I) = lo;
+      }
+    __syncthreads();
+  }
+}
+
+// The tile height, and whether the launch is the faster way: with few tiles
+// (short rows of tokens and a narrow intermediate) two GEMMs split over K fill
+// more of the chip.
+bool gemm_glu_plan(int M, int H, int I, int cus, int halves, int *bm) {
+  if (M <= 16 || H % 64 != 0 || I % 64 != 0) return false;
+  const int n2 = 2 * I;  // 128 + 128 rows a tile
+  *bm = gemm_tile_tokens(M, n2, halves * (H / 64), cus, halves);
+  const float fused = gemm_tile_cost(*bm, (long)((M + *bm - 1) / *bm) * ((n2 + 255) / 256), 64, cus) *
+                      (float)(halves * (H / 64) + 4) / 64.f;
+  int S, kp;
+  const float apart = 2.f * gemm_plan(M, H, I, cus, halves, &S, &kp) + 6.f + (float)M * (float)I * 20.f / 4.5e6f;
+  return fused < apart;
+}
+
+hipError_t launch_gemm_glu(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up, const float *s_up,
+                           const uint16_t *x, uint16_t *h2, int M, int H, int I, int halves, int gelu, int bm,
+                           hipStream_t stream) {
+  auto run = [&](auto bmc) {
+    constexpr int BM = decltype(bmc)::value;
+    constexpr int lds = Gemm2<BM, 256, GEMM2_WM, GEMM2_WN, GEMM2_NS, false>::LDS_DWORDS * 4;
+    static std::atomic<uint64_t> done;
+    const hipError_t e = opt_in_lds(reinterpret_cast<const void *>(&gemm2_glu_kernel<BM>), lds, done);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((gemm2_glu_kernel<BM>), dim3((I + 127) / 128, (M + BM - 1) / BM), dim3(256), lds, stream, w_gate,
+                       s_gate, w_up, s_up, x, h2, M, H, I, halves * H, gelu);
+    return hipGetLastError();
+  };
+  if (bm == 64) return run(std::integral_constant<int, 64>());
+  if (bm == 96) return run(std::integral_constant<int, 96>());
+  return run(std::integral_constant<int, 128>());
+}
 
 size_t gemm_splitk_workspace_bytes(int M, int N, int S) { return (size_t)S * M * N * 4; }
 
@@ -619,14 +732,6 @@ hipError_t launch_gemm_splitk(const uint32_t *w, const float *scale, const void 
   return hipGetLastError();
 }
 
-// Pipeline stages of the K loop.
-constexpr int GEMM2_NS = 4;
-// One wave per SIMD, each over the tile's tokens x 64 rows. Waves split
-// 2 x 2 over tokens and rows instead (half the activation reads from LDS,
-// twice each wave's weight decode) measured slower at 2048 x 4096 x 4096 /
-// 11008: dense 76 / 184 us against 65 / 175 us, 2:4 87 / 195 us against
-// 71 / 157 us.
-constexpr int GEMM2_WM = 1, GEMM2_WN = 4;
 // Tokens per tile of the 2:4 launches with at least one 128-token tile per
 // compute unit (64 measured slower there: 83 / 203 us against 71 / 158 us at
 // 2048 x 4096 x 4096 / 11008).

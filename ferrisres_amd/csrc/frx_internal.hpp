@@ -120,6 +120,14 @@ bool gemm_splitk_plan(int M, int K, int N, int cus, int *S, int *kp, int halves 
 size_t gemm_splitk_workspace_bytes(int M, int N, int S);
 hipError_t launch_gemm_splitk(const uint32_t *w, const float *scale, const void *x, void *y, int yt_bf16, int M, int K,
                               int N, int S, int kp, float *part, hipStream_t stream, const float *bias, int halves = 1);
+// Gate, up and the activation product of the FFN above 16 tokens in one launch
+// (H % 64 == 0, I % 64 == 0, 16-byte aligned weights and x): x [M][halves * H]
+// bf16 (halves = 2: hi | lo rows), h2 [M][2I] bf16 hi | lo rows; bm from the
+// plan, which also says whether two split GEMMs would be faster.
+bool gemm_glu_plan(int M, int H, int I, int cus, int halves, int *bm);
+hipError_t launch_gemm_glu(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up, const float *s_up,
+                           const uint16_t *x, uint16_t *h2, int M, int H, int I, int halves, int gelu, int bm,
+                           hipStream_t stream);
 // The split for 2:4 weights (GPU layout), any token count from 1, bf16 x.
 // halves = 2: x2 [M][2K] bf16 hi | lo rows (an fp32 activation), parts over
 // both halves.

@@ -370,3 +370,32 @@ def test_ffn_decode_batch_launches(ctx, M, H, I, xt):
         ctx.ternary_ffn(x, *wg, *wu, *wd, y)
         torch.cuda.synchronize()
         assert (torch.linalg.norm(y.double() - ref) / torch.linalg.norm(ref)).item() < tol
+
+
+@pytest.mark.parametrize("M,H,I,xt,act", [(17, 4096, 11008, "bf16", "silu"), (97, 1024, 4160, "f32", "silu"),
+                                          (333, 512, 11072, "bf16", "gelu"), (129, 2048, 5632, "f32", "gelu"),
+                                          (680, 256, 8256, "bf16", "silu"), (40, 4096, 1024, "bf16", "silu")])
+def test_ffn_prefill_one_gate_up_launch(ctx, M, H, I, xt, act):
+    """Above 16 tokens: gate, up and the product in one launch (each tile height,
+    last tiles of one token or of 64 of the 128 rows, f32 x as hi | lo rows; and a
+    shape that stays with two split GEMMs) against fp64 of the same codes, with
+    the bounds of test_ffn_decode_batch_launches."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + I)
+    x = torch.randn((M, H), generator=g, device="cuda:0").to(torch.bfloat16 if xt == "bf16" else torch.float32)
+    mat = lambda n, k: (torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 16), generator=g, device="cuda:0",  # noqa: E731
+                                      dtype=torch.int32), 0.01 + 0.01 * torch.rand(n, generator=g, device="cuda:0"))
+    wg, wu, wd = mat(I, H), mat(I, H), mat(H, I)
+
+    def lin(v, w):
+        sh = torch.arange(0, 32, 2, device="cuda:0", dtype=torch.int32)
+        c = ((w[0][:, :, None] >> sh) & 3).view(w[0].shape[0], -1)
+        return (v @ ((c == 2).double() - (c == 0).double()).t()) * w[1].double()
+
+    gv = lin(x.double(), wg)
+    gv = torch.nn.functional.gelu(gv, approximate="tanh") if act == "gelu" else torch.nn.functional.silu(gv)
+    ref = lin(gv * lin(x.double(), wu), wd)
+    for yt, tol in ((torch.float32, 2.0 ** -16), (torch.bfloat16, 2.0 ** -8)):
+        y = torch.full((M, H), float("nan"), dtype=yt, device="cuda:0")
+        ctx.ternary_ffn(x, *wg, *wu, *wd, y, act=frx.ACT_GELU_TANH if act == "gelu" else frx.ACT_SILU)
+        torch.cuda.synchronize()
+        assert (torch.linalg.norm(y.double() - ref) / torch.linalg.norm(ref)).item() < tol
