@@ -358,6 +358,23 @@ static frx_status check_linear(frx_ctx *ctx, const void *w, const void *scale,
 
 static frx_status ensure_buffer(frx_ctx *ctx, void **buf, size_t *have, size_t need, const char *what);
 
+// Whether a workspace of `have` bytes serves a call that needs `need`, growing
+// if it must: not while the stream is being captured (no allocation may happen
+// then). Paths that have a sibling without the workspace ask first, so that a
+// first call under capture runs there.
+static bool may_grow(frx_ctx *ctx, size_t have, size_t need) {
+  if (need <= have) return true;
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &c) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return c == hipStreamCaptureStatusNone;
+}
+
+// The same for the split kernels' arrival counters.
+static bool may_count(frx_ctx *ctx) { return ctx->sk_cnt || may_grow(ctx, 0, 1); }
+
 // x, scale and y as the kernels take them: 16-byte aligned. A caller's sub-
 // slice at another offset is copied into the context's staging workspace
 // (x and scale before the launch, y back after it), on the context stream.
@@ -466,7 +483,8 @@ static frx_status gemm_planes_auto(frx_ctx *ctx, const uint32_t *w, const float 
   hipError_t e;
   int S = 0, kp = 0;
   if (may_alloc && ctx->gemv_split != FRX_GEMV_SPLIT_NEVER &&
-      frx::gemm_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &kp, 2)) {
+      frx::gemm_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &kp, 2) &&
+      may_grow(ctx, ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S))) {
     if ((st = ensure_buffer(ctx, &ctx->gk_ws, &ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S),
                             "split-K GEMM workspace allocation")) != FRX_OK)
       return st;
@@ -486,7 +504,8 @@ static frx_status gemv_auto(frx_ctx *ctx, const uint32_t *w, const float *scale,
                             frx_dtype xt, void *y, frx_dtype yt, uint32_t M, uint32_t K, uint32_t N) {
   frx_status st;
   hipError_t e;
-  if (use_split(ctx, w, x, M, K, N, xt)) {
+  if (use_split(ctx, w, x, M, K, N, xt) && may_count(ctx) &&
+      may_grow(ctx, ctx->sk_ws_bytes, frx::gemv_sk_workspace_bytes((int)K, (int)N, ctx->cus))) {
     if ((st = ensure_buffer(ctx, &ctx->sk_ws, &ctx->sk_ws_bytes,
                             frx::gemv_sk_workspace_bytes((int)K, (int)N, ctx->cus),
                             "split-K workspace allocation")) != FRX_OK)
@@ -509,7 +528,8 @@ static frx_status gemv_auto(frx_ctx *ctx, const uint32_t *w, const float *scale,
   } else {
     int S = 0, kp = 0;
     if (ctx->gemv_split != FRX_GEMV_SPLIT_NEVER && xt == FRX_BF16 && aligned16(w) && aligned16(x) &&
-        (size_t)M * K * 2 < ((size_t)1 << 31) && frx::gemm_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &kp)) {
+        (size_t)M * K * 2 < ((size_t)1 << 31) && frx::gemm_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &kp) &&
+        may_grow(ctx, ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S))) {
       // 17 to a few hundred tokens: K split over workgroups so that the
       // grid covers the compute units
       if ((st = ensure_buffer(ctx, &ctx->gk_ws, &ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S),
@@ -611,7 +631,8 @@ static frx_status sp24_rows_auto(frx_ctx *ctx, const uint32_t *w, int prepared, 
   int ncs = 0, S = 0;
   // NEVER keeps the unsplit engine from 5 tokens, where it has one worth keeping
   *done = (ctx->gemv_split != FRX_GEMV_SPLIT_NEVER || M <= 4) &&
-          frx::sp24_rows_plan((int)M, (int)K, (int)N, xt == FRX_BF16, prepared, ctx->cus, &ncs, &S);
+          frx::sp24_rows_plan((int)M, (int)K, (int)N, xt == FRX_BF16, prepared, ctx->cus, &ncs, &S) &&
+          may_count(ctx) && may_grow(ctx, ctx->gk_ws_bytes, frx::sp24_rows_workspace_bytes((int)M, (int)N, S));
   if (!*done) return FRX_OK;
   frx_status st = ensure_buffer(ctx, &ctx->gk_ws, &ctx->gk_ws_bytes, frx::sp24_rows_workspace_bytes((int)M, (int)N, S),
                                 "split-K GEMM workspace allocation");
@@ -861,14 +882,18 @@ frx_status frx_moe_ternary_ffn(
   if ((size_t)T * top_k * I > (size_t)0x7FFFFFFF) return fail(ctx, FRX_ERR_SHAPE, "T*top_k*I too large");
   if (ctx->lora_on && ctx->lora_experts != E)
     return fail(ctx, FRX_ERR_SHAPE, "LoRA adapters were set for %u experts, the call has %u", ctx->lora_experts, E);
-  const size_t need = frx::moe_workspace_bytes((int)T, (int)H, (int)I, (int)E, (int)top_k);
+  // the decode batch's K parts only where the workspace may grow for them
+  const bool parts = (size_t)T * top_k <= (size_t)frx::MOE_ROWS_MAXA && may_count(ctx) &&
+                     may_grow(ctx, ctx->moe_ws_bytes,
+                              frx::moe_workspace_bytes((int)T, (int)H, (int)I, (int)E, (int)top_k, true));
+  const size_t need = frx::moe_workspace_bytes((int)T, (int)H, (int)I, (int)E, (int)top_k, parts);
   if ((st = ensure_buffer(ctx, &ctx->moe_ws, &ctx->moe_ws_bytes, need, "MoE workspace allocation")) != FRX_OK)
     return st;
   frx::MoeWorkspace ws;
-  frx::moe_workspace_carve(ctx->moe_ws, (int)T, (int)H, (int)I, (int)E, (int)top_k, &ws);
+  frx::moe_workspace_carve(ctx->moe_ws, (int)T, (int)H, (int)I, (int)E, (int)top_k, parts, &ws);
   // a few routed rows (the decode paths): the down launch also combines,
   // through the context's arrival counters
-  if ((size_t)T * top_k <= (size_t)frx::MOE_ROWS_MAXA) {
+  if ((size_t)T * top_k <= (size_t)frx::MOE_ROWS_MAXA && may_count(ctx)) {
     if ((st = ensure_sk_counters(ctx)) != FRX_OK) return st;
     ws.cnt = ctx->sk_cnt;
   }
@@ -982,7 +1007,9 @@ static frx_status ffn_down_planes(frx_ctx *ctx, const uint32_t *w_down, const fl
                                   void *y, frx_dtype yt, uint32_t M, uint32_t H, uint32_t I, bool may_alloc) {
   const bool split = may_alloc && ctx->gemv_split != FRX_GEMV_SPLIT_NEVER &&
                      (ctx->gemv_split == FRX_GEMV_SPLIT_ALWAYS || I > 4096) &&
-                     (H + 127) / 128 <= (uint32_t)frx::GEMV_SK_MAX_TILES && (size_t)M * I * 4 < ((size_t)1 << 32);
+                     (H + 127) / 128 <= (uint32_t)frx::GEMV_SK_MAX_TILES && (size_t)M * I * 4 < ((size_t)1 << 32) &&
+                     may_count(ctx) &&
+                     may_grow(ctx, ctx->sk_ws_bytes, frx::gemv_sk_workspace_bytes((int)I, (int)H, ctx->cus));
   hipError_t e;
   if (split) {
     frx_status st = ensure_buffer(ctx, &ctx->sk_ws, &ctx->sk_ws_bytes,

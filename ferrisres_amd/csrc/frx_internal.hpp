@@ -318,8 +318,9 @@ struct MoeLora {
   int rank = 0;
   float scaling = 0.f;
 };
-size_t moe_workspace_bytes(int T, int H, int I, int E, int top_k);
-void moe_workspace_carve(void *base, int T, int H, int I, int E, int top_k,
+// parts: room for a decode batch's K parts (dpart; null without).
+size_t moe_workspace_bytes(int T, int H, int I, int E, int top_k, bool parts);
+void moe_workspace_carve(void *base, int T, int H, int I, int E, int top_k, bool parts,
                          MoeWorkspace *ws);
 hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
                       int rt_bf16, const uint32_t *const *w_gate,

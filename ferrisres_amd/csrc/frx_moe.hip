@@ -40,7 +40,7 @@ static inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 static size_t mr_dpart_bytes(int A, int H, int I);
 
-size_t moe_workspace_bytes(int T, int H, int I, int E, int top_k) {
+size_t moe_workspace_bytes(int T, int H, int I, int E, int top_k, bool parts) {
   const size_t A = (size_t)T * top_k;
   const size_t max_tiles = (A + MOE_BM - 1) / MOE_BM + E;
   size_t b = 0;
@@ -54,11 +54,11 @@ size_t moe_workspace_bytes(int T, int H, int I, int E, int top_k) {
   b += align256(A * I * 2) * 2;         // h planes
   b += align256(A * H * 4) * 2;         // dout, dout_lo
   b += align256((size_t)T * H * 4);     // f32 x as bf16 hi | lo rows
-  b += align256(mr_dpart_bytes((int)A, H, I));  // decode batch: the down projection's K parts
+  if (parts) b += align256(mr_dpart_bytes((int)A, H, I));  // decode batch: the down projection's K parts
   return b;
 }
 
-void moe_workspace_carve(void *base, int T, int H, int I, int E, int top_k,
+void moe_workspace_carve(void *base, int T, int H, int I, int E, int top_k, bool parts,
                          MoeWorkspace *ws) {
   const size_t A = (size_t)T * top_k;
   const size_t max_tiles = (A + MOE_BM - 1) / MOE_BM + E;
@@ -80,7 +80,7 @@ void moe_workspace_carve(void *base, int T, int H, int I, int E, int top_k,
   ws->dout = reinterpret_cast<float *>(take(A * H * 4));
   ws->dout_lo = reinterpret_cast<float *>(take(A * H * 4));
   ws->x2 = reinterpret_cast<uint16_t *>(take((size_t)T * H * 4));
-  const size_t db = mr_dpart_bytes((int)A, H, I);
+  const size_t db = parts ? mr_dpart_bytes((int)A, H, I) : 0;
   ws->dpart = db ? reinterpret_cast<float *>(take(db)) : nullptr;
 }
 
@@ -2044,7 +2044,7 @@ hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
   const int mS = mr_down_parts(I, &mks);
   const int cols = xt_bf16 ? std::min(T, MR_COLS) : MR_COLS / 2 + std::min(T, MR_COLS / 2);
   const size_t gu_lds_rows = (size_t)cols * mr_stride(H) * 2;
-  if (engine2 && ws.dpart && !lora.tbl && moe_rows_fits(A, T, H, E) && mS <= MR_DN_MAXS &&
+  if (engine2 && ws.dpart && ws.cnt && !lora.tbl && moe_rows_fits(A, T, H, E) && mS <= MR_DN_MAXS &&
       gu_lds_rows <= 144 * 1024 && (size_t)mS * A * H * 4 < ((size_t)1 << 31) &&
       (size_t)H * I / 4 < ((size_t)1 << 31) && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
     // four-wave workgroups while four of them fit a compute unit's LDS, else

@@ -122,3 +122,57 @@ def test_noalloc_rejects_shapes_beyond_the_scratch(ctxs):
     with pytest.raises(frx.FrxError) as ei:
         na.ternary_ffn_noalloc(x, w, s, w, s, wd, sd, y)
     assert ei.value.kind == "Unsupported" and "scratch" in str(ei.value)
+
+
+@pytest.mark.parametrize("what", ["linear", "linear_f32", "sparse24", "moe"])
+def test_first_call_under_capture_keeps_its_route(what):
+    """Calls that now prefer a kernel with a workspace, as a context's first call
+    of that size under graph capture, where nothing can be allocated: they run on
+    the kernels that need none, and replay to the eager result of another
+    context within the f32 tolerance."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV)  # noqa: E731
+    words = lambda n, k: torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k), generator=g, device=DEV, dtype=torch.int32)  # noqa: E731
+    scale = lambda n: 0.02 + 0.01 * torch.rand(n, generator=g, device=DEV)  # noqa: E731
+    fresh, other = frx.Context(0), frx.Context(0)
+    if what == "moe":
+        H, I, E = 256, 512, 4
+        ws = [[words(n, k // 16) if p == 0 else scale(n) for _ in range(E)]
+              for n, k in ((I, H), (I, H), (H, I)) for p in (0, 1)]
+        router, big, x = rnd(E, H), rnd(300, H), rnd(8, H)
+        call = lambda c, xx, y: c.moe_ternary_ffn(xx, router, *ws, y, top_k=2)  # noqa: E731
+        call(fresh, big, torch.empty_like(big))  # a workspace from a larger prompt
+        out = torch.empty_like(x)
+    elif what == "sparse24":
+        K, N = 2064, 300
+        meta, s, x = words(N, (K // 4 + 5) // 6) & 0x3FFFFFFF, scale(N), rnd(8, K)
+        call = lambda c, xx, y: c.sparse24_ternary_linear(meta, s, xx, y)  # noqa: E731
+        out = torch.empty((8, N), device=DEV)
+    else:
+        M, K, N = 517, 4096, 4096
+        w, s, x = words(N, K // 16), scale(N), rnd(M, K)
+        if what == "linear":
+            x = x.to(torch.bfloat16)
+        else:
+            other_x = rnd(2048, K)
+            fresh.ternary_linear(w, s, other_x, torch.empty((2048, N), device=DEV))  # the planes workspace
+        call = lambda c, xx, y: c.ternary_linear(w, s, xx, y)  # noqa: E731
+        out = torch.empty((M, N), device=DEV)
+    ref = torch.empty_like(out)
+    call(other, x, ref)
+    torch.cuda.synchronize()
+    st = torch.cuda.Stream()
+    fresh.set_stream(st)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        call(fresh, x, out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert (torch.linalg.norm(out - ref) / torch.linalg.norm(ref)).item() < 2e-5
+    fresh.set_stream(None)
+    fresh.close()
+    other.close()
