@@ -647,10 +647,12 @@ static frx_status sp24_rows_auto(frx_ctx *ctx, const uint32_t *w, int prepared, 
 }
 
 // Token count from which a 2:4 linear decodes its metadata once into the
-// prepared form (one pass over the matrix, 10.6 us at 11008 x 4096) before
-// the GEMM: at 512 tokens and more the cheaper operand decode repays it
-// (4096 x 11008 at 2048 tokens: 160 -> 145 us; at 256 tokens it is even).
-constexpr uint32_t SP24_PREP_MIN_TOKENS = 512;
+// prepared form (one pass over the matrix, 8 us at 11008 x 4096) before the
+// GEMM, where the cheaper operand decode repays it: 512, or 160 in whole-K tiles
+// (11008 x 4096, 256 / 333 tokens 49.0 / 63.2 us from the 5-bit form, 35.2 /
+// 40.7 and the pass from the prepared one; split over K, 4096 x 4096 at 333
+// tokens, 34.1 against 29.9 and 7).
+constexpr uint32_t SP24_PREP_MIN_TOKENS = 512, SP24_PREP_MIN_TOKENS_WHOLE = 160;
 
 frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
                                        const float *scale, const void *x,
@@ -697,7 +699,10 @@ frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
     if (e != hipSuccess) return hip_fail(ctx, e, "sparse24_ternary_linear planes");
     xin = ctx->xpl_ws;
   }
-  if (engine && M >= SP24_PREP_MIN_TOKENS) {
+  // (from 512 tokens the pass was always made; below, only where its workspace
+  // is there or may be made)
+  if (engine && (M >= SP24_PREP_MIN_TOKENS || (M >= SP24_PREP_MIN_TOKENS_WHOLE && !split &&
+                                               may_grow(ctx, ctx->spp_ws_bytes, (size_t)N * K / 4)))) {
     // the metadata decoded once into its prepared form for every token tile
     if ((st = ensure_buffer(ctx, &ctx->spp_ws, &ctx->spp_ws_bytes, (size_t)N * K / 4,
                             "2:4 prepared metadata allocation")) != FRX_OK)

@@ -274,19 +274,43 @@ constexpr int GEMM_SK_BM = 64;
 //   256: 40.3 / 50.1 / 61.5    333: 54.4 / 50.3 / 61.9    517: 58.2 / 73.1 / 63.3
 //   680: 65.8 / 75.9 / 92.8    900: 92.2 / 82.0 / 95.3   1300: 123 / 122 / 109
 // and over 5632 x 2048 alone 23.3 / 29.1 / 35.8, 1300 tokens 35.8 / 43.9 / 39.4.
-static float gemm_tile_cost(int bm, long tiles, int steps, int cus) {
-  const float busy = fminf((float)tiles / (float)cus, 1.f);
-  const float one = (bm == 64   ? 36.5f + 3.5f * busy  // a tile alone
-                     : bm == 96 ? 46.f + 5.5f * busy
-                                : 57.f + 7.f * busy) / 74.f * (float)(steps + 10);
-  const float fill2 = (float)steps + 6.5f;
-  const float more = (bm == 64 ? 54.f : bm == 96 ? 73.f : 93.f) / 70.5f * fill2;   // the first units with two
-  const float two = (bm == 64 ? 67.f : bm == 96 ? 86.f : 112.f) / 70.5f * fill2;  // two on every unit
+struct TileTimes {
+  float one, busy;  // a tile alone on its unit, and what a full chip adds
+  float more, two;  // two on the first units, two on every unit
+};
+static float gemm_fill_time(const TileTimes &v, long tiles, int cus) {
+  const float one = v.one + v.busy * fminf((float)tiles / (float)cus, 1.f);
   const long q = tiles / (2L * cus), r = tiles % (2L * cus);
-  float t = (float)q * two;
-  if (r > cus) t += (q ? 0.93f : 1.f) * (more + (two - more) * (float)(r - cus) / (float)cus);
+  float t = (float)q * v.two;
+  if (r > cus) t += (q ? 0.93f : 1.f) * (v.more + (v.two - v.more) * (float)(r - cus) / (float)cus);
   else if (r > 0) t += (q ? 0.7f : 1.f) * one;
   return t;
+}
+static float gemm_tile_cost(int bm, long tiles, int steps, int cus) {
+  const float f1 = (float)(steps + 10) / 74.f, f2 = ((float)steps + 6.5f) / 70.5f;
+  const TileTimes v = bm == 64   ? TileTimes{36.5f * f1, 3.5f * f1, 54.f * f2, 67.f * f2}
+                      : bm == 96 ? TileTimes{46.f * f1, 5.5f * f1, 73.f * f2, 86.f * f2}
+                                 : TileTimes{57.f * f1, 7.f * f1, 93.f * f2, 112.f * f2};
+  return gemm_fill_time(v, tiles, cus);
+}
+
+// The same for the 2:4 tiles, over 11008 x 4096 in the prepared form (64 / 96 /
+// 128, tokens and us): 333: 46.3 / 40.7 / 45.6   517: 48.4 / 57.3 / 47.8   680:
+// 54.8 / 58.7 / 67.7   1000: 76.9 / 66.0 / 70.3   2048: 150 / 129 / 118. The
+// 5-bit form and fp32 halves keep the order.
+static int sp_tile_tokens(int M, int N, int cus) {
+  const TileTimes v[3] = {{31.5f, 3.5f, 46.f, 57.f}, {37.5f, 3.f, 57.f, 68.f}, {42.f, 5.f, 67.5f, 82.f}};
+  int best = 64;
+  float t = 0.f;
+  for (int i = 0; i < 3; i++) {
+    const int bm = 64 + 32 * i;
+    const float c = gemm_fill_time(v[i], (long)((M + bm - 1) / bm) * ((N + 255) / 256), cus);
+    if (i == 0 || c < t) {
+      best = bm;
+      t = c;
+    }
+  }
+  return best;
 }
 
 // Tokens of a tile with the least time: 64, 96 or 128.
@@ -732,10 +756,6 @@ hipError_t launch_gemm_splitk(const uint32_t *w, const float *scale, const void 
   return hipGetLastError();
 }
 
-// Tokens per tile of the 2:4 launches with at least one 128-token tile per
-// compute unit (64 measured slower there: 83 / 203 us against 71 / 158 us at
-// 2048 x 4096 x 4096 / 11008).
-constexpr int GEMM2SP_BM = 128;
 
 // Compute units of the current device (queried once).
 static int device_cus() {
@@ -826,15 +846,13 @@ static hipError_t launch_gemm2sp_bm(const uint32_t *meta, const float *scale, co
   return hipGetLastError();
 }
 
-// 64-token tiles while even those do not outnumber the compute units (at
-// 11008 x 4096, 512 tokens: 344 tiles of 64 took 72 us, 172 of 128 64 us).
 template <typename YT, bool PREP, int HV = 1>
 static hipError_t launch_gemm2sp_t(const uint32_t *meta, const float *scale, const void *x, void *y,
                                    int M, int K, int N, hipStream_t stream, const float *bias) {
-  const long tiles128 = (long)((M + GEMM2SP_BM - 1) / GEMM2SP_BM) * ((N + 255) / 256);
-  if (2 * tiles128 <= device_cus())
-    return launch_gemm2sp_bm<64, YT, PREP, HV>(meta, scale, x, y, M, K, N, stream, bias);
-  return launch_gemm2sp_bm<GEMM2SP_BM, YT, PREP, HV>(meta, scale, x, y, M, K, N, stream, bias);
+  const int bm = sp_tile_tokens(M, N, device_cus());
+  if (bm == 64) return launch_gemm2sp_bm<64, YT, PREP, HV>(meta, scale, x, y, M, K, N, stream, bias);
+  if (bm == 96) return launch_gemm2sp_bm<96, YT, PREP, HV>(meta, scale, x, y, M, K, N, stream, bias);
+  return launch_gemm2sp_bm<128, YT, PREP, HV>(meta, scale, x, y, M, K, N, stream, bias);
 }
 
 hipError_t launch_gemm_sp_prepared(const uint32_t *prep, const float *scale, const void *x, void *y, int yt_bf16,

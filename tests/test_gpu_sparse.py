@@ -375,3 +375,20 @@ def test_sparse_decode_paths_repeat_and_graph(ctx):
                 np.testing.assert_array_equal(host(cases[i][3]), refs[i])
     finally:
         ctx.set_stream(None)
+
+
+@pytest.mark.parametrize("M,K,N,xt", [(160, 1024, 11008, "bf16"), (333, 512, 11004, "f32"), (680, 512, 11008, "bf16"),
+                                      (1000, 576, 5632, "bf16"), (333, 1088, 8192, "bf16"), (1400, 256, 4096, "f32")])
+def test_sparse_gemm_tile_heights(ctx, M, K, N, xt):
+    """2:4 tiles of 64, 96 and 128 tokens, and metadata prepared per call from 160
+    tokens in whole-K tiles: dyadic activations give the exact product."""
+    t = synth.sparse24_uniform(f"sp/th/{M}x{K}x{N}", "w", N, K)
+    meta = frx.pack_sparse24_gpu(t)
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    x = (torch.randint(-8, 9, (M, K), generator=g, device="cuda:0").float() / 4)
+    s = 2.0 ** torch.randint(-4, 1, (N,), generator=g, device="cuda:0").float()
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda:0")
+    ctx.sparse24_ternary_linear(dev_u32(meta), s, x.to(torch.bfloat16) if xt == "bf16" else x, y)
+    torch.cuda.synchronize()
+    w = torch.from_numpy(np.asarray(t, np.float32).reshape(N, K)).to("cuda:0")
+    assert torch.equal(y.double(), (x.double() @ w.double().t()) * s.double())
