@@ -101,6 +101,22 @@ __device__ __forceinline__ void split2_bf16(float a, float b, uint32_t &hi, uint
   lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){ra, rb}, bf16x2));
 }
 
+// The same into three planes that hold all 24 bits of a value: x = hi + mid +
+// lo exactly (each remainder is a subtraction without rounding) for |x| from
+// 2^-102 up, where lo is a normal number; mid and lo are zero where hi is not
+// finite.
+__device__ __forceinline__ void split3_bf16(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+  const float ha = __uint_as_float(hi << 16), hb = __uint_as_float(hi & 0xFFFF0000u);
+  const float ra = __builtin_isfinite(ha) ? a - ha : 0.0f;
+  const float rb = __builtin_isfinite(hb) ? b - hb : 0.0f;
+  mid = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){ra, rb}, bf16x2));
+  const float sa = ra - __uint_as_float(mid << 16), sb = rb - __uint_as_float(mid & 0xFFFF0000u);
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){sa, sb}, bf16x2));
+}
+
 // Two 16-code words at once: the interleaved pairs of w0 (lo0 = pairs 0..3,
 // hi0 = pairs 4..7) and of w1, pair i = ~(w << (14 - 2i)) & 0xC000C000. The
 // words shift together as one 64-bit value (v_lshlrev_b64, full rate): the

@@ -150,6 +150,7 @@ hipError_t launch_sp24_gemv(const uint32_t *meta, const float *scale, const void
 // on the sparse pipe (frx_sp24.hip): slices of ncs 16-byte loads per lane, S
 // of them; part: sp24_rows_workspace_bytes; counters: the split-K GEMV's.
 constexpr int SP24_ROWS_MAX_BF16 = 32, SP24_ROWS_MAX_F32 = 24;  // most tokens
+constexpr int SP24_EXACT_MAX_F32 = 4;  // most f32 tokens in three bf16 planes (all bits of x)
 bool sp24_rows_plan(int M, int K, int N, int xt_bf16, int prepared, int cus, int *ncs, int *S);
 size_t sp24_rows_workspace_bytes(int M, int N, int S);
 hipError_t launch_sp24_rows(const uint32_t *w, int prepared, const float *scale, const void *x, int xt_bf16, void *y,

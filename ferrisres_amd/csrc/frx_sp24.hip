@@ -25,9 +25,12 @@
 // per two steps for the groups that straddle words. Columns past K are staged
 // as zeros and cancel whatever the words there hold, so any K % 4 == 0 and any
 // N run here (K % 64 != 0 used to take the register-staged engine).
-// The 16 columns of B are 16 bf16 tokens, or 8 f32 tokens' hi planes and the
-// same tokens' lo planes, added across lanes at the end; SETS of them share
-// the decoded operand.
+// The 16 columns of B are 16 bf16 tokens, 8 f32 tokens' hi planes and the same
+// tokens' lo planes, or up to 4 f32 tokens in three planes each, added across
+// lanes at the end; SETS of them share the decoded operand. Three planes hold
+// every bit of an f32 value: the few-token calls, which the columns have room
+// for, keep full fp32 products as a VALU kernel would (1-4 tokens over 4096 x
+// 11008, 8.4-9.2 us with two planes and with three).
 #include <type_traits>
 
 #include "frx_device.hpp"
@@ -72,10 +75,10 @@ __device__ __forceinline__ f32x4 spr_mul(const f32x4 &acc, const u32x4 &a, const
 }
 
 // grid (ceil(N / 128), S): rows of the tile over chunks s ncs .. of the
-// columns; part [S][M][Np].
+// columns; part [S][M][Np]. PL: planes of a token, f32 2 or 3, bf16 1.
 // NC: most chunks of a slice (2 or 4; the smaller one keeps more workgroups on a
 // compute unit).
-template <typename XT, typename YT, int SETS, bool PREP, int NC>
+template <typename XT, typename YT, int SETS, bool PREP, int NC, int PL>
 __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_t *__restrict__ W,
                                                                   const float *__restrict__ scale,
                                                                   const XT *__restrict__ X, float *__restrict__ part,
@@ -83,7 +86,8 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
                                                                   int M, int K, int N, int Np, int wpr, int ncs, int S) {
   constexpr bool F32 = sizeof(XT) == 4;
   constexpr int CH = spr_chunk(PREP), NJ = CH / 64, STRIDE = spr_stride(PREP, NC);
-  constexpr int TPS = F32 ? 8 : 16;  // tokens per set
+  static_assert(F32 ? PL == 2 || PL == 3 : PL == 1, "planes by type");
+  constexpr int TPS = PL == 1 ? 16 : PL == 2 ? 8 : 4;  // tokens per set, plane p at columns p TPS ..
   constexpr int PPT = NC * CH / 8, PCS = TPS * PPT, XR = (PCS + SPR_WAVES * 64 - 1) / (SPR_WAVES * 64), XL = F32 ? 2 : 1;
   extern __shared__ __align__(16) uint16_t xs[];  // [16 SETS][STRIDE]
   const int tid = threadIdx.x, lane = tid & 63;
@@ -110,25 +114,31 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
 #pragma unroll
     for (int r = 0; r < XR; r++) {
       const int pc = min(tid + r * SPR_WAVES * 64, PCS - 1), row = set * 16 + pc / PPT, o = pc % PPT * 8;
-      u32x4 hi, lo;
+      u32x4 v[PL];
       if constexpr (F32) {
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-          uint32_t h, l;
-          split2_bf16(__uint_as_float(xv[set][r][q >> 1][2 * (q & 1)]), __uint_as_float(xv[set][r][q >> 1][2 * (q & 1) + 1]), h,
-                      l);
-          hi[q] = h;
-          lo[q] = l;
+          const float a = __uint_as_float(xv[set][r][q >> 1][2 * (q & 1)]);
+          const float b = __uint_as_float(xv[set][r][q >> 1][2 * (q & 1) + 1]);
+          uint32_t h, m, l;
+          if constexpr (PL == 3) {
+            split3_bf16(a, b, h, m, l);
+            v[1][q] = m;
+          } else {
+            split2_bf16(a, b, h, l);
+          }
+          v[0][q] = h;
+          v[PL - 1][q] = l;
         }
-        *reinterpret_cast<u32x4 *>(xs + (row + 8) * STRIDE + o) = lo;
       } else {
-        hi = xv[set][r][0];
+        v[0] = xv[set][r][0];
         // K % 8 == 4: the second half of the last piece is the next row's
         const uint32_t keep = k0 + o + 4 < K ? 0xFFFFFFFFu : 0u;
-        hi.z &= keep;
-        hi.w &= keep;
+        v[0].z &= keep;
+        v[0].w &= keep;
       }
-      *reinterpret_cast<u32x4 *>(xs + row * STRIDE + o) = hi;
+#pragma unroll
+      for (int p = 0; p < PL; p++) *reinterpret_cast<u32x4 *>(xs + (row + p * TPS) * STRIDE + o) = v[p];
     }
   };
   // activations first (vector loads complete in issue order), then the wave's
@@ -178,11 +188,18 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
 #pragma unroll
   for (int t = 0; t < SETS; t++) {
     f32x4 v = acc[t][0] + acc[t][1];
-    if constexpr (F32) {
+    if constexpr (PL == 2) {
 #pragma unroll
       for (int q = 0; q < 4; q++)  // the other plane, 8 columns away (row_ror:8)
         v[q] += __uint_as_float(
             (uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v[q]), 0x128, 0xF, 0xF, true));
+    } else if constexpr (PL == 3) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {  // mid 4 columns on (row_ror:12), lo 8 (row_ror:8), the small ones first
+        const int u = (int)__float_as_uint(v[q]);
+        v[q] += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, u, 0x12C, 0xF, 0xF, true)) +
+                __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, u, 0x128, 0xF, 0xF, true));
+      }
     }
     const int tok = t * TPS + i, r0 = blockIdx.x * SPR_ROWS + wave * 16 + 4 * g;
     const uint32_t off = i < TPS && tok < M && r0 < Np
@@ -253,30 +270,31 @@ bool sp24_rows_plan(int M, int K, int N, int xt_bf16, int prepared, int cus, int
 
 size_t sp24_rows_workspace_bytes(int M, int N, int S) { return (size_t)S * M * ((size_t)(N + 3) / 4 * 4) * 4; }
 
-template <typename XT, typename YT, int SETS, bool PREP, int NC>
+template <typename XT, typename YT, int SETS, bool PREP, int NC, int PL>
 static hipError_t launch_sp24_rows_nc(const uint32_t *w, const float *scale, const void *x, void *y, int M, int K,
                                       int N, int ncs, int S, float *part, unsigned *counters, hipStream_t stream) {
   const size_t lds = (size_t)16 * SETS * spr_stride(PREP, NC) * 2;
   static std::atomic<uint64_t> done;
   const hipError_t e =
-      opt_in_lds(reinterpret_cast<const void *>(&sp24_rows_kernel<XT, YT, SETS, PREP, NC>), (int)lds, done);
+      opt_in_lds(reinterpret_cast<const void *>(&sp24_rows_kernel<XT, YT, SETS, PREP, NC, PL>), (int)lds, done);
   if (e != hipSuccess) return e;
   const int wpr = PREP ? K / 16 : (K / 4 + 5) / 6;
-  hipLaunchKernelGGL((sp24_rows_kernel<XT, YT, SETS, PREP, NC>), dim3((N + SPR_ROWS - 1) / SPR_ROWS, S),
+  hipLaunchKernelGGL((sp24_rows_kernel<XT, YT, SETS, PREP, NC, PL>), dim3((N + SPR_ROWS - 1) / SPR_ROWS, S),
                      dim3(SPR_WAVES * 64), lds, stream, w, scale, reinterpret_cast<const XT *>(x), part, counters,
                      reinterpret_cast<YT *>(y), M, K, N, (N + 3) / 4 * 4, wpr, ncs, S);
   return hipGetLastError();
 }
 
-template <typename XT, int SETS, bool PREP>
+template <typename XT, int SETS, bool PREP, int PL = sizeof(XT) == 4 ? 2 : 1>
 static hipError_t launch_sp24_rows_t(const uint32_t *w, const float *scale, const void *x, void *y, int yt_bf16, int M,
                                      int K, int N, int ncs, int S, float *part, unsigned *counters,
                                      hipStream_t stream) {
   auto run = [&](auto yp) {
     using YT = std::remove_pointer_t<decltype(yp)>;
-    return ncs <= 2 ? launch_sp24_rows_nc<XT, YT, SETS, PREP, 2>(w, scale, x, y, M, K, N, ncs, S, part, counters, stream)
-                    : launch_sp24_rows_nc<XT, YT, SETS, PREP, SPR_NC>(w, scale, x, y, M, K, N, ncs, S, part, counters,
-                                                                      stream);
+    return ncs <= 2 ? launch_sp24_rows_nc<XT, YT, SETS, PREP, 2, PL>(w, scale, x, y, M, K, N, ncs, S, part, counters,
+                                                                     stream)
+                    : launch_sp24_rows_nc<XT, YT, SETS, PREP, SPR_NC, PL>(w, scale, x, y, M, K, N, ncs, S, part,
+                                                                          counters, stream);
   };
   return yt_bf16 ? run((uint16_t *)nullptr) : run((float *)nullptr);
 }
@@ -288,6 +306,7 @@ hipError_t launch_sp24_rows(const uint32_t *w, int prepared, const float *scale,
   auto run = [&](auto f) { return f(w, scale, x, y, yt_bf16, M, K, N, ncs, S, part, counters, stream); };
   if (prepared) return sets == 1 ? run(launch_sp24_rows_t<uint16_t, 1, true>) : run(launch_sp24_rows_t<uint16_t, 2, true>);
   if (xt_bf16) return sets == 1 ? run(launch_sp24_rows_t<uint16_t, 1, false>) : run(launch_sp24_rows_t<uint16_t, 2, false>);
+  if (M <= SP24_EXACT_MAX_F32) return run(launch_sp24_rows_t<float, 1, false, 3>);
   return sets == 1   ? run(launch_sp24_rows_t<float, 1, false>)
          : sets == 2 ? run(launch_sp24_rows_t<float, 2, false>)
                      : run(launch_sp24_rows_t<float, 3, false>);

@@ -214,6 +214,10 @@ frx_status frx_ternary_stats(frx_ctx *ctx, const uint32_t *w, uint32_t N,
  * Replaces SparseTernaryMatMulOp::dispatch (src/compute/kernels/
  * sparse_ternary.rs:194-247), WGSL entry sparse_ternary_matmul_main (:54-112).
  *   meta [N][ceil(ceil(K/4)/6)] u32, scale [N] f32. Requires K % 4 == 0.
+ * 1-4 f32 tokens are multiplied in full fp32 (all 24 bits of x); from 5 on an
+ * f32 x travels as bf16 hi + lo, |x - hi - lo| <= 2^-17 |x|, as do the few-token
+ * calls that find no workspace (a context's first such call under graph
+ * capture) or whose metadata is 2 GiB and more.
  * With K % 64 == 0 both dtypes of x run on the sparse matrix pipe (f32 x as
  * bf16 hi | lo rows in a context workspace); below 512 tokens the K range is
  * split over workgroups where the token tiles leave compute units idle

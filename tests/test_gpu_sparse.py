@@ -323,6 +323,66 @@ def test_sparse_f32_activations_random_parity(ctx, M, K, N):
     assert_bf16_within_1ulp(yb.view(torch.int16).cpu().numpy().view(np.uint16), ref)
 
 
+def _dense64(meta, K):
+    """The signed 2:4 matrix of 5-bit metadata as float64 (patterns above 5 read as 5)."""
+    n, words = meta.shape
+    sh = torch.arange(0, 30, 5, device=meta.device, dtype=torch.int32)
+    v = ((meta[:, :, None] >> sh) & 31).view(n, words * 6)[:, :K // 4]
+    pairs = torch.tensor([(0, 1), (0, 2), (0, 3), (1, 2), (1, 3), (2, 3)], device=meta.device)
+    pos = pairs[(v & 7).clamp(max=5).long()]
+    full = torch.zeros((n, K // 4, 4), dtype=torch.float64, device=meta.device)
+    for j in range(2):
+        full.scatter_(2, pos[:, :, j:j + 1], (1 - 2 * ((v >> (3 + j)) & 1)).double()[:, :, None])
+    return full.view(n, K)
+
+
+def _random_meta(g, N, K):
+    return torch.randint(-2 ** 31, 2 ** 31 - 1, (N, (K // 4 + 5) // 6), generator=g, device="cuda:0", dtype=torch.int32)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 100, 12), (1, 4096, 4096), (1, 4096, 8192), (1, 11008, 8196), (2, 1040, 1000),
+                                   (2, 4096, 11008), (3, 4100, 8196), (3, 4096, 512), (4, 14336, 130), (4, 8188, 4100)])
+def test_sparse_f32_few_tokens_keep_every_bit(ctx, M, K, N):
+    """1-4 f32 tokens multiply all 24 bits of x. One nonzero activation per token:
+    every output is 0 or +- that value, whatever the order of the sums (two
+    bf16 planes would miss it by up to 2^-17). And random x against fp64: f32
+    sums of exact products, below 2^-20 of the result's norm where two planes
+    are 2^-18.6 off."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + K + N)
+    meta = _random_meta(g, N, K)
+    w = _dense64(meta, K)
+    one = torch.ones(N, device="cuda:0")
+    x = torch.zeros((M, K), device="cuda:0")
+    cols = torch.randint(0, K, (M,), generator=g, device="cuda:0")
+    odd = 2 * torch.randint(0, 2 ** 22, (M,), generator=g, device="cuda:0") + 1  # the last of 24 bits set
+    x[torch.arange(M, device="cuda:0"), cols] = 1.0 + odd.float() * 2.0 ** -23
+    y = torch.full((M, N), float("nan"), device="cuda:0")
+    ctx.sparse24_ternary_linear(meta, one, x, y)
+    torch.cuda.synchronize()
+    assert torch.equal(y.double(), x.double() @ w.t())
+    x = torch.randn((M, K), generator=g, device="cuda:0")
+    ctx.sparse24_ternary_linear(meta, one, x, y)
+    torch.cuda.synchronize()
+    ref = x.double() @ w.t()
+    assert (torch.linalg.norm(y.double() - ref) / torch.linalg.norm(ref)).item() < 2.0 ** -20
+
+
+@pytest.mark.parametrize("M,K,N", [(5, 4096, 1000), (8, 1040, 516), (16, 11008, 300), (24, 4100, 130), (25, 1024, 512),
+                                   (64, 2048, 1024)])
+def test_sparse_f32_planes_error(ctx, M, K, N):
+    """More f32 tokens travel as bf16 hi and lo: within 2^-16 of the result's
+    norm (2^-17 an element), which a wrong or missing lo plane (2^-9) is not."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + K + N)
+    meta = _random_meta(g, N, K)
+    x = torch.randn((M, K), generator=g, device="cuda:0")
+    s = 0.02 + 0.01 * torch.rand(N, generator=g, device="cuda:0")
+    y = torch.full((M, N), float("nan"), device="cuda:0")
+    ctx.sparse24_ternary_linear(meta, s, x, y)
+    torch.cuda.synchronize()
+    ref = (x.double() @ _dense64(meta, K).t()) * s.double()
+    assert (torch.linalg.norm(y.double() - ref) / torch.linalg.norm(ref)).item() < 2.0 ** -16
+
+
 def test_sparse_decode_paths_repeat_and_graph(ctx):
     """The decode GEMV (chunk sums added by the last-arriving chunk, its
     arrival counters left zero by every launch; and with a separate
