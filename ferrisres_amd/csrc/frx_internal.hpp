@@ -272,11 +272,13 @@ hipError_t launch_router_transpose(const void *src, int rt_bf16, void *dst, int 
 // Most routed rows (tokens x top_k) of the MoE decode path.
 constexpr int MOE_DEC_MAXA = 4;
 // Most routed rows of the decode-batch path (per-expert row tiles, frx_moe.hip),
-// and whether a batch takes it: up to 16 routes per expert. Above, an expert
-// has more tokens than the 16 columns of its row tiles and its weights are
-// decoded more than once, as the grouped GEMMs' 64-row tiles fill up (2048 /
-// 5632, 16 experts, top 2, bf16: 8 / 32 / 128 tokens 115.6 / 133.0 / 141.6 ->
-// 55.5 / 73.9 / 116.1 us; f32 157.6 / 186.1 / 196.3 -> 68.5 / 85.5 / 158.6).
+// and whether a batch takes it: up to 16 routes per expert. Above, the average
+// expert has more tokens than the 16 columns of its row tiles and its weights
+// are decoded more than once, as the grouped GEMMs' 64-row tiles fill up (2048 /
+// 5632, 16 experts, top 2, bf16: 8 / 32 / 128 tokens 107 / 130 / 130 -> 48 / 61
+// / 98 us; f32 145 / 180 / 185 -> 60 / 79 / 152). The average is enough to go
+// by: skewed routing runs in jobs of 16 routes, in 0.5 to 1.15 times the time of
+// even routing.
 constexpr int MOE_ROWS_MAXA = 512;
 inline bool moe_rows_fits(int A, int T, int H, int E) {
   return A <= MOE_ROWS_MAXA && (size_t)(H + 127) / 128 * T <= (size_t)GEMV_SK_MAX_TILES && A <= 16 * E;

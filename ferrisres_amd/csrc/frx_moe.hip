@@ -1478,10 +1478,20 @@ __global__ __launch_bounds__(512) void moe_dec_down_kernel(const DownArgs args, 
 // MFMA (fp32 activations as 8 tokens' hi planes and the same 8 tokens' lo
 // planes, added across lanes at the end), a wave owns whole 16-row tiles and
 // has its weights in flight before the activations are staged, and no wave
-// adds to another's sums. More tokens than columns: further passes.
-// A workgroup finds its expert's routes by a ballot over the selected
-// experts, so nothing has to group them first.
+// adds to another's sums. A workgroup takes one job, up to 16 routes of an
+// expert, and finds it by itself from the selected experts (mr_job), so nothing
+// has to group them first. However the routing falls, a launch has at most
+// (A + 15 E) / 16 jobs and a job at most two passes of the columns: an expert
+// that many tokens pick spreads over the chip. bf16, us, all of an expert's
+// passes in one workgroup / jobs / the grouped GEMMs: 128 tokens top 2 of 16
+// (2048 / 5632) at random 107 / 98 / 130, all on the same two 187 / 80 / 94; 512
+// tokens top 1 of 32 (1024 / 2048) 66 / 59 / 73, all on one 490 / 68 / 74. Jobs
+// of 24 and 32 routes: 109 and 109 at random, 90 and 92 on the same two. The
+// price is a second read of the weights of an expert with 17 routes and more
+// where they do not stay in cache (64 f32 tokens, 4096 / 8192, 8 experts: 172 ->
+// 188).
 constexpr int MR_COLS = 16;
+constexpr int MR_JOB = 16;           // routes of a job
 constexpr int MR_GU_CH = 2;          // 256-column blocks per weight batch (two batches in flight)
 constexpr int MR_DN_CH = 6;          // 256-column blocks of a down K part, all in flight
 constexpr int MR_DN_W = 4;           // waves of a down workgroup, 32 rows each
@@ -1492,18 +1502,56 @@ constexpr uint32_t MR_OOB = 0x80000000u;
 // 16 bytes that put the 16 rows of an operand read on different banks.
 __host__ __device__ constexpr int mr_stride(int n) { return (n + 255) / 256 * 256 + 8; }
 
-// Routes of expert e, in order, into list (by wave 0); every wave returns their
-// number.
-__device__ __forceinline__ int mr_routes(const uint32_t *idx, int A, int e, int *list) {
+// Jobs of a launch: up to MR_JOB tokens an expert each has one.
+static inline int mr_jobs(int T, int A, int E) {
+  return T <= MR_JOB ? E : (A + (MR_JOB - 1) * std::min(E, A)) / MR_JOB;
+}
+
+// Job j: its expert (-1 past the last job) and routes, in order, into list (by
+// wave 0), *n of them. single: job j is expert j, whose routes fit one job.
+// Every wave reads the selected experts once, all in flight, counts them in LDS
+// of its own (cnt) and scans the counts in registers: one memory latency and no
+// barrier. list is read after a barrier.
+__device__ __forceinline__ int mr_job(const uint32_t *idx, int A, int E, int j, bool single, int (*cnt)[64], int *list,
+                                      int *n) {
+  constexpr int R = MOE_ROWS_MAXA / 64;
   const int lane = threadIdx.x & 63;
-  int n = 0;
-  for (int a0 = 0; a0 < A; a0 += 64) {
-    const bool in = a0 + lane < A && (int)idx[min(a0 + lane, A - 1)] == e;
-    const unsigned long long m = __ballot(in);
-    if (in && threadIdx.x < 64) list[n + __popcll(m & ((1ull << lane) - 1ull))] = a0 + lane;
-    n += __popcll(m);
+  int sel[R];
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (64 * r < A) sel[r] = 64 * r + lane < A ? (int)idx[min(64 * r + lane, A - 1)] : -1;
+  int e = j, p0 = 0;
+  if (!single) {  // experts (at most 64, a lane each) in order, ceil(routes / MR_JOB) jobs each
+    int *c = cnt[threadIdx.x >> 6];
+    c[lane] = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (64 * r < A && sel[r] >= 0) atomicAdd(c + sel[r], 1);
+    const int jobs = (c[lane] + MR_JOB - 1) / MR_JOB;
+    int end = jobs;  // jobs of the experts up to this lane's: a scan within rows of 16, then over the rows
+    end += __builtin_amdgcn_update_dpp(0, end, 0x111, 0xF, 0xF, true);   // row_shr:1
+    end += __builtin_amdgcn_update_dpp(0, end, 0x112, 0xF, 0xF, true);   // row_shr:2
+    end += __builtin_amdgcn_update_dpp(0, end, 0x114, 0xF, 0xF, true);   // row_shr:4
+    end += __builtin_amdgcn_update_dpp(0, end, 0x118, 0xF, 0xF, true);   // row_shr:8
+    end += __builtin_amdgcn_update_dpp(0, end, 0x142, 0xA, 0xF, false);  // row_bcast:15, rows 1 and 3
+    end += __builtin_amdgcn_update_dpp(0, end, 0x143, 0xC, 0xF, false);  // row_bcast:31, rows 2 and 3
+    const unsigned long long past = __ballot(end > j);
+    if (past == 0) return -1;
+    e = __builtin_ctzll(past);
+    p0 = (j - __builtin_amdgcn_readlane(end - jobs, e)) * MR_JOB;
   }
-  return n;
+  int found = 0;
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (64 * r < A) {
+      const bool in = sel[r] == e;
+      const unsigned long long m = __ballot(in);
+      const int at = found + __popcll(m & ((1ull << lane) - 1ull)) - p0;
+      if (in && threadIdx.x < 64 && at >= 0 && at < MR_JOB) list[at] = 64 * r + lane;
+      found += __popcll(m);
+    }
+  *n = min(found - p0, MR_JOB);
+  return *n > 0 ? __builtin_amdgcn_readfirstlane(e) : -1;
 }
 
 // Rows src(r), r < rows, of n columns (n % 8 == 0, 16-byte aligned) into LDS
@@ -1608,21 +1656,21 @@ __device__ __forceinline__ f32x4 mr_add_planes(f32x4 v) {
   return v;
 }
 
-// grid (ceil(I / (16 WAVES)), E): a wave's 16 gate and 16 up rows of expert
-// blockIdx.y against its tokens; h = act(g, u) as bf16 hi and lo planes of
+// grid (ceil(I / (16 WAVES)), jobs): a wave's 16 gate and 16 up rows of the
+// job's expert against its tokens; h = act(g, u) as bf16 hi and lo planes of
 // the routes' rows [A][I].
 template <typename XT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void moe_rows_gateup_kernel(const GateUpArgs args, const XT *__restrict__ x,
-                                                                     int H, int I, int A, int top_k,
+                                                                     int H, int I, int E, int A, int top_k,
                                                                      const uint32_t *__restrict__ idx,
                                                                      uint16_t *__restrict__ h_hi,
                                                                      uint16_t *__restrict__ h_lo, int act) {
   constexpr int NP = sizeof(XT) == 2 ? 1 : 2, TP = MR_COLS / NP;  // planes, tokens per pass
   extern __shared__ __align__(16) uint16_t dsm[];
-  __shared__ int list[MOE_ROWS_MAXA];
-  const int e = blockIdx.y;
-  const int n = mr_routes(idx, A, e, list);
-  if (n == 0) return;
+  __shared__ int list[MR_JOB], cnt[WAVES][64];
+  int n;
+  const int e = mr_job(idx, A, E, blockIdx.y, A <= MR_JOB * top_k, cnt, list, &n);
+  if (e < 0) return;  // the whole workgroup
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 15, g = lane >> 4;
   const int n0 = (blockIdx.x * WAVES + wave) * 16, kw = H >> 4, nb = (H + 255) >> 8;
@@ -1699,24 +1747,24 @@ __global__ __launch_bounds__(WAVES * 64) void moe_rows_gateup_kernel(const GateU
   }
 }
 
-// grid (ceil(H / 128), S, E): a wave's 32 rows of W_down[e] over K part
-// blockIdx.y (ks columns) against h's planes of the expert's routes; the
+// grid (ceil(H / 128), S, jobs): a wave's 32 rows of W_down[e] over K part
+// blockIdx.y (ks columns) against h's planes of the job's routes; the
 // part's rows go to dpart[s][route][H] (device-coherent), and the last of a
 // token's S top_k workgroups of a row block adds them in order (d = part 0 +
 // part 1 + ..., acc from 0, k = 0, 1, ..., d * w rounded before the add,
 // CpuMoELayer's skip of |w| < 1e-8) and writes y.
 __global__ __launch_bounds__(MR_DN_W * 64, 3) void moe_rows_down_kernel(
     const DownArgs args, const uint16_t *__restrict__ h_hi, const uint16_t *__restrict__ h_lo, int H, int I, int ks,
-    int A, int top_k, const uint32_t *__restrict__ idx, float *__restrict__ dpart, unsigned *__restrict__ cnt,
+    int E, int A, int top_k, const uint32_t *__restrict__ idx, float *__restrict__ dpart, unsigned *__restrict__ cnt,
     const float *__restrict__ wts, int skip_small, void *__restrict__ y, int y_bf16) {
   constexpr int TP = MR_COLS / 2;
   constexpr int SC1 = 16;  // cache policy: performed at the point of coherence of all XCDs
   extern __shared__ __align__(16) uint16_t dsm[];
-  __shared__ int list[MOE_ROWS_MAXA];
-  __shared__ int last[MOE_ROWS_MAXA];
-  const int e = blockIdx.z, s = blockIdx.y, S = gridDim.y;
-  const int n = mr_routes(idx, A, e, list);
-  if (n == 0) return;
+  __shared__ int list[MR_JOB], last[MR_JOB], ecnt[MR_DN_W][64];
+  const int s = blockIdx.y, S = gridDim.y;
+  int n;
+  const int e = mr_job(idx, A, E, blockIdx.z, A <= MR_JOB * top_k, ecnt, list, &n);
+  if (e < 0) return;  // the whole workgroup
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 15, g = lane >> 4;
   const int n0 = (blockIdx.x * MR_DN_W + wave) * 32, kw = I >> 4;
@@ -2050,7 +2098,8 @@ hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
     // four-wave workgroups while four of them fit a compute unit's LDS, else
     // eight waves to a staged copy
     const int wv = gu_lds_rows <= 38 * 1024 ? 4 : 8;
-    const dim3 gg((I + 16 * wv - 1) / (16 * wv), E);
+    const int jobs = mr_jobs(T, A, E);
+    const dim3 gg((I + 16 * wv - 1) / (16 * wv), jobs);
 #define FRX_MR_GU(XT, WV)                                                                                            \
   {                                                                                                                  \
     static std::atomic<uint64_t> done;                                                                               \
@@ -2058,7 +2107,7 @@ hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
         hipSuccess)                                                                                                  \
       return err;                                                                                                    \
     hipLaunchKernelGGL((moe_rows_gateup_kernel<XT, WV>), gg, dim3(WV * 64), gu_lds_rows, stream, ga, (const XT *)x, H, \
-                       I, A, top_k, ws.idx, ws.h_hi, ws.h_lo, act);                                                  \
+                       I, E, A, top_k, ws.idx, ws.h_hi, ws.h_lo, act);                                               \
   }
     if (xt_bf16 && wv == 4) FRX_MR_GU(uint16_t, 4)
     else if (xt_bf16) FRX_MR_GU(uint16_t, 8)
@@ -2067,8 +2116,8 @@ hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
 #undef FRX_MR_GU
     if ((err = hipGetLastError()) != hipSuccess) return err;
     const size_t dl = (size_t)2 * std::min(T, MR_COLS / 2) * mr_stride(mks) * 2;
-    hipLaunchKernelGGL(moe_rows_down_kernel, dim3((H + 32 * MR_DN_W - 1) / (32 * MR_DN_W), mS, E), dim3(MR_DN_W * 64),
-                       dl, stream, da, ws.h_hi, ws.h_lo, H, I, mks, A, top_k, ws.idx, ws.dpart, ws.cnt, ws.wts,
+    hipLaunchKernelGGL(moe_rows_down_kernel, dim3((H + 32 * MR_DN_W - 1) / (32 * MR_DN_W), mS, jobs), dim3(MR_DN_W * 64),
+                       dl, stream, da, ws.h_hi, ws.h_lo, H, I, mks, E, A, top_k, ws.idx, ws.dpart, ws.cnt, ws.wts,
                        routing, y, yt_bf16);
     return hipGetLastError();
   }

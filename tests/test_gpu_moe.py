@@ -119,6 +119,80 @@ def test_moe_row_tiles_parity(ctx, T, H, I, E, k, act, xt):
             assert_bf16_within_1ulp(y.view(torch.int16).cpu().numpy().view(np.uint16), ref)
 
 
+@pytest.mark.parametrize("T,H,I,E,k,act,xt", [
+    (17, 64, 128, 4, 2, frx.ACT_SILU, "bf16"), (33, 128, 192, 64, 1, frx.ACT_GELU_TANH, "f32"),
+    (128, 192, 64, 16, 2, frx.ACT_SILU, "bf16"), (96, 64, 1600, 8, 1, frx.ACT_GELU_TANH_GATE, "f32"),
+    (250, 64, 64, 32, 2, frx.ACT_SILU, "bf16")])
+@pytest.mark.parametrize("skew", ["same", "one"])
+def test_moe_row_tiles_skewed_routing(ctx, T, H, I, E, k, act, xt, skew):
+    """Routing far from even: every token on the same experts, or one expert in
+    every token's choice and the rest at random. An expert's routes spread over
+    several jobs of 16 (the last one partly filled), other experts have one or
+    none."""
+    name = f"moe/skew/{T}x{H}x{I}x{E}x{k}"
+    xf, xb, rf, rb, ex = make_moe(name, T, H, I, E)
+    if xt == "f32":
+        xf = synth.normal(synth.seed_of(name, "xf32"), T * H).reshape(T, H)
+    # a common direction in the tokens, which the favoured experts' router rows follow
+    xf = xf.copy()
+    xf[:, :8] = 4.0
+    rf = rf.copy()
+    for j in range(k if skew == "same" else 1):
+        rf[j, :8] = 1.0 - 0.125 * j
+    xb, rb = synth.f32_to_bf16_bits(xf), synth.f32_to_bf16_bits(rf)
+    if xt == "bf16":
+        xf, rf = synth.bf16_bits_to_f32(xb), synth.bf16_bits_to_f32(rb)
+    ref, ridx, rw = run_oracle(xf, rf, ex, E, k, act)
+    assert (np.asarray(ridx).reshape(T, k)[:, 0] == 0).all()
+    for _ in range(2):  # the arrival counters are left at zero
+        y, idx, w = run_gpu(ctx, xf, xb, rf, rb, ex, E, k, act, xt=xt, no_up=act == frx.ACT_GELU_TANH_GATE)
+        np.testing.assert_array_equal(idx, ridx)
+        np.testing.assert_allclose(w, rw, rtol=0, atol=1e-6)
+        assert_close_f32(host(y), ref)
+
+
+def test_moe_time_does_not_hang_on_the_routing(ctx):
+    """512 tokens, top 1 of 32 experts: all of them on one expert may not cost
+    much more than spread over all (it took 7 times as long while an expert's
+    routes ran in one workgroup per row block; now about as long, so 2.5 times
+    is far from both)."""
+    T, H, I, E = 512, 1024, 2048, 32
+    g = torch.Generator(device="cuda:0").manual_seed(3)
+    words = lambda n, k: torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 16), generator=g, device="cuda:0",  # noqa: E731
+                                       dtype=torch.int32)
+    ws = [[words(n, k) if p == 0 else torch.rand(n, generator=g, device="cuda:0") for _ in range(E)]
+          for n, k in ((I, H), (I, H), (H, I)) for p in (0, 1)]
+    x = torch.randn((T, H), generator=g, device="cuda:0").to(torch.bfloat16)
+    x[:, :8] = 4.0
+    even = (torch.randn((E, H), generator=g, device="cuda:0") / H ** 0.5).to(torch.bfloat16)
+    even[:, :8] = 0.0
+    one = even.clone()
+    one[3, :8] = 2.0
+    y = torch.empty((T, H), device="cuda:0")
+    idx = torch.empty((T, 1), dtype=torch.int32, device="cuda:0")
+    st = torch.cuda.Stream()
+    ctx.set_stream(st)
+    took = {}
+    try:
+        for name, router in (("even", even), ("one", one)):
+            with torch.cuda.stream(st):
+                best = float("inf")
+                for _ in range(5):
+                    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                    a.record()
+                    for _ in range(20):
+                        ctx.moe_ternary_ffn(x, router, *ws, y, top_k=1, topk_idx=idx)
+                    b.record()
+                    torch.cuda.synchronize()
+                    best = min(best, a.elapsed_time(b))
+            took[name] = best
+            most = torch.bincount(idx.flatten().long(), minlength=E).max().item()
+            assert most == T if name == "one" else most < 64
+    finally:
+        ctx.set_stream(None)
+    assert took["one"] < 2.5 * took["even"], took
+
+
 @pytest.mark.parametrize("T", [1, 40])
 def test_moe_unaligned_tokens_and_router(ctx, T):
     """x and the router one bf16 element into larger buffers (element-aligned,
