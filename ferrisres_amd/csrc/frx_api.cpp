@@ -887,8 +887,10 @@ frx_status frx_moe_ternary_ffn(
   if ((size_t)T * top_k * I > (size_t)0x7FFFFFFF) return fail(ctx, FRX_ERR_SHAPE, "T*top_k*I too large");
   if (ctx->lora_on && ctx->lora_experts != E)
     return fail(ctx, FRX_ERR_SHAPE, "LoRA adapters were set for %u experts, the call has %u", ctx->lora_experts, E);
+  const frx::MoePath path = frx::moe_path(x, xt == FRX_BF16, w_gate, w_up, w_down, (int)T, (int)H, (int)I, (int)E,
+                                          (int)top_k, ctx->lora_on);
   // the decode batch's K parts only where the workspace may grow for them
-  const bool parts = (size_t)T * top_k <= (size_t)frx::MOE_ROWS_MAXA && may_count(ctx) &&
+  const bool parts = path == frx::MOE_ROWS && may_count(ctx) &&
                      may_grow(ctx, ctx->moe_ws_bytes,
                               frx::moe_workspace_bytes((int)T, (int)H, (int)I, (int)E, (int)top_k, true));
   const size_t need = frx::moe_workspace_bytes((int)T, (int)H, (int)I, (int)E, (int)top_k, parts);
@@ -898,7 +900,7 @@ frx_status frx_moe_ternary_ffn(
   frx::moe_workspace_carve(ctx->moe_ws, (int)T, (int)H, (int)I, (int)E, (int)top_k, parts, &ws);
   // a few routed rows (the decode paths): the down launch also combines,
   // through the context's arrival counters
-  if ((size_t)T * top_k <= (size_t)frx::MOE_ROWS_MAXA && may_count(ctx)) {
+  if (parts || (path == frx::MOE_DEC && may_count(ctx))) {
     if ((st = ensure_sk_counters(ctx)) != FRX_OK) return st;
     ws.cnt = ctx->sk_cnt;
   }

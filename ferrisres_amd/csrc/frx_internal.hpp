@@ -271,8 +271,8 @@ hipError_t launch_router_transpose(const void *src, int rt_bf16, void *dst, int 
 // MoE pipeline (frx_moe.hip).
 // Most routed rows (tokens x top_k) of the MoE decode path.
 constexpr int MOE_DEC_MAXA = 4;
-// Most routed rows of the decode-batch path (per-expert row tiles, frx_moe.hip),
-// and whether a batch takes it: up to 16 routes per expert. Above, the average
+// Most routed rows of the decode-batch path (per-expert row tiles, frx_moe.hip);
+// a batch takes it up to 16 routes per expert. Above, the average
 // expert has more tokens than the 16 columns of its row tiles and its weights
 // are decoded more than once, as the grouped GEMMs' 64-row tiles fill up (2048 /
 // 5632, 16 experts, top 2, bf16: 8 / 32 / 128 tokens 107 / 130 / 130 -> 48 / 61
@@ -280,9 +280,14 @@ constexpr int MOE_DEC_MAXA = 4;
 // by: skewed routing runs in jobs of 16 routes, in 0.5 to 1.15 times the time of
 // even routing.
 constexpr int MOE_ROWS_MAXA = 512;
-inline bool moe_rows_fits(int A, int T, int H, int E) {
-  return A <= MOE_ROWS_MAXA && (size_t)(H + 127) / 128 * T <= (size_t)GEMV_SK_MAX_TILES && A <= 16 * E;
-}
+
+// The kernels of a call: GEMVs per routed row, per-expert row tiles, the
+// pipelined grouped GEMMs or the register-staged ones. Asked once for the
+// workspace and once for the launch, so that nothing is allocated for a path
+// the call does not take.
+enum MoePath { MOE_DEC, MOE_ROWS, MOE_GROUPED, MOE_GROUPED_ANY };
+MoePath moe_path(const void *x, int xt_bf16, const uint32_t *const *w_gate, const uint32_t *const *w_up,
+                 const uint32_t *const *w_down, int T, int H, int I, int E, int top_k, bool lora);
 
 struct MoeWorkspace {
   uint32_t *idx;       // [T*k] selected experts (sorted order per token)
@@ -305,8 +310,8 @@ struct MoeWorkspace {
   float *dout_lo;      // [T*k][H] second partial (engine-2 path: the second
                        // K part)
   uint16_t *x2;        // [T][2H] f32 x as bf16 hi | lo rows (engine-2 path)
-  float *dpart;        // [S][T*k][H] K parts of the down projection (decode
-                       // batch; null above MOE_ROWS_MAXA routed rows)
+  float *dpart;        // [S][T*k][H] K parts of the down projection (MOE_ROWS;
+                       // null: such a call runs the grouped GEMMs)
   unsigned *cnt = nullptr;  // decode path: (column block, token) arrival
                             // counters, zero between launches; null: the
                             // combine runs as a launch of its own
@@ -321,7 +326,7 @@ struct MoeLora {
   int rank = 0;
   float scaling = 0.f;
 };
-// parts: room for a decode batch's K parts (dpart; null without).
+// parts: room for the K parts of MOE_ROWS (dpart; null without).
 size_t moe_workspace_bytes(int T, int H, int I, int E, int top_k, bool parts);
 void moe_workspace_carve(void *base, int T, int H, int I, int E, int top_k, bool parts,
                          MoeWorkspace *ws);

@@ -1904,7 +1904,35 @@ static int mr_down_parts(int I, int *ks) {
 
 static size_t mr_dpart_bytes(int A, int H, int I) {
   int ks;
-  return A <= MOE_ROWS_MAXA ? (size_t)mr_down_parts(I, &ks) * A * H * 4 : 0;
+  return (size_t)mr_down_parts(I, &ks) * A * H * 4;
+}
+
+// LDS of the gate/up launch: the staged columns of a pass.
+static size_t mr_gateup_lds(int T, int H, int xt_bf16) {
+  const int cols = xt_bf16 ? std::min(T, MR_COLS) : MR_COLS / 2 + std::min(T, MR_COLS / 2);
+  return (size_t)cols * mr_stride(H) * 2;
+}
+
+MoePath moe_path(const void *x, int xt_bf16, const uint32_t *const *w_gate, const uint32_t *const *w_up,
+                 const uint32_t *const *w_down, int T, int H, int I, int E, int top_k, bool lora) {
+  // the register-staged engine for everything but: H and I multiples of 64,
+  // 16-byte aligned weights, bf16 x or f32 x (8-byte aligned, split into bf16
+  // hi | lo rows for the gate/up GEMM)
+  const uintptr_t xa = reinterpret_cast<uintptr_t>(x);
+  if (!(xt_bf16 || (xa & 7) == 0) || H % 64 != 0 || I % 64 != 0) return MOE_GROUPED_ANY;
+  for (int i = 0; i < E; i++)
+    if ((reinterpret_cast<uintptr_t>(w_gate[i]) | reinterpret_cast<uintptr_t>(w_up[i]) |
+         reinterpret_cast<uintptr_t>(w_down[i])) & 15)
+      return MOE_GROUPED_ANY;
+  const size_t A = (size_t)T * top_k;
+  if (lora || (xa & 15) != 0 || A > MOE_ROWS_MAXA) return MOE_GROUPED;
+  if (A <= MOE_DEC_MAXA && H <= 8192 && I <= 16384) return MOE_DEC;  // LDS <= 40 KB
+  int ks;
+  // the rule (MOE_ROWS_MAXA), then what the launches can address and hold
+  const bool fits = A <= 16 * (size_t)E && (size_t)(H + 127) / 128 * T <= (size_t)GEMV_SK_MAX_TILES &&
+                    mr_down_parts(I, &ks) <= MR_DN_MAXS && mr_gateup_lds(T, H, xt_bf16) <= 144 * 1024 &&
+                    mr_dpart_bytes((int)A, H, I) < ((size_t)1 << 31) && (size_t)H * I / 4 < ((size_t)1 << 31);
+  return fits ? MOE_ROWS : MOE_GROUPED;
 }
 
 // ---- 5. combine ---------------------------------------------------------------
@@ -2041,13 +2069,8 @@ hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
                        (const float *)x, (const float *)router, T, H, E, EP, top_k, rch, ws.idx, ws.wts, topk_idx, topk_w, routing);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  // engine 2 (pipelined MFMA GEMMs): H and I multiples of 64, 16-byte
-  // aligned weights, bf16 x or f32 x (8-byte aligned, split into bf16 hi | lo
-  // rows for the gate/up GEMM); otherwise the register-staged engine 1
-  bool engine2 = (xt_bf16 || (reinterpret_cast<uintptr_t>(x) & 7) == 0) && H % 64 == 0 && I % 64 == 0;
-  for (int i = 0; i < E && engine2; i++)
-    engine2 = ((reinterpret_cast<uintptr_t>(w_gate[i]) | reinterpret_cast<uintptr_t>(w_up[i]) |
-                reinterpret_cast<uintptr_t>(w_down[i])) & 15) == 0;
+  const MoePath path = moe_path(x, xt_bf16, w_gate, w_up, w_down, T, H, I, E, top_k, lora.tbl != nullptr);
+  const bool engine2 = path != MOE_GROUPED_ANY;
   DownArgs da;
   for (int i = 0; i < MOE_MAXE; i++) {
     da.wd[i] = i < E ? w_down[i] : nullptr;
@@ -2061,8 +2084,7 @@ hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
     ga.sg[i] = v ? s_gate[i] : nullptr;
     ga.su[i] = v ? s_up[i] : nullptr;
   }
-  if (engine2 && A <= MOE_DEC_MAXA && !lora.tbl && H <= 8192 && I <= 16384 &&  // LDS <= 40 KB
-      (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+  if (path == MOE_DEC) {
     // decode: GEMVs per routed row (no grouping), down in two K parts
     const int ks = (I / 2 + 63) / 64 * 64;
     const size_t gl = (size_t)dec_pad2(H, MOE_DEC_GU_CH) * 4 + 2 * MOE_DEC_ROWS * 4 + 4 * 2 * 64 * 16;
@@ -2088,13 +2110,10 @@ hipError_t launch_moe(const void *x, int xt_bf16, const void *router,
                          ws.inv, H, top_k, (float *)y, routing);
     return hipGetLastError();
   }
-  int mks = 0;
-  const int mS = mr_down_parts(I, &mks);
-  const int cols = xt_bf16 ? std::min(T, MR_COLS) : MR_COLS / 2 + std::min(T, MR_COLS / 2);
-  const size_t gu_lds_rows = (size_t)cols * mr_stride(H) * 2;
-  if (engine2 && ws.dpart && ws.cnt && !lora.tbl && moe_rows_fits(A, T, H, E) && mS <= MR_DN_MAXS &&
-      gu_lds_rows <= 144 * 1024 && (size_t)mS * A * H * 4 < ((size_t)1 << 31) &&
-      (size_t)H * I / 4 < ((size_t)1 << 31) && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+  if (path == MOE_ROWS && ws.dpart && ws.cnt) {
+    int mks = 0;
+    const int mS = mr_down_parts(I, &mks);
+    const size_t gu_lds_rows = mr_gateup_lds(T, H, xt_bf16);
     // four-wave workgroups while four of them fit a compute unit's LDS, else
     // eight waves to a staged copy
     const int wv = gu_lds_rows <= 38 * 1024 ? 4 : 8;

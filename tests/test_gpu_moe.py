@@ -151,6 +151,40 @@ def test_moe_row_tiles_skewed_routing(ctx, T, H, I, E, k, act, xt, skew):
         assert_close_f32(host(y), ref)
 
 
+@pytest.mark.parametrize("what,T,H,I,E,k", [("average", 256, 2048, 512, 16, 2), ("lora", 64, 4096, 256, 8, 2),
+                                            ("long", 32, 4096, 12352, 4, 2), ("generic", 64, 2064, 528, 8, 2),
+                                            ("decode", 2, 4096, 4096, 4, 2)])
+def test_moe_workspace_without_unused_parts(what, T, H, I, E, k):
+    """Calls whose launch refuses the row tiles (more routes than 16 an expert,
+    LoRA, an intermediate of more than 8 K parts, widths of the register-staged
+    engine, a few routed rows) allocate no room for their K parts: the
+    workspace is what the other paths take (routed x, h planes, two outputs
+    per route, f32 x as planes; the rest is small), as computed here."""
+    g = torch.Generator(device="cuda:0").manual_seed(T)
+    words = lambda n, kk: torch.randint(-2 ** 31, 2 ** 31 - 1, (n, kk // 16), generator=g, device="cuda:0",  # noqa: E731
+                                        dtype=torch.int32)
+    mats = [[w] * E for n, kk in ((I, H), (I, H), (H, I)) for w in (words(n, kk), torch.rand(n, device="cuda:0"))]
+    x = torch.randn((T, H), generator=g, device="cuda:0").to(torch.bfloat16)
+    router = torch.randn((E, H), generator=g, device="cuda:0").to(torch.bfloat16)
+    y = torch.empty((T, H), device="cuda:0")
+    c = frx.Context(0)
+    try:
+        if what == "lora":
+            a, b = torch.zeros((8, H), device="cuda:0"), torch.zeros((I, 8), device="cuda:0")
+            c.set_moe_lora(8, 1.0, E, a_gate=[a] * E, b_gate=[b] * E)
+        live0 = c.workspace_stats()[0]
+        c.moe_ternary_ffn(x, router, *mats, y, top_k=k)
+        torch.cuda.synchronize()
+        A = T * k
+        base = A * I * 2 * 2 + A * H * 4 * 2 + T * H * 4
+        parts = -(-I // 1536) * A * H * 4
+        slack = 768 * 1024  # counters (256 KB), lists, alignment
+        assert c.workspace_stats()[0] - live0 < base + slack
+        assert what == "decode" or parts > slack  # so that the bound tells the two apart
+    finally:
+        c.close()
+
+
 def test_moe_time_does_not_hang_on_the_routing(ctx):
     """512 tokens, top 1 of 32 experts: all of them on one expert may not cost
     much more than spread over all (it took 7 times as long while an expert's
