@@ -649,10 +649,14 @@ static frx_status sp24_rows_auto(frx_ctx *ctx, const uint32_t *w, int prepared, 
 // Token count from which a 2:4 linear decodes its metadata once into the
 // prepared form (one pass over the matrix, 8 us at 11008 x 4096) before the
 // GEMM, where the cheaper operand decode repays it: 512, or 160 in whole-K tiles
-// (11008 x 4096, 256 / 333 tokens 49.0 / 63.2 us from the 5-bit form, 35.2 /
-// 40.7 and the pass from the prepared one; split over K, 4096 x 4096 at 333
-// tokens, 34.1 against 29.9 and 7).
+// whose K loop is long enough for it. Without / with the pass, us, 256 tokens,
+// K x N: bf16 x 1024 x 14336 17.7 / 20.7, 2048 x 14336 27.8 / 32.2, 3072 x 14336
+// 38.1 / 41.0, 4096 x 11008 47.9 / 45.2, 5120 x 13824 58 / 54, 11008 x 11008 116 /
+// 90; f32 x (two halves through the same weights) 512 x 14336 20.5 / 21.1, 1024 x
+// 14336 31.6 / 30.3, 4096 x 11008 96 / 74. Split over K it does not pay below
+// 512 (bf16 4096 x 4096 29.2 / 29.4, 11008 x 2048 28.9 / 30.8).
 constexpr uint32_t SP24_PREP_MIN_TOKENS = 512, SP24_PREP_MIN_TOKENS_WHOLE = 160;
+constexpr uint32_t SP24_PREP_WHOLE_MIN_K_BF16 = 4096, SP24_PREP_WHOLE_MIN_K_F32 = 1024;
 
 frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
                                        const float *scale, const void *x,
@@ -702,6 +706,7 @@ frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
   // (from 512 tokens the pass was always made; below, only where its workspace
   // is there or may be made)
   if (engine && (M >= SP24_PREP_MIN_TOKENS || (M >= SP24_PREP_MIN_TOKENS_WHOLE && !split &&
+                                               K >= (planes ? SP24_PREP_WHOLE_MIN_K_F32 : SP24_PREP_WHOLE_MIN_K_BF16) &&
                                                may_grow(ctx, ctx->spp_ws_bytes, (size_t)N * K / 4)))) {
     // the metadata decoded once into its prepared form for every token tile
     if ((st = ensure_buffer(ctx, &ctx->spp_ws, &ctx->spp_ws_bytes, (size_t)N * K / 4,

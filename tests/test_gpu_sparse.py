@@ -452,3 +452,27 @@ def test_sparse_gemm_tile_heights(ctx, M, K, N, xt):
     torch.cuda.synchronize()
     w = torch.from_numpy(np.asarray(t, np.float32).reshape(N, K)).to("cuda:0")
     assert torch.equal(y.double(), (x.double() @ w.double().t()) * s.double())
+
+
+@pytest.mark.parametrize("M,K,N,xt,prepares", [(256, 1024, 14336, "bf16", False), (200, 3072, 11008, "bf16", False),
+                                               (256, 512, 14336, "f32", False), (160, 4096, 11008, "bf16", True),
+                                               (200, 1024, 11008, "f32", True), (512, 512, 14336, "bf16", True)])
+def test_sparse_prepares_where_it_pays(M, K, N, xt, prepares):
+    """160 to 511 tokens in whole-K tiles decode the metadata into its prepared
+    form only over long rows (over 1024 columns the pass cost 17% of the call):
+    seen by the room it takes in the context, N K / 4 bytes. The output is the
+    same either way."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + K)
+    meta = _random_meta(g, N, K)
+    s = 2.0 ** torch.randint(-4, 1, (N,), generator=g, device="cuda:0").float()
+    x = torch.randint(-8, 9, (M, K), generator=g, device="cuda:0").float() / 4
+    y = torch.full((M, N), float("nan"), device="cuda:0")
+    c = frx.Context(0)
+    try:
+        c.sparse24_ternary_linear(meta, s, x.to(torch.bfloat16) if xt == "bf16" else x, y)
+        torch.cuda.synchronize()
+        live = c.workspace_stats()[0] - (M * K * 4 if xt == "f32" else 0)  # f32 x as planes
+        assert (live >= N * K // 4) == prepares and (prepares or live < 4096)
+    finally:
+        c.close()
+    assert torch.equal(y.double(), (x.double() @ _dense64(meta, K).t()) * s.double())
