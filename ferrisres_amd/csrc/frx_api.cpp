@@ -1007,18 +1007,14 @@ static frx_status check_ffn_down(frx_ctx *ctx, const uint32_t *w_down, const flo
   return FRX_OK;
 }
 
-// The dense FFN with its intermediate in `ws` (at least M*I*4 bytes, 256-byte
-// aligned). u_ws: the GEMM path's up projection (M > 16; null = the
-// context's workspace). allow_one: the one-launch kernel may run (it needs
-// the context's barrier words).
 // The down launch over h's bf16 planes [2][M][I] at 3-16 tokens: the split-K
 // GEMV (planes staged once per 128-row tile and column slice) where it
-// measured faster, i.e. I > 4096 (FFN_NUMS), and only where the call may allocate its
+// measured faster (ffn_down_split_min), and only where the call may allocate its
 // workspace; else the planes kernels of frx_gemv.hip.
 static frx_status ffn_down_planes(frx_ctx *ctx, const uint32_t *w_down, const float *s_down, const uint16_t *hp,
                                   void *y, frx_dtype yt, uint32_t M, uint32_t H, uint32_t I, bool may_alloc) {
   const bool split = may_alloc && ctx->gemv_split != FRX_GEMV_SPLIT_NEVER &&
-                     (ctx->gemv_split == FRX_GEMV_SPLIT_ALWAYS || I > 4096) &&
+                     (ctx->gemv_split == FRX_GEMV_SPLIT_ALWAYS || I >= (uint32_t)frx::ffn_down_split_min((int)M, (int)H, ctx->cus)) &&
                      (H + 127) / 128 <= (uint32_t)frx::GEMV_SK_MAX_TILES && (size_t)M * I * 4 < ((size_t)1 << 32) &&
                      may_count(ctx) &&
                      may_grow(ctx, ctx->sk_ws_bytes, frx::gemv_sk_workspace_bytes((int)I, (int)H, ctx->cus));
@@ -1037,6 +1033,10 @@ static frx_status ffn_down_planes(frx_ctx *ctx, const uint32_t *w_down, const fl
   return FRX_OK;
 }
 
+// The dense FFN with its intermediate in `ws` (at least M*I*4 bytes, 256-byte
+// aligned). u_ws: the GEMM path's up projection (M > 16; null = the
+// context's workspace). allow_one: the one-launch kernel may run (it needs
+// the context's barrier words).
 static frx_status ffn_run(frx_ctx *ctx, const void *x, frx_dtype xt, const uint32_t *w_gate, const float *s_gate,
                           const uint32_t *w_up, const float *s_up, const uint32_t *w_down, const float *s_down,
                           uint32_t M, uint32_t H, uint32_t I, frx_activation act, void *y, frx_dtype yt, void *ws,

@@ -1804,6 +1804,7 @@ static int gemv_xs_grid(int N, int tmax) {
 // 4096x11008, B = 16); 16 waves of four above. Two planes (16 KB per wave)
 // or two matrices (twice the weight registers): 8 waves of up to 2, 4 or 6
 // quads, so that a wave has 256 registers.
+// Two matrices take as many tiles as glu_staged_tiles says.
 // grp: the matrices of a same-x group (N = their 16-row tiles), else null.
 template <typename YT, int NW, int EPI, int XS, bool YSPLIT, bool GRP = false>
 static hipError_t launch_gemv_xs(const uint32_t *w, const float *scale, const uint32_t *w2, const float *scale2,
@@ -1833,8 +1834,11 @@ static hipError_t launch_gemv_xs(const uint32_t *w, const float *scale, const ui
     if (nq <= 32) FRX_XS_T(8, 4, 2);
     FRX_XS_T(8, 6, 1);
   } else {
-    if (nq <= 16) FRX_XS_T(8, 2, 4);
-    if (nq <= 32) FRX_XS_T(8, 4, 2);
+    const int tmax = glu_staged_tiles(K, N, XS == XS_BF16, device_cu_count());
+    if (nq <= 16 && tmax == 4) FRX_XS_T(8, 2, 4);
+    if (nq <= 16) FRX_XS_T(8, 2, 2);
+    if (nq <= 32 && tmax == 2) FRX_XS_T(8, 4, 2);
+    if (nq <= 32) FRX_XS_T(8, 4, 1);
     FRX_XS_T(8, 6, 1);
   }
 #undef FRX_XS_T
@@ -2356,16 +2360,14 @@ hipError_t launch_gemv_group(const void *x, int xt_bf16, int yt_bf16, int B, int
 hipError_t launch_gemv_glu(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up,
                            const float *s_up, const void *x, int xt_bf16, float *h, int B, int K,
                            int N, int gelu, hipStream_t stream) {
-  if (xt_bf16 && B >= gemv_glu_xs_min_b(K) && gemv_xs_ok(x, B, K, 1, 2)) {
+  if (xt_bf16 && B >= glu_staged_min_tokens(K, N) && gemv_xs_ok(x, B, K, 1, 2)) {
     if (gelu)
       return launch_gemv_xs<float, 2, GEMV_GEGLU, XS_BF16, false>(w_gate, s_gate, w_up, s_up, x, x, h, B, K, N,
                                                                    stream);
     return launch_gemv_xs<float, 2, GEMV_SWIGLU, XS_BF16, false>(w_gate, s_gate, w_up, s_up, x, x, h, B, K, N,
                                                                   stream);
   }
-  // fp32 x; one token over more than 4096 columns stays with the 16-row tiles
-  // (5120 / 13824 FFN 31.8 us so, 35.9 staged; 2048 / 5632 11.3 us staged)
-  if (!xt_bf16 && (B >= 2 || K <= 4096) && gemv_xs_ok(x, B, K, 2, 2)) {
+  if (!xt_bf16 && (B >= 2 || glu_staged_one_f32(K, N)) && gemv_xs_ok(x, B, K, 2, 2)) {
     if (gelu)
       return launch_gemv_xs<float, 2, GEMV_GEGLU, XS_F32, false>(w_gate, s_gate, w_up, s_up, x, x, h, B, K, N,
                                                                   stream);
@@ -2408,7 +2410,7 @@ hipError_t launch_glu_combine(const float *g, const float *u, float *h, size_t n
 hipError_t launch_gemv_glu_planes(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up,
                                   const float *s_up, const void *x, uint16_t *h_planes, int B, int K,
                                   int N, int gelu, hipStream_t stream) {
-  if (B >= gemv_glu_xs_min_b(K) && gemv_xs_ok(x, B, K, 1, 2)) {
+  if (B >= glu_staged_min_tokens(K, N) && gemv_xs_ok(x, B, K, 1, 2)) {
     if (gelu)
       return launch_gemv_xs<uint16_t, 2, GEMV_GEGLU, XS_BF16, true>(w_gate, s_gate, w_up, s_up, x, x, h_planes, B,
                                                                      K, N, stream);

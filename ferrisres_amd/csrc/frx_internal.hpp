@@ -5,6 +5,8 @@
 
 #include <atomic>
 
+#include "frx_policy.hpp"
+
 namespace frx {
 
 // Opts kernel `fn` in to `bytes` of dynamic LDS on the current device (the
@@ -29,16 +31,11 @@ inline hipError_t opt_in_lds(const void *fn, int bytes, std::atomic<uint64_t> &d
 //    (B = 5, 6, 7: 7.44 / 8.26, 7.62 / 9.60, 9.19 / 9.73 us with the 16-row
 //    tiles against 6.39 / 8.14, 6.57 / 8.31, 6.74 / 8.45 us staged); 2-4
 //    tokens take the 4-segment rows kernel before either.
-//  - the FFN's gate/up launch (h as bf16 planes): staged from 5 tokens (FFN at
-//    4096 / 14336, 5 / 7 tokens 25.9 / 27.4 us with operand loads, 24.4 / 23.7
-//    staged; 2048 / 5632 15.6 / 15.3 against 14.2 / 14.5), from 8 below 2048
-//    columns, where a workgroup's few quads leave its waves idle (1024 / 2048,
-//    5 tokens 8.8 against 9.3);
+//  - the FFN's gate/up launch (h as bf16 planes): frx_policy.hpp;
 //  - the FFN's down launch over those planes: staged from 6 tokens (FFN step
 //    at 6 / 7 tokens 26.6 / 28.3 us with operand loads, 25.9 / 26.4 us
 //    staged; at 4 / 5 tokens 25.2 / 25.2 against 25.7 / 25.2 us).
 constexpr int GEMV_XS_MIN_B = 5;
-constexpr int gemv_glu_xs_min_b(int K) { return K < 2048 ? 8 : 5; }
 constexpr int GEMV_PLANES_XS_MIN_B = 6;
 // The operand-load kernels (gemv_direct_kernel, gemv_tall_kernel) serve from
 // 8 tokens where the staged kernel does not fit (K above its quad limit).

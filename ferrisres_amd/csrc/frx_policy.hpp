@@ -1,5 +1,6 @@
-// frx_policy.hpp — host-side sizing rules of the context workspaces, kept
-// free of HIP so that a CPU build can check them.
+// frx_policy.hpp — host-side rules: the sizes of the context workspaces and
+// the kernels of the decode FFN, kept free of HIP so that a CPU build can check
+// them.
 #pragma once
 #include <stddef.h>
 
@@ -15,6 +16,62 @@ inline size_t grow_bytes(size_t have, size_t need) {
   const size_t g = have + have / 2;
   const size_t b = (g + 255) & ~(size_t)255;
   return b > a ? b : a;
+}
+
+// ---- the FFN of 1-16 tokens: gate and up over K columns and N rows each, then
+// the down projection (times are of the whole FFN, hidden / intermediate) -------
+
+// bf16 tokens from which gate and up leave the kernel with operand loads for the
+// staged one (gemv_xs_kernel): 5 over 2048 to 4096 columns (4096 / 14336, 5 / 7
+// tokens 25.9 / 27.4 us with operand loads, 24.4 / 23.7 staged; 4096 / 5632 15.3 /
+// 16.2 against 14.9 / 15.0; 5 tokens over few rows: 4096 / 4096 11.7 against 11.9),
+// else 8: below, a workgroup's few quads leave its waves idle (1024 / 2048, 5
+// tokens 8.8 against 9.3), above, its x outweighs its rows (5120 / 4096, 5 / 7
+// tokens 16.1 / 14.0 against 17.1 / 14.6, 5120 / 13824 28.3 / 30.5 against 29.8 /
+// 30.2) but where each unit has two tiles of them (5120 / 5632, 5 / 6 / 7 tokens 17.9
+// / 18.5 / 18.9 against 18.0 / 17.9 / 17.9, 5120 / 8192 20.0 / 20.7 / 21.2 against
+// 20.2 / 20.6 / 20.5).
+constexpr int glu_staged_min_tokens(int K, int N) {
+  if (K < 2048) return 8;
+  if (K > 4096) return N > 4096 && N <= 8192 ? 6 : 8;
+  return N > 4096 ? 5 : 6;
+}
+
+// Whether one f32 token takes the staged kernel: not over more than 4096
+// columns (5120 / 13824 31.8 us with the 16-row tiles, 35.9 staged) nor, where
+// short rows make a workgroup's start its time, over more than 4096 rows (1024 /
+// 5632 8.7 and 9.7, 1024 / 13824 12.1 and 13.7; but 1024 / 4096 7.7 and 7.6, 3072 /
+// 11008 18.0 and 16.6).
+constexpr bool glu_staged_one_f32(int K, int N) { return K <= 4096 && (K > 2048 || N <= 4096); }
+
+// Most 16-row tiles of both matrices in a workgroup of the staged kernel (its
+// weight registers allow 4 up to 4096 columns, 2 up to 8192, 1 above). bf16 x:
+// not so many that the fullest compute unit gets more of them, and where three
+// do not hold a unit's rows, two workgroups of two on it (their loads overlap)
+// before one of four. 5 / 16 tokens: 5120 / 11008, one tile 24.9 / 28.3 us, two
+// (344 workgroups, four tiles on the units that have two) 29.4 / 31.3; 5120 / 5632
+// 18.4 / 20.5 against 18.0 / 20.3; 4096 / 13824, two 21.7 / 24.8, four 22.1 / 25.6;
+// 4096 / 11008, two 20.8 / 23.9, three 19.3 / 22.2. f32 x has one workgroup per
+// unit anyway (LDS) and keeps the most tiles (2048 / 13824, 5 tokens 17.5 us with
+// four, 20.2 with two).
+constexpr int glu_staged_tiles(int K, int N, bool bf16, int cus) {
+  if (K > 8192) return 1;
+  if (K > 4096) {
+    const int one = ((N + 15) / 16 + cus - 1) / cus, two = 2 * (((N + 31) / 32 + cus - 1) / cus);
+    return bf16 && two > one ? 1 : 2;
+  }
+  return bf16 && N > 48 * cus ? 2 : 4;
+}
+
+// Intermediate from which the down projection of `tokens` is split over K. Up to
+// 8 tokens, whose planes share the 16 columns (whole rows / split: 4096 / 5632, 5 / 8
+// tokens 18.3 / 15.9 and 14.9 / 15.1 us; 2048 / 5632 16.5 / 14.0 and 13.1 / 13.3),
+// and above over H output rows whose 16-row tiles are few or past one round of
+// the compute units (12 / 16 tokens: 1024 / 5632 14.1 / 14.5 and 12.8 / 13.6, 5120 /
+// 5632 20.4 / 20.8 and 19.4 / 20.3; but 3072 / 5632 16.2 / 16.6 and 17.3 / 18.4, 4096 /
+// 5632 16.3 / 16.9 and 16.3 / 17.0, 2048 / 5632 14.5 / 14.8 and 14.4 / 15.0).
+constexpr int ffn_down_split_min(int tokens, int H, int cus) {
+  return tokens <= 8 || H < 2048 || H > 16 * cus ? 4097 : 8192;
 }
 
 }  // namespace frx

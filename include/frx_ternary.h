@@ -318,7 +318,8 @@ frx_status frx_ternary_glu(frx_ctx *ctx, const void *x, frx_dtype xt,
  *    4096.
  *  - bf16 x, 5 <= M <= 16: gate/up/act launch writing h as bf16 hi + lo
  *    planes (2^-17), then the down GEMV over both planes (split-K where
- *    I > 4096).
+ *    I > 4096, above 8 tokens and over 2048 to 4096 output columns I >=
+ *    8192).
  *  - M <= 3 in FRX_FFN_ONE_LAUNCH mode (H <= 4096, I <= 11520, multiples of
  *    64, 16-byte aligned weights): one launch with a grid barrier between
  *    the halves; h as bf16 hi + lo planes (2^-17).

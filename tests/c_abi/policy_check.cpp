@@ -1,6 +1,7 @@
 // Host check of the workspace growth rule (frx::grow_bytes): rising
 // requests make O(log) allocations and the retired buffers stay below twice
-// the final size. Built with g++ by tests/test_c_abi.py; no GPU.
+// the final size; and of the decode FFN's kernel rules. Built with g++ by
+// tests/test_c_abi.py; no GPU.
 #include <stdio.h>
 
 #include "frx_policy.hpp"
@@ -31,8 +32,49 @@ static int check(size_t first, size_t last, size_t step) {
   return 0;
 }
 
+// 16-row tiles on the fullest of `cus` units when workgroups hold up to t of
+// them (a workgroup per unit while the rows fit, as gemv_xs_grid).
+static int fullest(int N, int t, int cus) {
+  const int tiles = (N + 15) / 16;
+  int G = tiles < cus ? tiles : cus;
+  if ((N + G - 1) / G > 16 * t) G = (N + 16 * t - 1) / (16 * t);
+  const int rows = (N + G - 1) / G, per = (rows + 15) / 16;
+  return (G + cus - 1) / cus * per;
+}
+
+static int check_ffn_rules() {
+  const int units[] = {64, 228, 256, 304};
+  for (int cus : units)
+    for (int N = 16; N <= 40000; N += 16)
+      for (int K = 64; K <= 12288; K += 64)
+        for (int bf16 = 0; bf16 < 2; bf16++) {
+          const int t = frx::glu_staged_tiles(K, N, bf16, cus), most = K <= 4096 ? 4 : K <= 8192 ? 2 : 1;
+          bool ok = t >= 1 && t <= most && (bf16 || t == most);
+          // bf16: no fewer tiles would leave the fullest unit with fewer of them
+          if (bf16 && K > 4096) ok = ok && fullest(N, t, cus) <= fullest(N, 1, cus) + (t == 2 && N <= 32 * cus);
+          if (bf16 && K <= 4096 && N <= 64 * cus) ok = ok && fullest(N, t, cus) <= fullest(N, 2, cus);
+          if (!ok) {
+            printf("glu_staged_tiles(%d, %d, %d, %d) = %d\n", K, N, bf16, cus, t);
+            return 1;
+          }
+        }
+  // the measured sides of each line (hidden, intermediate)
+  const bool ok = frx::glu_staged_tiles(5120, 11008, true, 256) == 1 && frx::glu_staged_tiles(5120, 13824, true, 256) == 2 &&
+                  frx::glu_staged_tiles(5120, 11008, false, 256) == 2 && frx::glu_staged_tiles(4096, 11008, true, 256) == 4 &&
+                  frx::glu_staged_tiles(4096, 13824, true, 256) == 2 && frx::glu_staged_tiles(2048, 13824, false, 256) == 4 &&
+                  frx::glu_staged_min_tokens(5120, 4096) == 8 && frx::glu_staged_min_tokens(4096, 11008) == 5 &&
+                  frx::glu_staged_min_tokens(4096, 4096) == 6 && frx::glu_staged_min_tokens(1024, 2048) == 8 &&
+                  !frx::glu_staged_one_f32(1024, 13824) && frx::glu_staged_one_f32(1024, 4096) &&
+                  frx::glu_staged_one_f32(3072, 11008) && !frx::glu_staged_one_f32(5120, 13824) &&
+                  frx::glu_staged_min_tokens(5120, 5632) == 6 && frx::ffn_down_split_min(8, 3072, 256) <= 5632 &&
+                  frx::ffn_down_split_min(9, 3072, 256) > 5632 && frx::ffn_down_split_min(16, 3072, 256) <= 8192 &&
+                  frx::ffn_down_split_min(12, 1024, 256) <= 5632 && frx::ffn_down_split_min(12, 5120, 256) <= 5632;
+  if (!ok) printf("measured lines of the FFN rules\n");
+  return !ok;
+}
+
 int main() {
-  int bad = 0;
+  int bad = check_ffn_rules();
   // prefill M = 17..2048 at I = 11008 (fp32 h rows), and byte-sized steps
   bad |= check(17 * 11008 * 4, 2048 * 11008 * 4, 11008 * 4);
   bad |= check(1, 1 << 20, 1);

@@ -344,7 +344,11 @@ def test_ffn_one_launch_unsupported(one_launch):
 
 @pytest.mark.parametrize("M,H,I,xt", [(1, 1024, 2048, "f32"), (3, 2048, 5632, "f32"), (2, 4096, 16320, "f32"),
                                       (1, 5120, 1040, "f32"), (5, 2048, 4160, "bf16"), (7, 1024, 8208, "bf16"),
-                                      (16, 4096, 16400, "bf16"), (9, 8192, 8208, "bf16"), (16, 2064, 5632, "f32")])
+                                      (16, 4096, 16400, "bf16"), (9, 8192, 8208, "bf16"), (16, 2064, 5632, "f32"),
+                                      # a tile per workgroup over 5120 columns, two over 4096 and 13824 rows, 5-7
+                                      # tokens with operand loads, whole rows of h below 8192, one f32 token
+                                      (16, 5120, 11008, "bf16"), (12, 2064, 13824, "bf16"), (7, 5120, 2048, "bf16"),
+                                      (5, 4096, 4096, "bf16"), (12, 3072, 5632, "bf16"), (1, 1024, 5632, "f32")])
 def test_ffn_decode_batch_launches(ctx, M, H, I, xt):
     """The gate/up launch with three and four 16-row tiles per workgroup, its
     token and width limits, f32 x of up to three tokens in two launches, and the
