@@ -245,8 +245,8 @@ frx_status frx_sparse24_prepare(frx_ctx *ctx, const uint32_t *meta, uint32_t K,
 
 /* frx_sparse24_ternary_linear over prepared metadata (frx_sparse24_prepare):
  * the same products on the sparse matrix pipe, equal to it up to fp32
- * summation order (bit for bit where both take the same engine, i.e. bf16 x
- * with K % 64 == 0 at more than 16 tokens or where the K split applies).
+ * summation order (bit for bit above 32 tokens of bf16 x, where both take the
+ * same engine; up to 32 each form has slices and steps of its own).
  * x must be FRX_BF16 (FRX_ERR_UNSUPPORTED otherwise); y f32 or bf16. */
 frx_status frx_sparse24_prepared_linear(frx_ctx *ctx, const uint32_t *prepared,
                                         const float *scale, const void *x,

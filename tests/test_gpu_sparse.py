@@ -266,6 +266,31 @@ def test_prepared_linear_raw_metadata(ctx, M):
         np.testing.assert_array_equal(host(y), y5)
 
 
+@pytest.mark.parametrize("M,K,N", [(33, 4096, 4096), (48, 11008, 512), (160, 1024, 14336), (256, 4096, 11008),
+                                   (517, 2048, 1000), (1024, 512, 8192)])
+def test_prepared_linear_same_bits_above_32_tokens(ctx, M, K, N):
+    """Random activations, whose sums depend on their order: above 32 tokens both
+    forms give the same bits, split over K and in whole-K tiles, f32 and bf16
+    outputs; at 32 and below they agree within f32 sums."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + K)
+    meta = _random_meta(g, N, K)
+    s = 0.02 + 0.01 * torch.rand(N, generator=g, device="cuda:0")
+    prep = torch.empty((N, K // 16), dtype=torch.int32, device="cuda:0")
+    ctx.sparse24_prepare(meta, K, prep)
+    x = torch.randn((M, K), generator=g, device="cuda:0").to(torch.bfloat16)
+    for rows, same in ((M, True), (32, False), (17, False), (2, False)):
+        for dt in (torch.float32, torch.bfloat16):
+            y5, yp = (torch.full((rows, N), float("nan"), dtype=dt, device="cuda:0") for _ in range(2))
+            ctx.sparse24_ternary_linear(meta, s, x[:rows], y5)
+            ctx.sparse24_prepared_linear(prep, s, x[:rows], yp)
+            torch.cuda.synchronize()
+            if same:
+                assert torch.equal(y5, yp)
+            else:
+                err = torch.linalg.norm(y5.double() - yp.double()) / torch.linalg.norm(yp.double())
+                assert err.item() < (2.0 ** -20 if dt == torch.float32 else 2.0 ** -8)
+
+
 def test_prepared_entry_errors(ctx):
     """K % 64 != 0 and f32 activations are refused with a status, before any
     launch; the context stays usable."""
