@@ -629,8 +629,11 @@ frx_status frx_ternary_linear_group(frx_ctx *ctx, const void *x, frx_dtype xt, u
 static frx_status sp24_rows_auto(frx_ctx *ctx, const uint32_t *w, int prepared, const Staged &sg, frx_dtype xt,
                                  frx_dtype yt, uint32_t M, uint32_t K, uint32_t N, bool *done) {
   int ncs = 0, S = 0;
-  // NEVER keeps the unsplit engine from 5 tokens, where it has one worth keeping
-  *done = (ctx->gemv_split != FRX_GEMV_SPLIT_NEVER || M <= 4) &&
+  // NEVER keeps the whole-K engine, but for the 5-bit form's calls of one and two
+  // tokens and of up to four f32 ones, which have never had one of their own
+  // precision
+  const bool chunked = !prepared && (M <= 2 || (xt == FRX_F32 && M <= (uint32_t)frx::SP24_EXACT_MAX_F32));
+  *done = (ctx->gemv_split != FRX_GEMV_SPLIT_NEVER || chunked) &&
           frx::sp24_rows_plan((int)M, (int)K, (int)N, xt == FRX_BF16, prepared, ctx->cus, &ncs, &S) &&
           may_count(ctx) && may_grow(ctx, ctx->gk_ws_bytes, frx::sp24_rows_workspace_bytes((int)M, (int)N, S));
   if (!*done) return FRX_OK;

@@ -80,7 +80,9 @@ typedef enum frx_gemv_split {
                                 tokens at 14336 columns and from 3 tokens above 16384, at least
                                 3072 rows */
   FRX_GEMV_SPLIT_ALWAYS = 1, /* split K at every 2-16 token call */
-  FRX_GEMV_SPLIT_NEVER = 2,  /* whole-K kernels only */
+  FRX_GEMV_SPLIT_NEVER = 2,  /* whole-K kernels only; but the 2:4 linear over 5-bit metadata
+                                works in K chunks at 1-2 tokens and at 3-4 f32 tokens in
+                                every mode */
   FRX_GEMV_SPLIT_RANGE_ = 0x7fffffff
 } frx_gemv_split;
 

@@ -214,6 +214,40 @@ def test_sparse_split_k_raw_metadata(ctx, M, K, N):
     assert_close_f32(host(_run(ctx, meta, s, xf, xb, "bf16", "f32")), ref)
 
 
+@pytest.mark.parametrize("M,K,N,xt,prepared", [(3, 4096, 4096, "bf16", False), (4, 11008, 4096, "bf16", False),
+                                               (16, 4096, 512, "f32", False), (1, 4096, 4096, "bf16", True),
+                                               (4, 4096, 11008, "bf16", True), (24, 2048, 1024, "bf16", True)])
+def test_sparse_never_runs_whole_k(M, K, N, xt, prepared):
+    """Split mode NEVER: no K parts. Seen by the fp32 partials' room, which a call in
+    that mode does not allocate (and does in AUTO); the outputs agree within
+    f32 sums."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + K + N)
+    meta = _random_meta(g, N, K)
+    s = 0.02 + 0.01 * torch.rand(N, generator=g, device="cuda:0")
+    x = torch.randn((M, K), generator=g, device="cuda:0").to(torch.bfloat16 if xt == "bf16" else torch.float32)
+    c = frx.Context(0)
+    try:
+        prep = torch.empty((N, K // 16), dtype=torch.int32, device="cuda:0")
+        c.sparse24_prepare(meta, K, prep)
+        live, out = [], []
+        for mode in (frx.GEMV_SPLIT_NEVER, frx.GEMV_SPLIT_AUTO):
+            c.set_gemv_split(mode)
+            y = torch.full((M, N), float("nan"), device="cuda:0")
+            if prepared:
+                c.sparse24_prepared_linear(prep, s, x, y)
+            else:
+                c.sparse24_ternary_linear(meta, s, x, y)
+            torch.cuda.synchronize()
+            live.append(c.workspace_stats()[0])
+            out.append(y.double())
+    finally:
+        c.close()
+    planes = (M * K * 4 + 255) // 256 * 256 if xt == "f32" else 0  # f32 x as bf16 hi | lo rows
+    assert live[0] == planes and live[1] > planes
+    err = (torch.linalg.norm(out[0] - out[1]) / torch.linalg.norm(out[1])).item()
+    assert err < (2.0 ** -20 if xt == "bf16" else 2.0 ** -16)
+
+
 def _prepare(ctx, meta, K):
     N = meta.shape[0]
     prep = torch.empty((N, K // 16), dtype=torch.int32, device="cuda:0")
