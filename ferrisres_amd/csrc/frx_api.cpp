@@ -693,7 +693,8 @@ frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
       planes || (xt == FRX_BF16 && aligned16(sg.x) && K % 64 == 0 && (size_t)M * K * 2 < ((size_t)1 << 31));
   const int halves = planes ? 2 : 1;
   const bool split = engine && ctx->gemv_split != FRX_GEMV_SPLIT_NEVER &&
-                     frx::gemm_sp_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &sp, halves);
+                     frx::gemm_sp_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &sp, halves) &&
+                     may_grow(ctx, ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S));
   const uint32_t *wm = meta;
   const void *xin = sg.x;
   int prepared = 0;
@@ -773,7 +774,8 @@ frx_status frx_sparse24_prepared_linear(frx_ctx *ctx, const uint32_t *prepared, 
   if ((st = sp24_rows_auto(ctx, prepared, 1, sg, xt, yt, M, K, N, &done)) != FRX_OK || done) return st;
   hipError_t e;
   int S = 0, sp = 0;
-  if (ctx->gemv_split != FRX_GEMV_SPLIT_NEVER && frx::gemm_sp_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &sp)) {
+  if (ctx->gemv_split != FRX_GEMV_SPLIT_NEVER && frx::gemm_sp_splitk_plan((int)M, (int)K, (int)N, ctx->cus, &S, &sp) &&
+      may_grow(ctx, ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S))) {
     if ((st = ensure_buffer(ctx, &ctx->gk_ws, &ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S),
                             "split-K GEMM workspace allocation")) != FRX_OK)
       return st;

@@ -124,7 +124,8 @@ def test_noalloc_rejects_shapes_beyond_the_scratch(ctxs):
     assert ei.value.kind == "Unsupported" and "scratch" in str(ei.value)
 
 
-@pytest.mark.parametrize("what", ["linear", "linear_f32", "sparse24", "moe"])
+@pytest.mark.parametrize("what", ["linear", "linear_f32", "sparse24", "sparse24_split", "prepared", "ffn", "ffn_f32",
+                                  "moe"])
 def test_first_call_under_capture_keeps_its_route(what):
     """Calls that now prefer a kernel with a workspace, as a context's first call
     of that size under graph capture, where nothing can be allocated: they run on
@@ -143,6 +144,27 @@ def test_first_call_under_capture_keeps_its_route(what):
         call = lambda c, xx, y: c.moe_ternary_ffn(xx, router, *ws, y, top_k=2)  # noqa: E731
         call(fresh, big, torch.empty_like(big))  # a workspace from a larger prompt
         out = torch.empty_like(x)
+    elif what in ("sparse24_split", "prepared"):
+        # the row tiles and, behind them, the K parts of the tile engine
+        K, N = 4096, 512
+        meta, s, x = words(N, (K // 4 + 5) // 6) & 0x3FFFFFFF, scale(N), rnd(8, K).to(torch.bfloat16)
+        prep = torch.empty((N, K // 16), dtype=torch.int32, device=DEV)
+        other.sparse24_prepare(meta, K, prep)
+        call = (lambda c, xx, y: c.sparse24_prepared_linear(prep, s, xx, y)) if what == "prepared" else (
+            lambda c, xx, y: c.sparse24_ternary_linear(meta, s, xx, y))
+        out = torch.empty((8, N), device=DEV)
+    elif what in ("ffn", "ffn_f32"):
+        # the split down launch (planes of h; f32 h)
+        H, I = 512, 8192
+        ws = [words(I, H // 16), scale(I), words(I, H // 16), scale(I), words(H, I // 16), scale(H)]
+        big, x = rnd(16, H).to(torch.bfloat16), rnd(3, H)
+        if what == "ffn":
+            x = x.to(torch.bfloat16)
+        call = lambda c, xx, y: c.ternary_ffn(xx, *ws, y)  # noqa: E731
+        fresh.set_gemv_split(frx.GEMV_SPLIT_NEVER)  # a workspace for h, none for the parts
+        call(fresh, big, torch.empty((16, H), device=DEV))
+        fresh.set_gemv_split(frx.GEMV_SPLIT_AUTO)
+        out = torch.empty((3, H), device=DEV)
     elif what == "sparse24":
         K, N = 2064, 300
         meta, s, x = words(N, (K // 4 + 5) // 6) & 0x3FFFFFFF, scale(N), rnd(8, K)
