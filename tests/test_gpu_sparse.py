@@ -65,15 +65,19 @@ def test_sparse_parity_random(ctx, M, K, N, xt, yt):
 
 @pytest.mark.parametrize("M,K,N,xt", [(1, 100, 12, "bf16"), (2, 388, 260, "bf16"), (1, 4100, 1028, "bf16"),
                                       (2, 6004, 516, "bf16"), (1, 388, 260, "f32"), (3, 4100, 8196, "f32"),
-                                      (4, 8188, 4100, "f32")])
+                                      (4, 8188, 4100, "f32"),
+                                      (1, 388, 8196, "bf16"), (1, 100, 8192, "f32"), (1, 4100, 8192, "bf16"),
+                                      (1, 4100, 8196, "f32"), (1, 4612, 8192, "f32"), (1, 6004, 8708, "bf16")])
 @pytest.mark.parametrize("yt", ["f32", "bf16"])
 def test_sparse_decode_gemv_ragged(ctx, M, K, N, xt, yt):
-    """The one-token table GEMV (1-2 bf16 tokens; 3-4 f32 tokens over >= 32 M
-    codes) on ragged shapes: rows whose word count is not a multiple of 4 (a
-    row's last 16-byte metadata load runs into the next row, whose words are
-    cleared), a last chunk shorter than 16 words, a last row block shorter
-    than 256 rows, and chunk counts on both sides of the fused reduction's
-    limit (6004 columns: 16 chunks, added by the separate launch)."""
+    """Few tokens on ragged shapes, in the row tiles (fewer than 8192 rows, or
+    more than one token) and in the table GEMV (one token, 8192 rows and more):
+    rows whose word count is not a multiple of 4 (a row's last 16-byte metadata
+    load runs into the next row, whose words are cleared), a last chunk shorter
+    than 16 words, a last row block shorter than 256 rows, row blocks that are
+    and are not a multiple of 8 (both block orders), and chunk counts on both
+    sides of the fused reduction's limit (4612 and 6004 columns: 13 and 16
+    chunks, added by the separate launch)."""
     name = f"sp24/gemv/{M}x{K}x{N}"
     t = synth.sparse24_uniform(name, "w", N, K)
     meta = frx.pack_sparse24_gpu(t)
@@ -179,8 +183,9 @@ def test_sparse_split_k_bit_exact_on_dyadic(ctx, M, K, N):
     """Decode and small prefill, where 64-token tiles leave compute units
     idle: K is split into parts of whole 64-column steps (each reading its
     own metadata windows) whose fp32 partials are added in part order. Dyadic
-    inputs: every sum exact, the same bits as the unsplit kernels (split mode
-    NEVER) and as the dense product, f32 and bf16 outputs."""
+    inputs: every sum exact, the same bits in split mode NEVER (the unsplit
+    kernels; one and two tokens work in K chunks there too) and as the dense
+    product, f32 and bf16 outputs."""
     rng = np.random.default_rng(5 * M + K + N)
     t = synth.sparse24_uniform(f"dysk/{M}x{K}x{N}", "w", N, K)
     meta = frx.pack_sparse24_gpu(t)
@@ -351,10 +356,12 @@ def test_prepared_entry_errors(ctx):
 @pytest.mark.parametrize("M,K,N", [(1, 4096, 11008), (7, 2048, 1000), (130, 4096, 512), (700, 1024, 2048),
                                    (300, 1024, 11008), (2048, 1024, 2048), (4, 4096, 11008), (3, 11008, 4096)])
 def test_sparse_f32_activations_bit_exact_on_dyadic(ctx, M, K, N):
-    """f32 activations (the reference's dtype) split once into bf16 hi | lo
-    rows and multiplied on the sparse pipe over both halves: split over K,
-    whole-K, and from 512 tokens over the prepared form. Dyadic x lies in
-    the hi half: exact products and sums, f32 and bf16 outputs."""
+    """f32 activations (the reference's dtype) as bf16 planes on the sparse pipe
+    (one token over 8192 rows and more: in the table GEMV), in the row tiles,
+    split over K, whole-K, and over the prepared form. Dyadic x lies in the hi
+    plane: exact products and sums, f32 and bf16 outputs (what the other planes
+    hold is test_sparse_f32_few_tokens_keep_every_bit's and
+    test_sparse_f32_planes_error's)."""
     rng = np.random.default_rng(3 * M + K + N)
     t = synth.sparse24_uniform(f"f32sp/{M}x{K}x{N}", "w", N, K)
     meta = frx.pack_sparse24_gpu(t)
