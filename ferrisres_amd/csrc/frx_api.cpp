@@ -576,11 +576,12 @@ frx_status frx_ternary_linear_bias(frx_ctx *ctx, const uint32_t *w, const float 
 // 2-16 tokens: the matrices of a group run as one launch of the staged kernel
 // (x staged once for all their rows, one start-up) where each of them alone
 // would run that kernel, whose order of additions depends on K only, so the
-// outputs are the separate calls' bit for bit; and while a workgroup per compute
-// unit holds all the 16-row tiles, four each. 3 x 4096 x 4096, 5 / 16 bf16
-// tokens 13.6 / 14.2 -> 7.6 / 8.0 us, 2 / 5 / 16 f32 tokens 16.9 / 17.3 / 23.3 ->
-// 9.3 / 9.5 / 11.2; 2 x 11008 x 4096 (1376 tiles) would go from 14.0 / 15.0 to
-// 14.4 / 15.6 (bf16) and from 17.7 / 22.0 to 19.6 / 23.0 (f32).
+// outputs are the separate calls' bit for bit; and while all the 16-row tiles
+// come to at most four per compute unit and to fewer rounds of workgroups than
+// apart (group_fewer_rounds). 3 x 4096 x 4096, 5 / 16 bf16 tokens 13.6 / 14.2 ->
+// 7.6 / 8.0 us, 2 / 5 / 16 f32 tokens 16.9 / 17.3 / 23.3 -> 9.3 / 9.5 / 11.2; 2 x
+// 11008 x 4096 (1376 tiles) would go from 14.0 / 15.0 to 14.4 / 15.6 (bf16) and
+// from 17.7 / 22.0 to 19.6 / 23.0 (f32).
 static bool group_one_launch(const frx_ctx *ctx, const void *x, frx_dtype xt, uint32_t M, uint32_t K, uint32_t count,
                              const uint32_t *const *w, const int *n) {
   size_t rows = 0;
@@ -588,7 +589,9 @@ static bool group_one_launch(const frx_ctx *ctx, const void *x, frx_dtype xt, ui
     rows += (size_t)n[i];
     if (use_split(ctx, w[i], x, M, K, (uint32_t)n[i], xt)) return false;
   }
-  return rows <= (size_t)64 * ctx->cus && frx::gemv_group_xs_fits(x, xt == FRX_BF16, (int)M, (int)K, (int)count, w, n);
+  return rows <= (size_t)64 * ctx->cus &&
+         frx::group_fewer_rounds((int)count, n, (int)K, xt == FRX_BF16 ? 1 : 2, ctx->cus) &&
+         frx::gemv_group_xs_fits(x, xt == FRX_BF16, (int)M, (int)K, (int)count, w, n);
 }
 
 frx_status frx_ternary_linear_group(frx_ctx *ctx, const void *x, frx_dtype xt, uint32_t M, uint32_t K,

@@ -1824,6 +1824,7 @@ static hipError_t launch_gemv_xs(const uint32_t *w, const float *scale, const ui
     if (tiles <= 3 || TMAX == 3) FRX_XS(WV, (TMAX >= 3 ? 3 : 1), UM);                        \
     FRX_XS(WV, (TMAX >= 4 ? 4 : 1), UM);                                                     \
   }
+  // (the last argument of the linears: linear_staged_tiles)
   if constexpr (XS == XS_BF16 && NW == 1) {
     if (nq <= 16) FRX_XS_T(16, 1, 4);
     if (nq <= 32) FRX_XS_T(16, 2, 4);

@@ -74,4 +74,33 @@ constexpr int ffn_down_split_min(int tokens, int H, int cus) {
   return tokens <= 8 || H < 2048 || H > 16 * cus ? 4097 : 8192;
 }
 
+// ---- the staged kernel over one matrix, 2-16 tokens ----------------------------
+
+// Most 16-row tiles of a workgroup, by its weight registers (planes: 2 for f32 x).
+constexpr int linear_staged_tiles(int K, int planes) {
+  return planes == 1 ? (K <= 8192 ? 4 : 2) : K <= 4096 ? 4 : K <= 8192 ? 2 : 1;
+}
+
+// Rounds of workgroups, one to a compute unit, over `tiles` 16-row tiles: a
+// workgroup per unit while it holds them, else as many as hold them.
+constexpr int staged_rounds(int tiles, int tmax, int cus) {
+  return tiles <= tmax * cus ? 1 : ((tiles + tmax - 1) / tmax + cus - 1) / cus;
+}
+
+// Whether one launch over the tiles of a group's matrices takes fewer rounds
+// than a launch for each: above 8192 columns a workgroup holds two tiles, and
+// two launches of one round are ahead of one of two (5 / 16 bf16 tokens, us, apart /
+// one launch: 5504 and 2752 rows of 9216 15.4 / 15.9 and 16.9 / 17.3, 8192 and
+// 4096 rows of 11008 17.6 / 18.5 and 18.9 / 19.3; but 3 x 5440 of 11008 30.3 / 31.5
+// and 21.0 / 21.4, 2 x 4096 of 11008 15.0 / 15.4 and 10.2 / 10.6).
+constexpr bool group_fewer_rounds(int count, const int *n, int K, int planes, int cus) {
+  const int tmax = linear_staged_tiles(K, planes);
+  int tiles = 0, apart = 0;
+  for (int i = 0; i < count; i++) {
+    tiles += (n[i] + 15) / 16;
+    apart += staged_rounds((n[i] + 15) / 16, tmax, cus);
+  }
+  return staged_rounds(tiles, tmax, cus) < apart;
+}
+
 }  // namespace frx

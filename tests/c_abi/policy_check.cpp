@@ -73,8 +73,21 @@ static int check_ffn_rules() {
   return !ok;
 }
 
+// Groups of one round are always fewer than apart; more rounds, only if so.
+static int check_group_rule() {
+  const int qkv[] = {4096, 4096, 4096}, two[] = {5504, 2752}, wide[] = {8192, 4096}, three[] = {5440, 5440, 5440};
+  const int even[] = {4096, 4096}, one[] = {512};
+  const bool ok = frx::group_fewer_rounds(3, qkv, 4096, 1, 256) && frx::group_fewer_rounds(3, qkv, 4096, 2, 256) &&
+                  !frx::group_fewer_rounds(2, two, 9216, 1, 256) && frx::group_fewer_rounds(2, two, 8192, 1, 256) &&
+                  !frx::group_fewer_rounds(2, wide, 11008, 1, 256) && frx::group_fewer_rounds(3, three, 11008, 1, 256) &&
+                  frx::group_fewer_rounds(2, even, 11008, 1, 256) && !frx::group_fewer_rounds(2, even, 8256, 2, 256) &&
+                  !frx::group_fewer_rounds(1, one, 4096, 1, 256);
+  if (!ok) printf("measured lines of the group rule\n");
+  return !ok;
+}
+
 int main() {
-  int bad = check_ffn_rules();
+  int bad = check_ffn_rules() | check_group_rule();
   // prefill M = 17..2048 at I = 11008 (fp32 h rows), and byte-sized steps
   bad |= check(17 * 11008 * 4, 2048 * 11008 * 4, 11008 * 4);
   bad |= check(1, 1 << 20, 1);
