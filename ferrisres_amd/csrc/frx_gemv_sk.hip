@@ -10,11 +10,10 @@
 // weights against 16 x 11008 activations (352 KB as bf16, 704 KB as f32),
 // and every tile of the launch streams all of them through its L1 and LDS.
 // Here a workgroup owns 128 rows (eight waves of 16) and a slice of at most
-// SK_NC 256-column chunks (as few as keep the grid within two workgroups per
-// two or three per unit): the activations of the slice are staged once in LDS
-// for all 128 rows, which cuts the activation stream per weight byte by 8x; the
-// slices of a row tile run on other compute units and write fp32 partial
-// tiles part[s][16][Np] with device-coherent stores. The last slice of a row
+// SK_NC 256-column chunks (gemv_sk_chunks): the activations of the slice are
+// staged once in LDS for all 128 rows, which cuts the activation stream per
+// weight byte by 8x; the slices of a row tile run on other compute units and
+// write fp32 partial tiles part[s][B][Np] with device-coherent stores. The last slice of a row
 // tile to finish (a per-tile counter, agent-scope atomic) adds the slices of
 // each output in slice order (deterministic whatever the arrival order),
 // applies the row scale (and bias) and converts; no second launch and no

@@ -246,15 +246,17 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
 }
 
 // Chunks per slice: the fewest that keep the grid within three workgroups per
-// compute unit (11008 x 4096, 16 f32 tokens: 16.7 us within two, 14.7 within
-// three; the prepared form decodes faster and is ahead within two: 8 / 32
-// tokens 8.5 / 14.5 against 9.4 / 17.0) and the slices within one batch of the last workgroup's loads
-// (prepared 1024 x 14336, 16 tokens: 15.0 us in 56 slices, 8.0 in 14).
-// Measured over the tile engine that served these calls (launches back to
-// back, 4096 x 11008): f32 x, 2 / 8 / 16 / 24 tokens 11.6 / 30.1 / 30.7 / 31.5
-// -> 10.5 / 11.2 / 14.7 / 21.1 us; bf16 8 / 16 / 32 tokens 19.6 / 20.6 / 24.0
-// -> 10.4 / 11.6 / 17.9, prepared 16.3 / 17.6 / 19.9 -> 8.5 / 9.3 / 14.5. At 48
-// bf16 tokens (a third column set) the tile engine is level or ahead.
+// compute unit (13824 rows of 5120, 16 f32 / 32 bf16 tokens: 17.2 / 18.2 us
+// within two, 14.7 / 15.5 within three; the prepared form decodes faster and
+// keeps to two: 11008 rows of 4096, 8 / 32 tokens 8.5 / 14.5 against 9.4 / 17.0) and
+// the slices within one batch of the last workgroup's loads (1024 prepared rows
+// of 14336, 16 tokens: 15.0 us in 56 slices, 8.0 in 14).
+// Against what served these calls before (graph replays, 11008 rows of 4096
+// columns): f32 x, 2 / 4 tokens in the table GEMV 10.7 / 19.1 -> 8.8 / 9.0 us, 8 /
+// 16 / 24 in the tile engine 28.0 / 29.3 / 30.7 -> 9.8 / 12.9 / 16.1; bf16 8 / 16 /
+// 32 tokens 17.2 / 18.8 / 22.1 -> 9.3 / 10.7 / 15.2, prepared 14.4 / 15.7 / 18.6
+// -> 7.3 / 8.0 / 12.5. At 48 bf16 tokens (a third column set) the tile engine is
+// level or ahead.
 bool sp24_rows_plan(int M, int K, int N, int xt_bf16, int prepared, int cus, int *ncs, int *S) {
   if (M < 1 || K % 4 != 0 || M > (xt_bf16 ? SP24_ROWS_MAX_BF16 : SP24_ROWS_MAX_F32)) return false;
   const size_t wpr = prepared ? (size_t)K / 16 : ((size_t)K / 4 + 5) / 6;

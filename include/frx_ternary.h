@@ -220,10 +220,12 @@ frx_status frx_ternary_stats(frx_ctx *ctx, const uint32_t *w, uint32_t N,
  * f32 x travels as bf16 hi + lo, |x - hi - lo| <= 2^-17 |x|, as do the few-token
  * calls that find no workspace (a context's first such call under graph
  * capture) or whose metadata is 2 GiB and more.
- * With K % 64 == 0 both dtypes of x run on the sparse matrix pipe (f32 x as
- * bf16 hi | lo rows in a context workspace); below 512 tokens the K range is
- * split over workgroups where the token tiles leave compute units idle
- * (fp32 partials in a context workspace, added in a fixed order). */
+ * Up to 32 bf16 (24 f32) tokens run in 128-row tiles over slices of K, any K and
+ * N (one token over 8192 rows and more: a table-driven GEMV); more tokens with K
+ * % 64 == 0 in token tiles on the sparse matrix pipe (f32 x as bf16 hi | lo rows
+ * in a context workspace), K split over workgroups where the tiles leave compute
+ * units idle. fp32 partials live in a context workspace and are added in a
+ * fixed order. */
 frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
                                        const float *scale, const void *x,
                                        frx_dtype xt, void *y, frx_dtype yt,
@@ -240,8 +242,9 @@ frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
  *   16-byte aligned), K % 64 == 0; patterns 6 and 7 read as 5 and bits
  *   30-31 of a word are ignored, as in frx_sparse24_ternary_linear.
  * frx_sparse24_ternary_linear prepares into a context workspace by itself
- * from 512 tokens; a caller that prepares at upload saves that pass
- * (10.6 us at 11008 x 4096). */
+ * from 512 tokens, and from 160 where K is not split and long enough to repay
+ * the pass (4096 columns, f32 x 1024); a caller that prepares at upload saves
+ * that pass (8 us at 11008 x 4096). */
 frx_status frx_sparse24_prepare(frx_ctx *ctx, const uint32_t *meta, uint32_t K,
                                 uint32_t N, uint32_t *prepared);
 
@@ -327,8 +330,11 @@ frx_status frx_ternary_glu(frx_ctx *ctx, const void *x, frx_dtype xt,
  *    the halves; h as bf16 hi + lo planes (2^-17).
  *  - f32 x at M <= 16, and every other shape at M <= 16: h in fp32, then the
  *    down GEMV with fp32 input, as the reference keeps it.
- *  - M > 16: gate and up GEMMs (the up projection in a second context
- *    workspace), an element-wise fp32 combine, then the down GEMM.
+ *  - M > 16 (H, I multiples of 64, 16-byte aligned weights): one gate/up GEMM
+ *    that writes h as bf16 hi | lo rows (2^-17), then the down GEMM over them.
+ *    With few tiles, and for other shapes, gate and up GEMMs (the up projection
+ *    in a second context workspace), an element-wise fp32 combine, then the down
+ *    GEMM.
  * Workspaces grow on the first call at a larger size, and that first call
  * must not be under graph capture. A workspace replaced by a larger one is
  * kept until frx_destroy, so graphs captured at smaller sizes stay valid.
@@ -350,8 +356,9 @@ frx_status frx_ternary_ffn(frx_ctx *ctx, const void *x, frx_dtype xt,
  * forbid hipMalloc. Same arguments, semantics and kernels as frx_ternary_ffn
  * in FRX_FFN_TWO_LAUNCH execution with FRX_GEMV_SPLIT_NEVER (whatever
  * frx_set_ffn_mode and frx_set_gemv_split selected: the split-K down launch
- * needs a context workspace), but
- * the intermediate lives in a fixed device array of the library
+ * needs a context workspace; f32 x above 16 tokens is split into bf16 hi + lo
+ * inside the GEMMs instead of in a workspace, so that only the order of the
+ * sums differs), but the intermediate lives in a fixed device array of the library
  * (FRX_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends) and the
  * call allocates nothing. It needs M*I*4 bytes of that array (rounded up to
  * 256) for M <= 16 and twice that above; larger shapes return
