@@ -1522,11 +1522,15 @@ __device__ __forceinline__ int mr_job(const uint32_t *idx, int A, int E, int j, 
     if (64 * r < A) sel[r] = 64 * r + lane < A ? (int)idx[min(64 * r + lane, A - 1)] : -1;
   int e = j, p0 = 0;
   if (!single) {  // experts (at most 64, a lane each) in order, ceil(routes / MR_JOB) jobs each
+    // (a wave's LDS operations complete in order; the barriers, which cost no
+    // instruction, keep the compiler to it)
     int *c = cnt[threadIdx.x >> 6];
     c[lane] = 0;
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int r = 0; r < R; r++)
       if (64 * r < A && sel[r] >= 0) atomicAdd(c + sel[r], 1);
+    __builtin_amdgcn_wave_barrier();
     const int jobs = (c[lane] + MR_JOB - 1) / MR_JOB;
     int end = jobs;  // jobs of the experts up to this lane's: a scan within rows of 16, then over the rows
     end += __builtin_amdgcn_update_dpp(0, end, 0x111, 0xF, 0xF, true);   // row_shr:1
