@@ -655,14 +655,16 @@ static frx_status sp24_rows_auto(frx_ctx *ctx, const uint32_t *w, int prepared, 
 // Token count from which a 2:4 linear decodes its metadata once into the
 // prepared form (one pass over the matrix, 8 us at 11008 x 4096) before the
 // GEMM, where the cheaper operand decode repays it: 512, or 160 in whole-K tiles
-// whose K loop is long enough for it. Without / with the pass, us, 256 tokens,
-// K x N: bf16 x 1024 x 14336 17.7 / 20.7, 2048 x 14336 27.8 / 32.2, 3072 x 14336
-// 38.1 / 41.0, 4096 x 11008 47.9 / 45.2, 5120 x 13824 58 / 54, 11008 x 11008 116 /
-// 90; f32 x (two halves through the same weights) 512 x 14336 20.5 / 21.1, 1024 x
-// 14336 31.6 / 30.3, 4096 x 11008 96 / 74. Split over K it does not pay below
-// 512 (bf16 4096 x 4096 29.2 / 29.4, 11008 x 2048 28.9 / 30.8).
+// whose K loop is long enough for it, the longer the more rows the pass decodes.
+// Without / with the pass, us, K x N: bf16 x, 256 tokens 1024 x 14336 17.7 /
+// 20.7, 2048 x 14336 27.8 / 32.2, 3072 x 14336 38.1 / 41.0, 3840 x 14336 46.2 / 43.8,
+// 4096 x 11008 47.9 / 45.2, 11008 x 11008 116 / 90; 400 tokens 2048 x 8192 28.1 /
+// 29.0, 3328 x 8192 40.9 / 37.5, 3072 x 5312 37.3 / 33.7; f32 x (two halves through
+// the same weights), 256 tokens 512 x 14336 20.5 / 21.1, 896 x 11008 28.7 / 26.3,
+// 4096 x 11008 96 / 74; 400 tokens 512 x 5312 20.1 / 18.8. Split over K it does not
+// pay below 512 (bf16 4096 x 4096 29.2 / 29.4, 11008 x 2048 28.9 / 30.8).
 constexpr uint32_t SP24_PREP_MIN_TOKENS = 512, SP24_PREP_MIN_TOKENS_WHOLE = 160;
-constexpr uint32_t SP24_PREP_WHOLE_MIN_K_BF16 = 4096, SP24_PREP_WHOLE_MIN_K_F32 = 1024;
+constexpr uint32_t sp24_prep_whole_min_k(bool planes, uint32_t N) { return planes ? 256 + N / 32 : 2560 + N / 11; }
 
 frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
                                        const float *scale, const void *x,
@@ -713,7 +715,7 @@ frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
   // (from 512 tokens the pass was always made; below, only where its workspace
   // is there or may be made)
   if (engine && (M >= SP24_PREP_MIN_TOKENS || (M >= SP24_PREP_MIN_TOKENS_WHOLE && !split &&
-                                               K >= (planes ? SP24_PREP_WHOLE_MIN_K_F32 : SP24_PREP_WHOLE_MIN_K_BF16) &&
+                                               K >= sp24_prep_whole_min_k(planes, N) &&
                                                may_grow(ctx, ctx->spp_ws_bytes, (size_t)N * K / 4)))) {
     // the metadata decoded once into its prepared form for every token tile
     if ((st = ensure_buffer(ctx, &ctx->spp_ws, &ctx->spp_ws_bytes, (size_t)N * K / 4,

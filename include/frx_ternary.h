@@ -243,7 +243,7 @@ frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
  *   30-31 of a word are ignored, as in frx_sparse24_ternary_linear.
  * frx_sparse24_ternary_linear prepares into a context workspace by itself
  * from 512 tokens, and from 160 where K is not split and long enough to repay
- * the pass (4096 columns, f32 x 1024); a caller that prepares at upload saves
+ * the pass (about 3000 to 4000 columns by N, f32 x 500 to 700); a caller that prepares at upload saves
  * that pass (8 us at 11008 x 4096). */
 frx_status frx_sparse24_prepare(frx_ctx *ctx, const uint32_t *meta, uint32_t K,
                                 uint32_t N, uint32_t *prepared);

@@ -522,6 +522,7 @@ def test_sparse_gemm_tile_heights(ctx, M, K, N, xt):
 
 @pytest.mark.parametrize("M,K,N,xt,prepares", [(256, 1024, 14336, "bf16", False), (200, 3072, 11008, "bf16", False),
                                                (256, 512, 14336, "f32", False), (160, 4096, 11008, "bf16", True),
+                                               (443, 3328, 5312, "bf16", True), (400, 768, 8192, "f32", True),
                                                (200, 1024, 11008, "f32", True), (512, 512, 14336, "bf16", True)])
 def test_sparse_prepares_where_it_pays(M, K, N, xt, prepares):
     """160 to 511 tokens in whole-K tiles decode the metadata into its prepared
