@@ -24,8 +24,9 @@ inline size_t grow_bytes(size_t have, size_t need) {
 // bf16 tokens from which gate and up leave the kernel with operand loads for the
 // staged one (gemv_xs_kernel): 5 over 2048 to 4096 columns (4096 / 14336, 5 / 7
 // tokens 25.9 / 27.4 us with operand loads, 24.4 / 23.7 staged; 4096 / 5632 15.3 /
-// 16.2 against 14.9 / 15.0; 5 tokens over few rows: 4096 / 4096 11.7 against 11.9),
-// else 8: below, a workgroup's few quads leave its waves idle (1024 / 2048, 5
+// 16.2 against 14.9 / 15.0), else 8: over few rows they are level with the down
+// launch behind them and behind by themselves (gate and up of 2304 columns and 2048
+// rows, 6 / 7 tokens 4.6 / 4.8 us against 5.0 / 5.0); below, a workgroup's few quads leave its waves idle (1024 / 2048, 5
 // tokens 8.8 against 9.3), above, its x outweighs its rows (5120 / 4096, 5 / 7
 // tokens 16.1 / 14.0 against 17.1 / 14.6, 5120 / 13824 28.3 / 30.5 against 29.8 /
 // 30.2) but where each unit has two tiles of them (5120 / 5632, 5 / 6 / 7 tokens 17.9
@@ -34,7 +35,7 @@ inline size_t grow_bytes(size_t have, size_t need) {
 constexpr int glu_staged_min_tokens(int K, int N) {
   if (K < 2048) return 8;
   if (K > 4096) return N > 4096 && N <= 8192 ? 6 : 8;
-  return N > 4096 ? 5 : 6;
+  return N > 4096 ? 5 : 8;
 }
 
 // Whether one f32 token takes the staged kernel: not over more than 4096
