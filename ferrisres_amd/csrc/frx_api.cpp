@@ -677,7 +677,7 @@ frx_status frx_sparse24_ternary_linear(frx_ctx *ctx, const uint32_t *meta,
   if ((st = stage_linear(ctx, x, xt, scale, y, yt, M, K, N, &sg)) != FRX_OK) return st;
   hipError_t e = hipSuccess;
   int S = 0, sp = 0;
-  if (frx::sp24_gemv_plan((int)M, (int)K, (int)N, &S)) {
+  if (frx::sp24_gemv_plan((int)M, (int)K, (int)N, xt == FRX_BF16, ctx->cus, &S)) {
     // decode: the metadata read once by a table-driven GEMV
     if ((st = ensure_buffer(ctx, &ctx->gk_ws, &ctx->gk_ws_bytes, frx::gemm_splitk_workspace_bytes((int)M, (int)N, S),
                             "split-K GEMM workspace allocation")) != FRX_OK)

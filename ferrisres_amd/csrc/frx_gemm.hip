@@ -648,9 +648,15 @@ __global__ __launch_bounds__(256) void sp24_gemv_kernel(const uint32_t *__restri
 // compute units and a code costs one LDS read and one add. Below 8192 rows,
 // and from two tokens, the sparse pipe is ahead (frx_sp24.hip): 4096 x 4096
 // f32 / bf16 7.6 / 7.8 here against 7.1 / 6.9 us, 4096 x 11008 9.7 / 9.7
-// against 9.4 / 8.9, 11008 x 4096 8.8 / 8.9 against 10.5 / 9.9.
-bool sp24_gemv_plan(int M, int K, int N, int *S) {
-  if (M != 1 || N < 8192 || K % 4 != 0 || N % 4 != 0 || (N + 255) / 256 > GEMV_SK_MAX_TILES) return false;
+// against 9.4 / 8.9, 11008 x 4096 8.8 / 8.9 against 10.5 / 9.9; but from 6144 rows
+// on only while its slices are at most two workgroups per unit (rows x columns,
+// f32, here / there: 6144 x 4096 7.2 / 8.4, 528 workgroups; 8188 x 4096 7.4 / 9.2,
+// 704; 7680 x 14336 13.1 / 15.3, 600; 7168 x 5120 8.4 / 8.0, 392).
+bool sp24_gemv_plan(int M, int K, int N, int xt_bf16, int cus, int *S) {
+  if (M != 1 || N < 6144 || K % 4 != 0 || N % 4 != 0 || (N + 255) / 256 > GEMV_SK_MAX_TILES) return false;
+  int ncs, slices;
+  if (N < 8192 && sp24_rows_plan(M, K, N, xt_bf16, 0, cus, &ncs, &slices) && (N + 127) / 128 * slices <= 2 * cus)
+    return false;
   const int wpr = ((K >> 2) + 5) / 6;
   if ((long)N * wpr * 4 >= (1L << 32)) return false;  // the metadata's buffer range
   *S = (wpr + SPV_WORDS - 1) / SPV_WORDS;

@@ -140,7 +140,7 @@ hipError_t launch_gemm_sp_planes(const uint32_t *meta, int prepared, const float
 // 0): S chunk partials of N fp32 in part, added in order into y by the last
 // chunk of each 256-row block (counters: the split-K GEMV's, zero between
 // launches).
-bool sp24_gemv_plan(int M, int K, int N, int *S);
+bool sp24_gemv_plan(int M, int K, int N, int xt_bf16, int cus, int *S);
 hipError_t launch_sp24_gemv(const uint32_t *meta, const float *scale, const void *x, int xt_bf16, void *y,
                             int yt_bf16, int K, int N, int S, float *part, unsigned *counters, hipStream_t stream);
 // A decode batch over 2:4 metadata (GPU 5-bit layout, or prepared with bf16 x)

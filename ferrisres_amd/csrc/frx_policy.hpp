@@ -24,14 +24,14 @@ inline size_t grow_bytes(size_t have, size_t need) {
 // bf16 tokens from which gate and up leave the kernel with operand loads for the
 // staged one (gemv_xs_kernel): 5 over 2048 to 4096 columns (4096 / 14336, 5 / 7
 // tokens 25.9 / 27.4 us with operand loads, 24.4 / 23.7 staged; 4096 / 5632 15.3 /
-// 16.2 against 14.9 / 15.0), else 8: over few rows they are level with the down
-// launch behind them and behind by themselves (gate and up of 2304 columns and 2048
-// rows, 6 / 7 tokens 4.6 / 4.8 us against 5.0 / 5.0); below, a workgroup's few quads leave its waves idle (1024 / 2048, 5
-// tokens 8.8 against 9.3), above, its x outweighs its rows (5120 / 4096, 5 / 7
-// tokens 16.1 / 14.0 against 17.1 / 14.6, 5120 / 13824 28.3 / 30.5 against 29.8 /
-// 30.2) but where each unit has two tiles of them (5120 / 5632, 5 / 6 / 7 tokens 17.9
-// / 18.5 / 18.9 against 18.0 / 17.9 / 17.9, 5120 / 8192 20.0 / 20.7 / 21.2 against
-// 20.2 / 20.6 / 20.5).
+// 16.2 against 14.9 / 15.0), else 8. Over up to 4096 rows the FFN is level and
+// frx_ternary_glu slower (2304 columns, 2048 rows, 6 / 7 tokens 4.6 / 4.8 us against
+// 5.0 / 5.0). Below 2048 columns a workgroup's few quads leave its waves idle
+// (1024 / 2048, 5 tokens 8.8 against 9.3). Above 4096 its x outweighs its rows
+// (5120 / 4096, 5 / 7 tokens 16.1 / 14.0 against 17.1 / 14.6, 5120 / 13824 28.3 / 30.5
+// against 29.8 / 30.2) but where each unit has two tiles of them (5120 / 5632, 5 / 6
+// / 7 tokens 17.9 / 18.5 / 18.9 against 18.0 / 17.9 / 17.9, 5120 / 8192 20.0 / 20.7 /
+// 21.2 against 20.2 / 20.6 / 20.5).
 constexpr int glu_staged_min_tokens(int K, int N) {
   if (K < 2048) return 8;
   if (K > 4096) return N > 4096 && N <= 8192 ? 6 : 8;

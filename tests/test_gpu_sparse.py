@@ -67,7 +67,8 @@ def test_sparse_parity_random(ctx, M, K, N, xt, yt):
                                       (2, 6004, 516, "bf16"), (1, 388, 260, "f32"), (3, 4100, 8196, "f32"),
                                       (4, 8188, 4100, "f32"),
                                       (1, 388, 8196, "bf16"), (1, 100, 8192, "f32"), (1, 4100, 8192, "bf16"),
-                                      (1, 4100, 8196, "f32"), (1, 4612, 8192, "f32"), (1, 6004, 8708, "bf16")])
+                                      (1, 4100, 8196, "f32"), (1, 4612, 8192, "f32"), (1, 6004, 8708, "bf16"),
+                                      (1, 4612, 6148, "f32"), (1, 4100, 7684, "bf16"), (1, 5124, 7172, "f32")])
 @pytest.mark.parametrize("yt", ["f32", "bf16"])
 def test_sparse_decode_gemv_ragged(ctx, M, K, N, xt, yt):
     """Few tokens on ragged shapes, in the row tiles (fewer than 8192 rows, or
