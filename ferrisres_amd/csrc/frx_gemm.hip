@@ -447,7 +447,11 @@ bool gemm_glu_plan(int M, int H, int I, int cus, int halves, int *bm) {
                       (float)(halves * (H / 64) + 4) / 64.f;
   int S, kp;
   const float apart = 2.f * gemm_plan(M, H, I, cus, halves, &S, &kp) + 6.f + (float)M * (float)I * 20.f / 4.5e6f;
-  return fused < apart;
+  // a few tiles take longer than the model's fill (2816 / 512, 61 tokens, four
+  // tiles: 27.4 us against 27.6 by the model, the whole FFN 44.3 against 39.2;
+  // 2816 / 2048, 16 tiles: 46.9 against 44.8)
+  const long tiles = (long)((M + *bm - 1) / *bm) * ((n2 + 255) / 256);
+  return fused + (tiles <= 32 ? 5.f : 0.f) < apart;
 }
 
 hipError_t launch_gemm_glu(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up, const float *s_up,

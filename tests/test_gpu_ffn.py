@@ -331,6 +331,29 @@ def test_ffn_one_launch_repeat_and_graph(one_launch):
         ctx.set_stream(None)
 
 
+@pytest.mark.parametrize("M,H,I,fused", [(61, 2816, 512, False), (75, 2816, 1536, False), (61, 2048, 2048, True),
+                                         (333, 4096, 11008, True), (100, 4096, 1024, False)])
+def test_ffn_prefill_fuses_gate_and_up_where_it_pays(M, H, I, fused):
+    """Above 16 tokens, few tiles of a long K stay two GEMMs split over K: seen by
+    the up projection's workspace (M I f32), which one gate/up launch does not
+    take. Split mode NEVER keeps the parts' workspace out of the count; the
+    choice is the same."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + H + I)
+    mat = lambda n, k: (torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 16), generator=g, device="cuda:0",  # noqa: E731
+                                      dtype=torch.int32), 0.01 + 0.01 * torch.rand(n, generator=g, device="cuda:0"))
+    x = torch.randn((M, H), generator=g, device="cuda:0").to(torch.bfloat16)
+    y = torch.empty((M, H), device="cuda:0")
+    c = frx.Context(0)
+    try:
+        c.set_gemv_split(frx.GEMV_SPLIT_NEVER)
+        c.ternary_ffn(x, *mat(I, H), *mat(I, H), *mat(H, I), y)
+        torch.cuda.synchronize()
+        h = (M * I * 4 + 255) // 256 * 256
+        assert c.workspace_stats()[0] == (h if fused else 2 * h)
+    finally:
+        c.close()
+
+
 def test_ffn_one_launch_unsupported(one_launch):
     ctx = one_launch
     xf, xb, mats = make_ffn("ffn1/unsup", 4, 128, 192)  # M = 4 > 3
