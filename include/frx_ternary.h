@@ -221,7 +221,7 @@ frx_status frx_ternary_stats(frx_ctx *ctx, const uint32_t *w, uint32_t N,
  * calls that find no workspace (a context's first such call under graph
  * capture) or whose metadata is 2 GiB and more.
  * Up to 32 bf16 (24 f32) tokens run in 128-row tiles over slices of K, any K and
- * N (one token over 8192 rows and more: a table-driven GEMV); more tokens with K
+ * N (one token over tall matrices: a table-driven GEMV); more tokens with K
  * % 64 == 0 in token tiles on the sparse matrix pipe (f32 x as bf16 hi | lo rows
  * in a context workspace), K split over workgroups where the tiles leave compute
  * units idle. fp32 partials live in a context workspace and are added in a
