@@ -78,7 +78,7 @@ __device__ __forceinline__ f32x4 spr_mul(const f32x4 &acc, const u32x4 &a, const
 // columns; part [S][M][Np]. PL: planes of a token, f32 2 or 3, bf16 1.
 // NC: most chunks of a slice (2 or 4; the smaller one keeps more workgroups on a
 // compute unit).
-template <typename XT, typename YT, int SETS, bool PREP, int NC, int PL, bool XMAP>
+template <typename XT, typename YT, int SETS, bool PREP, int NC, int PL>
 __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_t *__restrict__ W,
                                                                   const float *__restrict__ scale,
                                                                   const XT *__restrict__ X, float *__restrict__ part,
@@ -93,13 +93,7 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nch = (K + CH - 1) / CH;
-  // XMAP: a one-dimensional grid, workgroup i dispatched to XCD i % 8, tile t's
-  // slices all on XCD t % 8; slots past the tiles exit at once
-  const int slot = (int)(blockIdx.x >> 3);
-  const int tile = XMAP ? slot / S * 8 + (int)(blockIdx.x & 7) : (int)blockIdx.x;
-  const int s = XMAP ? slot % S : (int)blockIdx.y;
-  if (XMAP && tile * SPR_ROWS >= N) return;  // the whole workgroup
-  const int c0 = s * ncs, nc = min(ncs, nch - c0), k0 = c0 * CH;
+  const int s = blockIdx.y, c0 = s * ncs, nc = min(ncs, nch - c0), k0 = c0 * CH;
   const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(X, (uint32_t)M * (uint32_t)K * (uint32_t)sizeof(XT));
   const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(W, (uint32_t)N * (uint32_t)wpr * 4u);
   // 8-column pieces of a set's tokens, zeros past M and K and past the slice
@@ -153,7 +147,7 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
   for (int set = 0; set < SETS; set++) xload(set);
   __builtin_amdgcn_sched_barrier(0);
   const int i = lane & 15, g = lane >> 4;
-  const int row = tile * SPR_ROWS + wave * 16 + i;
+  const int row = blockIdx.x * SPR_ROWS + wave * 16 + i;
   u32x4 wv[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++)
@@ -207,7 +201,7 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
                 __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, u, 0x128, 0xF, 0xF, true));
       }
     }
-    const int tok = t * TPS + i, r0 = tile * SPR_ROWS + wave * 16 + 4 * g;
+    const int tok = t * TPS + i, r0 = blockIdx.x * SPR_ROWS + wave * 16 + 4 * g;
     const uint32_t off = i < TPS && tok < M && r0 < Np
                              ? (((uint32_t)s * (uint32_t)M + (uint32_t)tok) * (uint32_t)Np + (uint32_t)r0) * 4u
                              : SPR_OOB;
@@ -219,14 +213,14 @@ __global__ __launch_bounds__(SPR_WAVES * 64) void sp24_rows_kernel(const uint32_
   wait_vmcnt<0>();  // this wave's partial stores are complete
   __syncthreads();
   if (tid == 0) {
-    const unsigned old = __hip_atomic_fetch_add(counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned old = __hip_atomic_fetch_add(counters + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     last = old == (unsigned)S - 1u;
-    if (last) __hip_atomic_store(counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (last) __hip_atomic_store(counters + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (!last) return;  // workgroup-uniform
   for (int u = tid; u < M * (SPR_ROWS / 4); u += SPR_WAVES * 64) {
-    const int t = u / (SPR_ROWS / 4), n = tile * SPR_ROWS + (u % (SPR_ROWS / 4)) * 4;
+    const int t = u / (SPR_ROWS / 4), n = blockIdx.x * SPR_ROWS + (u % (SPR_ROWS / 4)) * 4;
     if (n >= N) continue;
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < S; s0 += SPR_CG) {
@@ -282,29 +276,14 @@ template <typename XT, typename YT, int SETS, bool PREP, int NC, int PL>
 static hipError_t launch_sp24_rows_nc(const uint32_t *w, const float *scale, const void *x, void *y, int M, int K,
                                       int N, int ncs, int S, float *part, unsigned *counters, hipStream_t stream) {
   const size_t lds = (size_t)16 * SETS * spr_stride(PREP, NC) * 2;
-  static std::atomic<uint64_t> done[2];
-  const int wpr = PREP ? K / 16 : (K / 4 + 5) / 6, tiles = (N + SPR_ROWS - 1) / SPR_ROWS;
-  // Prepared rows, two column sets, short slices: the slices of a tile on one XCD,
-  // whose L2 then holds the lines they share and the activations once (with a
-  // multiple of 8 tiles the plain order does that by itself). 7296 rows of 1920
-  // columns, 24 / 32 tokens 12.3 -> 10.8 / 14.2 -> 12.2 us (the tile engine 11.7 /
-  // 12.1), 11008 of 1024, 32 tokens 12.2 -> 11.3 (11.5). Longer slices and fewer
-  // tokens lose by it, an XCD's share of the tiles being uneven (11008 of 4096, 16 /
-  // 28 tokens 8.1 -> 9.2 / 11.0 -> 12.9).
-  constexpr bool XM = PREP && SETS == 2 && NC == 2;
-  const bool xmap = XM && tiles % 8 != 0 && S > 1 && (ncs == 1 || M > 24);
-  const void *fn = xmap ? reinterpret_cast<const void *>(&sp24_rows_kernel<XT, YT, SETS, PREP, NC, PL, XM>)
-                        : reinterpret_cast<const void *>(&sp24_rows_kernel<XT, YT, SETS, PREP, NC, PL, false>);
-  const hipError_t e = opt_in_lds(fn, (int)lds, done[xmap]);
+  static std::atomic<uint64_t> done;
+  const hipError_t e =
+      opt_in_lds(reinterpret_cast<const void *>(&sp24_rows_kernel<XT, YT, SETS, PREP, NC, PL>), (int)lds, done);
   if (e != hipSuccess) return e;
-  if (xmap)
-    hipLaunchKernelGGL((sp24_rows_kernel<XT, YT, SETS, PREP, NC, PL, XM>), dim3(8 * S * ((tiles + 7) / 8)),
-                       dim3(SPR_WAVES * 64), lds, stream, w, scale, reinterpret_cast<const XT *>(x), part, counters,
-                       reinterpret_cast<YT *>(y), M, K, N, (N + 3) / 4 * 4, wpr, ncs, S);
-  else
-    hipLaunchKernelGGL((sp24_rows_kernel<XT, YT, SETS, PREP, NC, PL, false>), dim3(tiles, S), dim3(SPR_WAVES * 64), lds,
-                       stream, w, scale, reinterpret_cast<const XT *>(x), part, counters, reinterpret_cast<YT *>(y), M,
-                       K, N, (N + 3) / 4 * 4, wpr, ncs, S);
+  const int wpr = PREP ? K / 16 : (K / 4 + 5) / 6;
+  hipLaunchKernelGGL((sp24_rows_kernel<XT, YT, SETS, PREP, NC, PL>), dim3((N + SPR_ROWS - 1) / SPR_ROWS, S),
+                     dim3(SPR_WAVES * 64), lds, stream, w, scale, reinterpret_cast<const XT *>(x), part, counters,
+                     reinterpret_cast<YT *>(y), M, K, N, (N + 3) / 4 * 4, wpr, ncs, S);
   return hipGetLastError();
 }
 
