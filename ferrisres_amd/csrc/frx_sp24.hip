@@ -267,6 +267,14 @@ bool sp24_rows_plan(int M, int K, int N, int xt_bf16, int prepared, int cus, int
   while (n < SPR_NC && (tiles * ((nch + n - 1) / n) > (size_t)(prepared ? 2 : 3) * cus || (nch + n - 1) / n > SPR_CG)) n++;
   *ncs = n;
   *S = (nch + n - 1) / n;
+  // prepared rows past 24 tokens in many short slices: with tiles that are no
+  // multiple of 4 a tile's slices lie on up to eight XCDs, each of which fetches
+  // the lines they share, and the tile engine is level or ahead (rows x columns, 32
+  // tokens, engine / here: 7296 x 1920 12.1 / 14.2 us, 3904 x 2752 12.2 / 13.3, 11008
+  // x 1024 11.5 / 12.2; but 6632 x 4096, 52 tiles, 27 tokens 13.1 / 10.4). Keeping
+  // them on one XCD gained 7-14% there and lost as much on others (28 tokens, 3328 x
+  // 3392 11.5 -> 12.7, 11008 x 4096 11.0 -> 12.9).
+  if (prepared && M > 24 && tiles % 4 != 0 && n <= 2 && 10 * tiles * (size_t)*S > 13 * (size_t)cus) return false;
   return sp24_rows_workspace_bytes(M, N, *S) < SPR_OOB;
 }
 

@@ -331,6 +331,29 @@ def test_prepared_linear_same_bits_above_32_tokens(ctx, M, K, N):
                 assert err.item() < (2.0 ** -20 if dt == torch.float32 else 2.0 ** -8)
 
 
+@pytest.mark.parametrize("M,K,N", [(17, 512, 300), (24, 1920, 7296), (32, 2752, 8250), (25, 1024, 1025), (32, 4096, 7300),
+                                   (20, 448, 4), (28, 2048, 1024)])
+@pytest.mark.parametrize("yt", ["f32", "bf16"])
+def test_prepared_17_to_32_tokens(ctx, M, K, N, yt):
+    """17-32 tokens over prepared rows, in the row tiles and, past 24 tokens in
+    many short slices (2752 x 8250, 4096 x 7300), in the tile engine, ragged rows,
+    against fp64; twice (the arrival counters are left at zero). f32 sums of
+    exact products: below 2^-20 of the norm; bf16 outputs one rounding."""
+    g = torch.Generator(device="cuda:0").manual_seed(M + K + N)
+    meta = _random_meta(g, N, K)
+    s = 0.02 + 0.01 * torch.rand(N, generator=g, device="cuda:0")
+    prep = torch.empty((N, K // 16), dtype=torch.int32, device="cuda:0")
+    ctx.sparse24_prepare(meta, K, prep)
+    x = torch.randn((M, K), generator=g, device="cuda:0").to(torch.bfloat16)
+    ref = (x.double() @ _dense64(meta, K).t()) * s.double()
+    for _ in range(2):
+        y = torch.full((M, N), float("nan"), dtype=torch.float32 if yt == "f32" else torch.bfloat16, device="cuda:0")
+        ctx.sparse24_prepared_linear(prep, s, x, y)
+        torch.cuda.synchronize()
+        err = (torch.linalg.norm(y.double() - ref) / torch.linalg.norm(ref)).item()
+        assert err < (2.0 ** -20 if yt == "f32" else 2.0 ** -8)
+
+
 def test_prepared_entry_errors(ctx):
     """K % 64 != 0 and f32 activations are refused with a status, before any
     launch; the context stays usable."""
