@@ -2361,7 +2361,7 @@ hipError_t launch_gemv_group(const void *x, int xt_bf16, int yt_bf16, int B, int
 hipError_t launch_gemv_glu(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up,
                            const float *s_up, const void *x, int xt_bf16, float *h, int B, int K,
                            int N, int gelu, hipStream_t stream) {
-  if (xt_bf16 && B >= glu_staged_min_tokens(K, N) && gemv_xs_ok(x, B, K, 1, 2)) {
+  if (xt_bf16 && B >= glu_staged_min_tokens(K, N, false) && gemv_xs_ok(x, B, K, 1, 2)) {
     if (gelu)
       return launch_gemv_xs<float, 2, GEMV_GEGLU, XS_BF16, false>(w_gate, s_gate, w_up, s_up, x, x, h, B, K, N,
                                                                    stream);
@@ -2411,7 +2411,7 @@ hipError_t launch_glu_combine(const float *g, const float *u, float *h, size_t n
 hipError_t launch_gemv_glu_planes(const uint32_t *w_gate, const float *s_gate, const uint32_t *w_up,
                                   const float *s_up, const void *x, uint16_t *h_planes, int B, int K,
                                   int N, int gelu, hipStream_t stream) {
-  if (B >= glu_staged_min_tokens(K, N) && gemv_xs_ok(x, B, K, 1, 2)) {
+  if (B >= glu_staged_min_tokens(K, N, true) && gemv_xs_ok(x, B, K, 1, 2)) {
     if (gelu)
       return launch_gemv_xs<uint16_t, 2, GEMV_GEGLU, XS_BF16, true>(w_gate, s_gate, w_up, s_up, x, x, h_planes, B,
                                                                      K, N, stream);

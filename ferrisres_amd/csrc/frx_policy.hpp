@@ -22,20 +22,28 @@ inline size_t grow_bytes(size_t have, size_t need) {
 // the down projection (times are of the whole FFN, hidden / intermediate) -------
 
 // bf16 tokens from which gate and up leave the kernel with operand loads for the
-// staged one (gemv_xs_kernel): 5 over 2048 to 4096 columns (4096 / 14336, 5 / 7
-// tokens 25.9 / 27.4 us with operand loads, 24.4 / 23.7 staged; 4096 / 5632 15.3 /
-// 16.2 against 14.9 / 15.0), else 8. Over up to 4096 rows the FFN is level and
-// frx_ternary_glu slower (2304 columns, 2048 rows, 6 / 7 tokens 4.6 / 4.8 us against
-// 5.0 / 5.0). Below 2048 columns a workgroup's few quads leave its waves idle
-// (1024 / 2048, 5 tokens 8.8 against 9.3). Above 4096 its x outweighs its rows
-// (5120 / 4096, 5 / 7 tokens 16.1 / 14.0 against 17.1 / 14.6, 5120 / 13824 28.3 / 30.5
-// against 29.8 / 30.2) but where each unit has two tiles of them (5120 / 5632, 5 / 6
-// / 7 tokens 17.9 / 18.5 / 18.9 against 18.0 / 17.9 / 17.9, 5120 / 8192 20.0 / 20.7 /
-// 21.2 against 20.2 / 20.6 / 20.5).
-constexpr int glu_staged_min_tokens(int K, int N) {
+// staged one (gemv_xs_kernel), 8 where it is not ahead from 5 or 6. Writing h as
+// planes (the FFN): over 2048 to 4096 columns past 4096 rows (4096 / 14336, 5 / 7
+// tokens 25.9 / 27.4 us with operand loads, 24.4 / 23.7 staged; 2560 / 8192 15.9 / 16.7
+// and 15.4 / 15.6; over fewer rows the FFN is level). Writing fp32 h
+// (frx_ternary_glu): past 8192 rows, and below where the columns fill its waves'
+// quads (2816 / 12288 8.1 / 8.5 and 7.6 / 7.6, 4096 / 5632 7.6 / 7.9 and 7.1 / 7.1; but
+// 3328 / 5632 6.4 / 6.6 and 7.0 / 6.9, 2432 / 5632 5.8 / 6.0 and 6.9 / 6.9). Below 2048
+// columns a workgroup's few quads leave its waves idle (FFN 1024 / 2048, 5 tokens
+// 8.8 against 9.3). Above 4096 its x outweighs its rows (FFN 5120 / 4096, 5 / 7 tokens
+// 16.1 / 14.0 against 17.1 / 14.6, 5120 / 13824 28.3 / 30.5 against 29.8 / 30.2) but
+// where the FFN gives each unit two tiles of them (5120 / 5632, 5 / 6 / 7 tokens 17.9 /
+// 18.5 / 18.9 against 18.0 / 17.9 / 17.9, 5120 / 8192 20.0 / 20.7 / 21.2 against 20.2 /
+// 20.6 / 20.5). fp32 h leaves the operand loads there only where rows that are no
+// multiple of 16 bytes narrow them (5 / 7 tokens: 4432 / 5632 11.3 / 12.3 against 9.6 /
+// 9.5, 5136 / 8192 12.6 / 14.6 against 10.0 / 10.1; 4416 / 5632 7.8 / 8.7 against 9.5 /
+// 9.5, 5120 / 5632 8.8 / 9.8 against 9.7 / 9.7).
+constexpr int glu_staged_min_tokens(int K, int N, bool planes) {
   if (K < 2048) return 8;
-  if (K > 4096) return N > 4096 && N <= 8192 ? 6 : 8;
-  return N > 4096 ? 5 : 8;
+  if (K > 4096 && (N <= 4096 || N > 8192)) return 8;
+  if (K > 4096) return planes ? 6 : K % 64 != 0 ? 5 : 8;
+  if (planes) return N > 4096 ? 5 : 8;
+  return N > 8192 || (K > 3840 && N > 4096) ? 5 : 8;
 }
 
 // Whether one f32 token takes the staged kernel: not over more than 4096

@@ -62,11 +62,15 @@ static int check_ffn_rules() {
   const bool ok = frx::glu_staged_tiles(5120, 11008, true, 256) == 1 && frx::glu_staged_tiles(5120, 13824, true, 256) == 2 &&
                   frx::glu_staged_tiles(5120, 11008, false, 256) == 2 && frx::glu_staged_tiles(4096, 11008, true, 256) == 4 &&
                   frx::glu_staged_tiles(4096, 13824, true, 256) == 2 && frx::glu_staged_tiles(2048, 13824, false, 256) == 4 &&
-                  frx::glu_staged_min_tokens(5120, 4096) == 8 && frx::glu_staged_min_tokens(4096, 11008) == 5 &&
-                  frx::glu_staged_min_tokens(4096, 4096) == 8 && frx::glu_staged_min_tokens(1024, 2048) == 8 &&
+                  frx::glu_staged_min_tokens(5120, 4096, true) == 8 && frx::glu_staged_min_tokens(4096, 11008, true) == 5 &&
+                  frx::glu_staged_min_tokens(4096, 4096, true) == 8 && frx::glu_staged_min_tokens(1024, 2048, true) == 8 &&
+                  frx::glu_staged_min_tokens(2560, 8192, true) == 5 && frx::glu_staged_min_tokens(5120, 5632, true) == 6 &&
+                  frx::glu_staged_min_tokens(2816, 12288, false) == 5 && frx::glu_staged_min_tokens(2816, 5632, false) == 8 &&
+                  frx::glu_staged_min_tokens(4096, 5632, false) == 5 && frx::glu_staged_min_tokens(4432, 7328, false) == 5 &&
+                  frx::glu_staged_min_tokens(5120, 5632, false) == 8 && frx::glu_staged_min_tokens(4416, 8192, false) == 8 &&
                   !frx::glu_staged_one_f32(1024, 13824) && frx::glu_staged_one_f32(1024, 4096) &&
                   frx::glu_staged_one_f32(3072, 11008) && !frx::glu_staged_one_f32(5120, 13824) &&
-                  frx::glu_staged_min_tokens(5120, 5632) == 6 && frx::ffn_down_split_min(8, 3072, 256) <= 5632 &&
+                  frx::ffn_down_split_min(8, 3072, 256) <= 5632 &&
                   frx::ffn_down_split_min(9, 3072, 256) > 5632 && frx::ffn_down_split_min(16, 3072, 256) <= 8192 &&
                   frx::ffn_down_split_min(12, 1024, 256) <= 5632 && frx::ffn_down_split_min(12, 5120, 256) <= 5632;
   if (!ok) printf("measured lines of the FFN rules\n");
